@@ -18,7 +18,10 @@
 // k_conv_bf16: the same GEMM for the other channel counts (64 and 8): 4-row x
 //   TW-pixel tiles, the whole input tile in LDS, weights in chunk groups
 //   staged through registers, output staged through LDS.
-// k_conv_f32: the same on v_mfma_f32_16x16x4_f32 (2-row tile, float32 maps).
+// k_conv_split (conv_split.hip): the float32 layers of 100 and 64 channels, as
+//   six bf16 products of exactly split operands.
+// k_conv_f32: 8-channel float32 layers on v_mfma_f32_16x16x4_f32 (2-row tile),
+//   whose reduction is too short to fill a 32-deep step's four groups.
 // k_conv_generic: VALU direct convolution for the 1- and 3-channel input layer
 //   and any shape the MFMA kernels do not cover.
 #include <cmath>
@@ -27,6 +30,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "conv_split.hpp"
 
 namespace ccs {
 
@@ -849,9 +853,11 @@ static bool launch_mfma(const ConvShape& s, int precision, const void* x, const 
            try_bf16<3, 3, 8, 4>(s, x, wpk, b, act, y, st) || try_bf16<3, 3, 1, 1>(s, x, wpk, b, act, y, st) ||
            try_bf16<2, 2, 1, 1>(s, x, wpk, b, act, y, st);
   }
-  return try_f32<3, 3, 13, 7>(s, x, wpk, b, act, y, st) || try_f32<2, 2, 13, 7>(s, x, wpk, b, act, y, st) ||
-         try_f32<3, 3, 8, 4>(s, x, wpk, b, act, y, st) || try_f32<3, 3, 1, 1>(s, x, wpk, b, act, y, st) ||
-         try_f32<2, 2, 1, 1>(s, x, wpk, b, act, y, st);
+  if (split_supported(s.K, s.C, s.KH, s.KW)) {
+    split_launch((const float*)x, s.H, s.W, s.C, wpk, b, s.K, s.KH, s.KW, act, (float*)y, st);
+    return true;
+  }
+  return try_f32<3, 3, 1, 1>(s, x, wpk, b, act, y, st) || try_f32<2, 2, 1, 1>(s, x, wpk, b, act, y, st);
 }
 
 static size_t packed_bytes(int K, int C, int KH, int KW, int precision) {
@@ -861,6 +867,7 @@ static size_t packed_bytes(int K, int C, int KH, int KW, int precision) {
     const int NQ = packed_chunks(Cs / 8, KH * KW);
     return (size_t)NQ * NP * RPB * 2;
   }
+  if (split_supported(K, C, KH, KW)) return split_packed_bytes(K, C, KH, KW);
   const int NQ = (KH * KW * Cs + 3) / 4;
   return (size_t)NQ * 4 * NP * 4;
 }
@@ -884,6 +891,8 @@ extern "C" int ccs_conv_pack_weights(ccs_handle_t h, const float* w, int K, int 
     const int NQ = packed_chunks(Cs / 8, KH * KW);
     const long total = (long)NQ * NP * RPB;
     k_pack_bf16<<<ceil_div(total, 256), 256, 0, h->stream>>>(w, K, C, Cs, KH, KW, NQ, NP, (bf16*)packed);
+  } else if (split_supported(K, C, KH, KW)) {
+    split_pack(w, K, C, KH, KW, packed, h->stream);
   } else {
     const int NQ = (KH * KW * Cs + 3) / 4;
     const long total = (long)NQ * 4 * NP;
@@ -969,7 +978,7 @@ extern "C" int ccs_conv_forward_packed(ccs_handle_t h, const void* x, int x_layo
 // GPU (held until the process ends) instead of the handle's scratch.  The
 // array's name is a host-side stand-in, not a device address: host code uses
 // only the address hipGetSymbolAddress returns on each device.
-constexpr size_t kNoAllocScratchBytes = 512u << 10;  // the largest MFMA pack is 419,328 bytes
+constexpr size_t kNoAllocScratchBytes = 640u << 10;  // the largest MFMA pack is 645,120 bytes
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -1,0 +1,36 @@
+// float32 convolution layers on the bf16 matrix cores (conv_split.hip).
+#pragma once
+
+#include "common.hpp"
+
+namespace ccs {
+
+// Whether a KH x KW layer from Cs_in = feature_stride(C) to K channels has a
+// split kernel: the 100-channel layers (3x3 and 2x2) and the 64-channel 3x3 one.
+bool split_supported(int K, int C, int KH, int KW);
+size_t split_packed_bytes(int K, int C, int KH, int KW);
+void split_pack(const float* w, int K, int C, int KH, int KW, void* packed, hipStream_t st);
+void split_launch(const float* x, int H, int W, int C, const void* packed, const float* b, int K, int KH, int KW,
+                  int act, float* y, hipStream_t st);
+
+// x = h + m + l in bfloat16, exactly for every finite float32 down to l's
+// underflow: h is x rounded to nearest, m the residual x - h rounded to nearest
+// (|m| <= 2^-9 |x|), l what is left (at most 6 significant bits).  A value that
+// would round to infinity is clamped first; an infinity or a NaN goes to l
+// alone (h = m = 0), so that a product with a split finite y, which takes
+// l only with y's h, keeps its sign or its NaN.
+template <int N>
+__device__ __forceinline__ void split3(const float (&x)[N], bf16 (&h)[N], bf16 (&m)[N], bf16 (&l)[N]) {
+  constexpr float kMaxBf16 = 3.38953139e38f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const bool fin = (__float_as_uint(x[e]) & 0x7fffffffu) < 0x7f800000u;
+    const float v = fin ? x[e] : 0.f;
+    h[e] = (bf16)__builtin_amdgcn_fmed3f(v, -kMaxBf16, kMaxBf16);
+    const float r = v - (float)h[e];
+    m[e] = (bf16)r;
+    l[e] = (bf16)(fin ? r - (float)m[e] : x[e]);
+  }
+}
+
+}  // namespace ccs
