@@ -28,6 +28,38 @@ struct ChainArgs {
   float L1, L2;
 };
 
+// Column sweeps of large volumes keep the backward messages of every
+// seg_len()-th node only; the forward pass recomputes a segment's messages from
+// the checkpoint at its end, bit for bit (0: every message is stored and
+// re-read).
+#ifndef CCS_CRF_SEG
+#define CCS_CRF_SEG 12
+#endif
+constexpr int kSeg = CCS_CRF_SEG;
+// Segment length by labels per lane: a segment keeps two segments' unaries and
+// costs and one segment's messages in registers, so four labels per lane take
+// half the length (two waves per SIMD without spills).
+constexpr int seg_length(int lpl) { return kSeg <= 0 ? 0 : lpl >= 4 ? (kSeg / 2 > 0 ? kSeg / 2 : 1) : kSeg; }
+
+// Row sweeps with a message wave keep a ring of kRowRing segments' messages in LDS.
+constexpr int kRowRing = 3;
+
+constexpr size_t kLdsPerCu = 160 * 1024;
+
+// LDS of one row chain with the message wave: b, w, u, [w2], v floats rounded
+// to 16 bytes, then the message ring.
+constexpr size_t row_seg_lds(int lpl, bool per_edge, int n) {
+  return sizeof(float) * ((((per_edge ? 6 : 5) * (size_t)n + 3) & ~(size_t)3) +
+                          (size_t)kRowRing * seg_length(lpl) * 64 * lpl);
+}
+
+// Compute units of the current device.
+int cu_count();
+
+// One sweep for LPL (1, 2 or 4) labels per lane; seg: the checkpointed schemes.
+template <int LPL>
+int launch_labels(ChainMode mode, ChainArgs& a, bool seg, hipStream_t st);
+
 // Launches one sweep of `mode` over all chains of `a` on `st`.
 int launch_chain(ChainMode mode, ChainArgs& a, hipStream_t st);
 
