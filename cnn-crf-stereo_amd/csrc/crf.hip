@@ -45,10 +45,40 @@ __global__ void k_sum_f64(const double* __restrict__ in, int n, double* __restri
   if (threadIdx.x == 0) out[0] = s[0];
 }
 
-// lb = sums[j] (+ kept[j-1] if j > 0).
-__global__ void k_bound(const double* __restrict__ sums, int iters, double* __restrict__ lb) {
-  const int j = 2 * iters;
-  lb[0] = iters == 0 ? sums[0] : sums[j] + sums[2 * iters + 1 + (j - 1)];
+// The sums of a batch of half-steps of a run, one block per sum: block 2 s is
+// the chain minima S_{j0 + s}, block 2 s + 1 the kept constants K_{j0 + s} (not
+// of the decode), each summed as k_sum_f64 sums.  Half-step j's chains are in
+// slot j % kSumSlots of `chains` (nmax minima, then nmax constants); even j are
+// row sweeps (H chains; the last one is the decode), odd j column sweeps (W).
+// The block past the last sum forms the bound S_{2 iters} + K_{2 iters - 1}.
+__global__ void k_run_sums(const double* __restrict__ chains, int nmax, int H, int W, int j0, int steps, int iters,
+                           double* __restrict__ S, double* __restrict__ K, double* __restrict__ lb) {
+  __shared__ double s[256];
+  auto sum = [&](int j, int kept) {
+    const double* in = chains + ((long)(j % kSumSlots) * 2 + kept) * nmax;
+    const int n = (j & 1) ? W : H;
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) acc += in[i];
+    s[threadIdx.x] = acc;
+    __syncthreads();
+    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
+      if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+      __syncthreads();
+    }
+    const double total = s[0];
+    __syncthreads();  // s is reused by a second sum
+    return total;
+  };
+  if ((int)blockIdx.x == 2 * steps) {
+    double v = sum(2 * iters, 0);
+    if (iters > 0) v += sum(2 * iters - 1, 1);
+    if (threadIdx.x == 0) lb[0] = v;
+    return;
+  }
+  const int j = j0 + (blockIdx.x >> 1), kept = blockIdx.x & 1;
+  if (kept && j == 2 * iters) return;  // (uniform) the decode keeps nothing
+  const double v = sum(j, kept);
+  if (threadIdx.x == 0) (kept ? K : S)[j] = v;
 }
 
 __device__ __forceinline__ float rho(int d, float L1, float L2, int delta) {
@@ -209,9 +239,11 @@ static int check_crf_args(int H, int W, int D, float L1, float L2, int delta) {
 // One half-step.  pen == nullptr: edge weights wx / wy with L1, L2; otherwise
 // per-edge penalties pen (levels x H x W x 2: P1 = pen[levels-1], P2 = pen[0],
 // x components for the row edges, y for the column edges) and wx, wy unused.
+// chains (2 max(H, W) doubles): where the per-chain minima and constants go
+// (nullptr: the handle's scratch).
 static int sweep(ccs_handle_t h, const float* cost, float* A, const float* wx, const float* wy, const float* pen,
                  int levels, int H, int W, int D, float L1, float L2, int delta, int direction, int* labels,
-                 double* chain_sum, double* kept_sum) {
+                 double* chain_sum, double* kept_sum, double* chains = nullptr) {
   CCS_CHECK(h && A, CCS_ERR_ARG, "ccs_slackprop_sweep: NULL argument");
   int rc = check_crf_args(H, W, D, pen ? 0.f : L1, pen ? 0.f : L2, delta);
   if (rc) return rc;
@@ -224,8 +256,11 @@ static int sweep(ccs_handle_t h, const float* cost, float* A, const float* wx, c
   const size_t vol = (size_t)H * W * D;
   if ((rc = h->crf_msg.reserve(vol * sizeof(float), h->stream))) return rc;
   const int nmax = H > W ? H : W;
-  if ((rc = h->crf_small.reserve(sizeof(double) * 2 * (size_t)nmax, h->stream))) return rc;
-  double* lam = (double*)h->crf_small.ptr;
+  if (!chains) {  // a half-step of its own
+    if ((rc = h->crf_small.reserve(sizeof(double) * 2 * (size_t)nmax, h->stream))) return rc;
+    chains = (double*)h->crf_small.ptr;
+  }
+  double* lam = chains;
   double* kept = lam + nmax;
   ChainArgs a{};
   if (direction == 3) {  // the first sweep of a run reads every cost: it flags NaN per row
@@ -275,32 +310,43 @@ static int run(ccs_handle_t h, const float* cost, const float* wx, const float* 
   int rc = check_crf_args(H, W, D, pen ? 0.f : L1, pen ? 0.f : L2, delta);
   if (rc) return rc;
   CCS_CHECK(iters >= 0 && iters <= 10000, CCS_ERR_ARG, "ccs_slackprop: bad iteration count %d", iters);
-  const size_t vol = (size_t)H * W * D;
-  if ((rc = h->crf_a.reserve(vol * sizeof(float), h->stream))) return rc;
+  const size_t vol = (size_t)H * W * D, bytes = vol * sizeof(float);
+  // The state lives in unaries_out where the caller wants the final unaries
+  // (no copy at the end), unless that overlaps the costs every sweep reads.
+  const uintptr_t u0 = (uintptr_t)unaries_out, c0 = (uintptr_t)cost;
+  const bool own = !unaries_out || (u0 < c0 + bytes && c0 < u0 + bytes);
+  if (own && (rc = h->crf_a.reserve(bytes, h->stream))) return rc;
   if ((rc = h->crf_sums.reserve(sizeof(double) * (4 * (size_t)iters + 2), h->stream))) return rc;
-  float* A = (float*)h->crf_a.ptr;
-  double* S = (double*)h->crf_sums.ptr;  // S_0 .. S_{2 iters}
-  double* K = S + 2 * iters + 1;         // K_0 .. K_{2 iters - 1}
+  const int nmax = H > W ? H : W;
+  if ((rc = h->crf_small.reserve(sizeof(double) * run_chain_doubles(nmax, iters), h->stream))) return rc;
+  float* A = own ? (float*)h->crf_a.ptr : unaries_out;
+  double* S = sums ? sums : (double*)h->crf_sums.ptr;  // S_0 .. S_{2 iters}
+  double* K = S + 2 * iters + 1;                       // K_0 .. K_{2 iters - 1}
+  double* chains = (double*)h->crf_small.ptr;
   if (iters == 0) {
-    CCS_HIP(hipMemcpyAsync(A, cost, vol * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
+    CCS_HIP(hipMemcpyAsync(A, cost, bytes, hipMemcpyDeviceToDevice, h->stream));
     h->nan_chains = 0;  // no row sweep reads the costs
   }
-  for (int it = 0; it < iters; ++it) {
+  // Half-steps 0 .. 2 iters - 1 alternate rows and columns, 2 iters is the
+  // decode.  Their per-chain results keep kSumSlots slots, and one launch sums
+  // a batch of slots (two launches per half-step took 4.6 us each between the
+  // sweeps).
+  int j0 = 0;
+  for (int j = 0; j <= 2 * iters; ++j) {
+    const bool last = j == 2 * iters;
     // The first row sweep reads the unaries from cost (A = cost is never copied).
-    if ((rc = sweep(h, cost, A, wx, wy, pen, levels, H, W, D, L1, L2, delta, it == 0 ? 3 : 0, nullptr, S + 2 * it,
-                    K + 2 * it)))
+    const int direction = last ? 2 : j == 0 ? 3 : j & 1;
+    if ((rc = sweep(h, cost, A, wx, wy, pen, levels, H, W, D, L1, L2, delta, direction, labels, nullptr, nullptr,
+                    chains + (size_t)(j % kSumSlots) * 2 * nmax)))
       return rc;
-    if ((rc = sweep(h, cost, A, wx, wy, pen, levels, H, W, D, L1, L2, delta, 1, nullptr, S + 2 * it + 1,
-                    K + 2 * it + 1)))
-      return rc;
+    if (last || j - j0 + 1 == kSumSlots) {
+      const int steps = j - j0 + 1;
+      k_run_sums<<<2 * steps + (last && lower_bound ? 1 : 0), 256, 0, h->stream>>>(chains, nmax, H, W, j0, steps,
+                                                                                  iters, S, K, lower_bound);
+      j0 = j + 1;
+    }
   }
-  if ((rc = sweep(h, cost, A, wx, wy, pen, levels, H, W, D, L1, L2, delta, 2, labels, S + 2 * iters, nullptr)))
-    return rc;
-  if (lower_bound) k_bound<<<1, 1, 0, h->stream>>>(S, iters, lower_bound);
-  if (sums)
-    CCS_HIP(hipMemcpyAsync(sums, S, sizeof(double) * (4 * (size_t)iters + 1), hipMemcpyDeviceToDevice, h->stream));
-  if (unaries_out)
-    CCS_HIP(hipMemcpyAsync(unaries_out, A, vol * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
+  if (own && unaries_out) CCS_HIP(hipMemcpyAsync(unaries_out, A, bytes, hipMemcpyDeviceToDevice, h->stream));
   CCS_LAUNCH_CHECK();
   return CCS_OK;
 }

@@ -581,18 +581,20 @@ __device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D, fl
 template <int LPL, int FIT>
 __device__ __forceinline__ void st_buf(Rsrc r, int soff, int lane, int D, const Vec<LPL>& x) {
   if constexpr (FIT != kFitAny) {
-    if (FIT == kFitLanes && lane * LPL >= D) return;
+    // The lanes without labels store past the resource's range, which the
+    // hardware drops: no branch around the store.
+    const int voff = FIT == kFitFull || lane * LPL < D ? lane * LPL * 4 : (int)0x80000000;
     if constexpr (LPL == 4) {  // two 64-bit stores (see kNoWideStores)
       const u32x2 t = {__float_as_uint(x.v[0]), __float_as_uint(x.v[1])};
       const u32x2 u = {__float_as_uint(x.v[2]), __float_as_uint(x.v[3])};
-      __builtin_amdgcn_raw_buffer_store_b64(t, r, lane * 16, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(t, r, voff, soff, 0);
       asm volatile("" ::: "memory");
-      __builtin_amdgcn_raw_buffer_store_b64(u, r, lane * 16 + 8, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(u, r, voff + 8, soff, 0);
     } else if constexpr (LPL == 2) {
       const u32x2 t = {__float_as_uint(x.v[0]), __float_as_uint(x.v[1])};
-      __builtin_amdgcn_raw_buffer_store_b64(t, r, lane * 8, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(t, r, voff, soff, 0);
     } else {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x.v[0]), r, lane * 4, soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x.v[0]), r, voff, soff, 0);
     }
   } else {
 #pragma unroll

@@ -40,5 +40,5 @@ def test_lane_path_equals_element_path(handle, D, H, W):
     wx, wy = torch.rand((2, H, W), generator=g, device="cuda")
     want = run(handle, shifted(cost), wx, wy, shifted(cost), 3)
     got = run(handle, cost, wx, wy, torch.empty_like(cost), 3)
-    for a, b in zip(got, want):
-        assert torch.equal(a, b)
+    for a, b in zip(got, want):  # (an infinite cost leaves NaN unaries: inf - inf)
+        assert torch.allclose(a, b, rtol=0, atol=0, equal_nan=True)
