@@ -579,7 +579,7 @@ extern "C" int ccs_correlation_volume_backward(ccs_handle_t h, const void* f0, c
   const int Cs = feature_stride(C);
   const long total = (long)H * W * Cs;
   const int o0 = -disp_min, ostep = -disp_step;
-  if (corr_bwd_split_supported(Cs, ostep)) {
+  if (corr_bwd_split_supported(Cs, W, D, ostep)) {
     corr_bwd_split({f0, f1, G, df0, df1, H, W, Cs, D, o0, ostep, 0}, precision, h->stream);
     CCS_LAUNCH_CHECK();
     return CCS_OK;

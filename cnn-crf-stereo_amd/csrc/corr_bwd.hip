@@ -21,11 +21,12 @@
 // add it, as conv_split.hip does.  The result rows are channels (F is the A
 // operand), so a lane stores four consecutive channels of a pixel.
 //
-// The old kernel (v_mfma_f32_16x16x4_f32 on operands gathered from LDS one
-// float at a time) took 3.7 ms per map at 1488 x 992, D = 256 in bf16, 20
-// TFLOP/s.  Here the matrix cores need 0.12 ms of it, and reading G (1.51 GB)
-// sets the pace, so both maps of a row run on the same XCD one after the other
-// and share G through its L2.
+// The kernel it replaces (v_mfma_f32_16x16x4_f32 on operands gathered from LDS
+// one float at a time) took 7.39 ms for both maps at 1488 x 992, D = 256 in
+// bf16; this one takes 1.52 ms, of which reading G costs 0.5 and staging 0.4
+// (timed without them).  G (1.51 GB) and the maps at copy rate are 0.57 ms; both
+// maps of a row run on the same XCD one after the other, so that they share G
+// through its L2.  64-disparity chunks with three workgroups per CU: 2.27 ms.
 #include <type_traits>
 
 #include "conv_split.hpp"
@@ -117,15 +118,18 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
     *reinterpret_cast<u32x4*>(lds + pl * Cfg::plane + (Cs * (PITCH / 8) + w) * 16) = u32x4{0u, 0u, 0u, 0u};
   }
 
-  // Columns R = 0 .. COLS-1 of the chunk that starts at disparity kc: four
-  // columns of one channel group per unit, consecutive threads on consecutive
-  // columns (their transposed stores are contiguous).
+  // Columns R = 0 .. COLS-1 of the chunk that starts at disparity kc, four
+  // columns of one channel group per unit.
   auto stage = [&](int kc, int kn) {
     constexpr int VE = 16 / (int)sizeof(T);
     const int groups = Cs / VE, last = MPW - 1 + kn;  // columns past `last` are never multiplied by a G entry
     const int col0 = s > 0 ? P0 + e0 + kc : P0 + MPW - 1 + e0 - kc;
-    for (int v = tid; v < groups * (COLS / 4); v += Cfg::THREADS) {
-      const int g = v / (COLS / 4), q = v % (COLS / 4);
+    constexpr int QB = (COLS + 63) / 64;  // blocks of 16 column quads
+    for (int v = tid; v < (groups + 3) / 4 * QB * 64; v += Cfg::THREADS) {
+      // 16 lanes take 16 column quads of one group, the wave four groups: a
+      // pixel is read 64 bytes at a time, and 16 lanes store 128 bytes in a row.
+      const int b = v >> 6, q = b % QB * 16 + (v & 15), g = b / QB * 4 + ((v >> 4) & 3);
+      if (g >= groups || 4 * q >= COLS) continue;
       u32x4 r[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -170,35 +174,55 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
     sm[mt] = s > 0 ? 16 * mt + lrow : PW - 1 - 16 * mt - lrow;
   }
   // The G entries of step st of the chunk (kc, kn): k = 32 st + 8 lgrp + j - sm.
-  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  // The row of G is a buffer resource: an entry that does not exist is read
+  // past its range, which gives zero.  In the inner steps every entry exists,
+  // and a lane's eight are 16-byte loads (df0) or a fixed stride of D + s apart
+  // (df1), one address for all.
+  const __amdgpu_buffer_rsrc_t rG =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(grow), (short)0, W * D * 4, 0x00020000);
+  constexpr int kNone = (int)0x80000000;
+  const int gstep = (s * D + 1) * 4;  // bytes between a lane's entries of df1
   auto load_g = [&](int kc, int kn, int st, float (&x)[MT][8]) {
-    const bool inner = st >= 1 && 32 * st + 32 <= kn;  // every lane's eight k exist (uniform)
+    bool inner = st >= 1 && 32 * st + 32 <= kn;  // (uniform) every lane's eight k exist
+    if (gather) {  // and so do the columns of the wave's 32
+      const int c0 = (s > 0 ? P0 + e0 + kc : P0 + MPW - 1 + e0 - kc) + s * (bw + 32 * st), c1 = c0 + 31 * s;
+      inner = inner && min(c0, c1) >= 0 && max(c0, c1) < W;
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int k0 = 32 * st + 8 * lgrp - sm[mt];
       if (!gather) {
-        const bool in = pix[mt] < W;
-        const float* src = grow + (long)min(pix[mt], W - 1) * D + kc;
+        const int off = (pix[mt] * D + kc + k0) * 4;
         if (inner) {
-          const f32x4u u = *reinterpret_cast<const f32x4u*>(src + k0), v = *reinterpret_cast<const f32x4u*>(src + k0 + 4);
+          const int v = pix[mt] < W ? off : kNone;
+          const u32x4 p = __builtin_amdgcn_raw_buffer_load_b128(rG, v, 0, 0);
+          const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rG, v, 16, 0);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) x[mt][j] = in ? (j < 4 ? u[j & 3] : v[j & 3]) : 0.f;
+          for (int j = 0; j < 8; ++j) x[mt][j] = __uint_as_float(j < 4 ? p[j & 3] : q[j & 3]);
         } else {
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const int k = k0 + j;
-            const float v = src[min(max(k, 0), kn - 1)];
-            x[mt][j] = in && k >= 0 && k < kn ? v : 0.f;
+            const bool ok = pix[mt] < W && k0 + j >= 0 && k0 + j < kn;
+            x[mt][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rG, ok ? off + 4 * j : kNone, 0, 0));
           }
         }
       } else {
-        const int col0 = pix[mt] + e0 + s * kc;
+        const int col0 = pix[mt] + e0 + s * (kc + k0);
+        const int off = (col0 * D + kc + k0) * 4;
+        if (inner) {
+          const int v = gstep >= 0 ? off : off + 7 * gstep;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int k = k0 + j, col = col0 + s * k;
-          const bool ok = k >= 0 && k < kn && col >= 0 && col < W && pix[mt] < W;
-          const float v = grow[(long)(ok ? col : 0) * D + (ok ? kc + k : 0)];
-          x[mt][j] = ok ? v : 0.f;
+          for (int j = 0; j < 8; ++j)
+            x[mt][j] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rG, v, gstep >= 0 ? j * gstep : (j - 7) * gstep, 0));
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int col = col0 + s * j;
+            const bool ok = pix[mt] < W && k0 + j >= 0 && k0 + j < kn && col >= 0 && col < W;
+            x[mt][j] =
+                __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rG, ok ? off + j * gstep : kNone, 0, 0));
+          }
         }
       }
     }
@@ -265,7 +289,10 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
   }
 }
 
-bool corr_bwd_split_supported(int Cs, int ostep) { return Cs > 64 && Cs <= 16 * kCorrNT && (ostep == 1 || ostep == -1); }
+// A row of G is addressed with 32-bit byte offsets, also a tile past its end.
+bool corr_bwd_split_supported(int Cs, int W, int D, int ostep) {
+  return Cs > 64 && Cs <= 16 * kCorrNT && (ostep == 1 || ostep == -1) && ((long)W + 1024) * D <= 0x7fffffffL / 4;
+}
 
 template <typename T>
 static void launch(CorrBwdArgs a, hipStream_t st) {

@@ -16,7 +16,7 @@ struct CorrBwdArgs {
   int tiles;      // pixel tiles per row (set by the launch)
 };
 
-bool corr_bwd_split_supported(int Cs, int ostep);
+bool corr_bwd_split_supported(int Cs, int W, int D, int ostep);
 void corr_bwd_split(const CorrBwdArgs& a, int precision, hipStream_t st);
 
 }  // namespace ccs
