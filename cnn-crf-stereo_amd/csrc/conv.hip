@@ -45,11 +45,14 @@ constexpr int RPB = 32;
 __host__ __device__ __forceinline__ int bswz(int n, int g) { return g ^ ((n >> 1) & 3); }
 // f32 layout: [q][kk < 4][n] (n contiguous).
 
+// adj: the filters of the input gradient, Wt[n][c][a][b] = w[c][n][KH-1-a][KW-1-b]
+// (w holds C x K x KH x KW).
 __device__ __forceinline__ float flipped_weight(const float* __restrict__ w, int n, int c, int tap, int K, int C,
-                                                int KH, int KW) {
+                                                int KH, int KW, int adj) {
   const int taps = KH * KW;
   if (n >= K || c >= C || tap >= taps) return 0.f;
   const int i = tap / KW, j = tap % KW;
+  if (adj) return w[(((long)c * K + n) * KH + i) * KW + j];
   return w[(((long)n * C + c) * KH + (KH - 1 - i)) * KW + (KW - 1 - j)];
 }
 
@@ -68,7 +71,7 @@ __host__ __device__ constexpr int packed_chunks(int CG, int taps) {
 }
 
 __global__ void k_pack_bf16(const float* __restrict__ w, int K, int C, int Cs, int KH, int KW, int NQ, int NP,
-                            bf16* __restrict__ out) {
+                            int adj, bf16* __restrict__ out) {
   const long total = (long)NQ * NP * RPB;
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
@@ -81,11 +84,11 @@ __global__ void k_pack_bf16(const float* __restrict__ w, int K, int C, int Cs, i
   const int kg = 4 * (q - (st ? stage_nq(CG, taps, 0) : 0)) + bswz(n, kk / 8);  // the swizzle is an involution
   const int tap = kg < taps * ng ? kg / ng : taps;  // taps: a padding group (zero)
   const int c = (stage_cg0(CG, st) + kg % ng) * 8 + kk % 8;
-  out[idx] = f32_to_bf16(flipped_weight(w, n, c, tap, K, C, KH, KW));
+  out[idx] = f32_to_bf16(flipped_weight(w, n, c, tap, K, C, KH, KW, adj));
 }
 
 __global__ void k_pack_f32(const float* __restrict__ w, int K, int C, int Cs, int KH, int KW, int NQ, int NP,
-                           float* __restrict__ out) {
+                           int adj, float* __restrict__ out) {
   const long total = (long)NQ * 4 * NP;
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
@@ -93,7 +96,7 @@ __global__ void k_pack_f32(const float* __restrict__ w, int K, int C, int Cs, in
   const int kk = (int)((idx / NP) % 4);
   const int q = (int)(idx / ((long)NP * 4));
   const int k = q * 4 + kk;
-  out[idx] = flipped_weight(w, n, k % Cs, k / Cs, K, C, KH, KW);
+  out[idx] = flipped_weight(w, n, k % Cs, k / Cs, K, C, KH, KW, adj);
 }
 
 // ---------------------------------------------------------------------------
@@ -880,24 +883,42 @@ extern "C" size_t ccs_conv_packed_bytes(int K, int C, int KH, int KW, int precis
   return packed_bytes(K, C, KH, KW, precision);
 }
 
-extern "C" int ccs_conv_pack_weights(ccs_handle_t h, const float* w, int K, int C, int KH, int KW, int precision,
-                                     void* packed) {
-  CCS_CHECK(h && w && packed, CCS_ERR_ARG, "ccs_conv_pack_weights: NULL argument");
-  CCS_CHECK(K >= 1 && C >= 1 && KH >= 1 && KW >= 1, CCS_ERR_ARG, "ccs_conv_pack_weights: bad shape");
-  CCS_CHECK(precision == CCS_FP32 || precision == CCS_BF16, CCS_ERR_ARG, "ccs_conv_pack_weights: bad precision");
+static void pack_weights(const float* w, int K, int C, int KH, int KW, int precision, int adj, void* packed,
+                         hipStream_t st) {
   const int Cs = feature_stride(C);
   const int NP = 16 * ((K + 15) / 16);
   if (precision == CCS_BF16) {
     const int NQ = packed_chunks(Cs / 8, KH * KW);
     const long total = (long)NQ * NP * RPB;
-    k_pack_bf16<<<ceil_div(total, 256), 256, 0, h->stream>>>(w, K, C, Cs, KH, KW, NQ, NP, (bf16*)packed);
+    k_pack_bf16<<<ceil_div(total, 256), 256, 0, st>>>(w, K, C, Cs, KH, KW, NQ, NP, adj, (bf16*)packed);
   } else if (split_supported(K, C, KH, KW)) {
-    split_pack(w, K, C, KH, KW, packed, h->stream);
+    split_pack(w, K, C, KH, KW, adj, packed, st);
   } else {
     const int NQ = (KH * KW * Cs + 3) / 4;
     const long total = (long)NQ * 4 * NP;
-    k_pack_f32<<<ceil_div(total, 256), 256, 0, h->stream>>>(w, K, C, Cs, KH, KW, NQ, NP, (float*)packed);
+    k_pack_f32<<<ceil_div(total, 256), 256, 0, st>>>(w, K, C, Cs, KH, KW, NQ, NP, adj, (float*)packed);
   }
+}
+
+extern "C" int ccs_conv_pack_weights(ccs_handle_t h, const float* w, int K, int C, int KH, int KW, int precision,
+                                     void* packed) {
+  CCS_CHECK(h && w && packed, CCS_ERR_ARG, "ccs_conv_pack_weights: NULL argument");
+  CCS_CHECK(K >= 1 && C >= 1 && KH >= 1 && KW >= 1, CCS_ERR_ARG, "ccs_conv_pack_weights: bad shape");
+  CCS_CHECK(precision == CCS_FP32 || precision == CCS_BF16, CCS_ERR_ARG, "ccs_conv_pack_weights: bad precision");
+  pack_weights(w, K, C, KH, KW, precision, 0, packed, h->stream);
+  CCS_LAUNCH_CHECK();
+  return CCS_OK;
+}
+
+int ccs::conv_input_gradient(ccs_handle_t h, const void* dz, int H, int W, int K, const float* w, int C, int KH,
+                             int KW, int precision, void* dx, bool* done) {
+  const ConvShape s{H, W, K, C, KH, KW};
+  *done = mfma_supported(s);
+  if (!*done) return CCS_OK;
+  int rc = h->conv_w.reserve(packed_bytes(C, K, KH, KW, precision), h->stream);
+  if (rc) return rc;
+  pack_weights(w, C, K, KH, KW, precision, 1, h->conv_w.ptr, h->stream);
+  launch_mfma(s, precision, dz, h->conv_w.ptr, nullptr, 0, dx, h->stream);
   CCS_LAUNCH_CHECK();
   return CCS_OK;
 }

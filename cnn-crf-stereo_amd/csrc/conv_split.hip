@@ -71,7 +71,7 @@ __host__ __device__ inline void split_step(int q, int lgrp, int* tap, int* c0) {
 // Packed layout: [q][t][plane][lane][8], the fragment of channel tile t, with
 // lane (lrow, lgrp) holding output channel 16 t + lrow.  One thread per lane.
 template <class Cfg>
-__global__ void k_pack_split(const float* __restrict__ w, int K, int C, bf16* __restrict__ out) {
+__global__ void k_pack_split(const float* __restrict__ w, int K, int C, int adj, bf16* __restrict__ out) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= Cfg::NQ * Cfg::NT * 64) return;
   const int lane = idx & 63, t = (idx >> 6) % Cfg::NT, q = (idx >> 6) / Cfg::NT;
@@ -84,8 +84,10 @@ __global__ void k_pack_split(const float* __restrict__ w, int K, int C, bf16* __
   for (int e = 0; e < 8; ++e) {
     const int c = c0 + e;
     const int i = tap / Cfg::KW, j = tap % Cfg::KW;
+    // adj: Wt[n][c] flipped, Wt[n][c][a][b] = w[c][n][KH-1-a][KW-1-b]
     v[e] = n < K && c0 >= 0 && c < C
-               ? w[(((long)n * C + c) * Cfg::KH + (Cfg::KH - 1 - i)) * Cfg::KW + (Cfg::KW - 1 - j)]
+               ? w[adj ? (((long)c * K + n) * Cfg::KH + i) * Cfg::KW + j
+                       : (((long)n * C + c) * Cfg::KH + (Cfg::KH - 1 - i)) * Cfg::KW + (Cfg::KW - 1 - j)]
                : 0.f;
   }
   split3(v, p[0], p[1], p[2]);
@@ -313,10 +315,10 @@ size_t split_packed_bytes(int K, int C, int KH, int KW) {
   return n;
 }
 
-void split_pack(const float* w, int K, int C, int KH, int KW, void* packed, hipStream_t st) {
+void split_pack(const float* w, int K, int C, int KH, int KW, int adj, void* packed, hipStream_t st) {
   with_split_cfg(K, C, KH, KW, [&](auto cfg) {
     using Cfg = decltype(cfg);
-    k_pack_split<Cfg><<<ceil_div((long)Cfg::NQ * Cfg::NT * 64, 256), 256, 0, st>>>(w, K, C, (bf16*)packed);
+    k_pack_split<Cfg><<<ceil_div((long)Cfg::NQ * Cfg::NT * 64, 256), 256, 0, st>>>(w, K, C, adj, (bf16*)packed);
   });
 }
 

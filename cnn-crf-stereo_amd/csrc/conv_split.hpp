@@ -9,9 +9,17 @@ namespace ccs {
 // split kernel: the 100-channel layers (3x3 and 2x2) and the 64-channel 3x3 one.
 bool split_supported(int K, int C, int KH, int KW);
 size_t split_packed_bytes(int K, int C, int KH, int KW);
-void split_pack(const float* w, int K, int C, int KH, int KW, void* packed, hipStream_t st);
+// adj: the filters of the input gradient, w holding C x K x KH x KW.
+void split_pack(const float* w, int K, int C, int KH, int KW, int adj, void* packed, hipStream_t st);
 void split_launch(const float* x, int H, int W, int C, const void* packed, const float* b, int K, int KH, int KW,
                   int act, float* y, hipStream_t st);
+
+// Input gradient of a layer with filters w (K x C x KH x KW) on the MFMA
+// forward kernels: dx (C channels) = true convolution of the padded dz (H x W,
+// K channels) with Wt[c][k][a][b] = w[k][c][KH-1-a][KW-1-b].  *done is false
+// (and nothing is queued) where the shape has no MFMA kernel.  (conv.hip)
+int conv_input_gradient(ccs_handle_t h, const void* dz, int H, int W, int K, const float* w, int C, int KH, int KW,
+                        int precision, void* dx, bool* done);
 
 // x = h + m + l in bfloat16, exactly for every finite float32 down to l's
 // underflow: h is x rounded to nearest, m the residual x - h rounded to nearest

@@ -6,8 +6,9 @@
 //   dW[k][c][KH-1-i][KW-1-j] = sum_p dz[p][k] x[p + (i,j)][c]
 //   dx = true convolution of dz zero-padded by (KH-1, KW-1) with
 //        Wt[c][k][a][b] = W[k][c][KH-1-a][KW-1-b]
-// dW runs on v_mfma_f32_16x16x4_f32 (k_dw_mfma: per tap, a K x C GEMM reduced
-// over pixels), dx on the forward MFMA kernels.  Maps are float32 or bfloat16
+// dW runs on the bf16 matrix cores (conv_grad.hip) for equal types and 65 to 112
+// channels on both sides, on v_mfma_f32_16x16x4_f32 (k_dw_mfma: per tap, a K x C
+// GEMM reduced over pixels) elsewhere, dx on the forward MFMA kernels.  Maps are float32 or bfloat16
 // (the BF16 form keeps activations and activation gradients in bf16 and
 // accumulates in float32).  Reductions over pixels are split into blocks and
 // summed in a fixed order: results do not depend on scheduling.
@@ -15,6 +16,8 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "conv_grad.hpp"
+#include "conv_split.hpp"
 
 namespace ccs {
 
@@ -23,25 +26,59 @@ __device__ __forceinline__ float ldf(const T* p, long i) {
   return (float)p[i];
 }
 
-// dz = dy (1 - y^2) (act) or dy for the K live channels, 0 in the pad
-// channels, and the bias-gradient partials: block b takes pixels
-// [b chunk, (b+1) chunk), thread c channel c, and writes the sum of its stored
-// (rounded) dz values to part[c][b] (channel-major, for k_reduce_cols).
-template <typename T>
-__global__ void k_dz_db(const T* __restrict__ y, const T* __restrict__ dy, long P, int Cs, int K, int act, int chunk,
-                        T* __restrict__ dz, float* __restrict__ part) {
+// dz = dy (1 - y^2) (act) or dy for the K live channels, 0 in the pad channels,
+// written into a map padded by py rows and px columns of zeros on every side
+// (what the input gradient's convolution reads; py = px = 0 without it), and the
+// bias-gradient partials: block b takes padded pixels [b chunk, (b+1) chunk) and
+// writes the sum of its stored (rounded) dz values to part[c][b] (channel-major,
+// for k_reduce_cols).  A thread keeps one group of V channels (16 bytes, or one
+// channel where y or dy is not aligned to that) and steps over the pixels.
+// Bound by memory; 524 x 268 x 100 bf16: 19 us, the scalar form and the separate
+// padding pass took 31 + 33 us.
+template <typename T, int V>
+__global__ __launch_bounds__(256) void k_dz_pad(const T* __restrict__ y, const T* __restrict__ dy, int Ho, int Wo,
+                                                int Cs, int K, int act, int py, int px, int chunk,
+                                                T* __restrict__ dz, float* __restrict__ part) {
+  typedef __attribute__((ext_vector_type(V))) T vec;
+  const int Wp = Wo + 2 * px;
+  const long P = (long)(Ho + 2 * py) * Wp;
   const long p0 = (long)blockIdx.x * chunk;
-  const long p1 = p0 + chunk < P ? p0 + chunk : P;
-  for (int c = threadIdx.x; c < Cs; c += blockDim.x) {
-    float s = 0.f;
-    for (long p = p0; p < p1; ++p) {
-      const long i = p * Cs + c;
-      const float yv = ldf(y, i), g = ldf(dy, i);
-      const T t = (T)(c < K ? (act ? g * (1.f - yv * yv) : g) : 0.f);
-      dz[i] = t;
-      s += (float)t;
+  const int np = (int)(p0 + chunk < P ? chunk : P - p0);
+  const int G = Cs / V, Gb = G < 256 ? G : 256, lanes = 256 / Gb;  // groups side by side, pixels at a time
+  const int gl = threadIdx.x % Gb, pl = threadIdx.x / Gb;
+  __shared__ float sh[256 * V];
+  for (int g0 = 0; g0 < G; g0 += Gb) {
+    const int g = g0 + gl;
+    float s[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) s[e] = 0.f;
+    if (pl < lanes && g < G) {
+      for (int i = pl; i < np; i += lanes) {
+        const long p = p0 + i;
+        const int yy = (int)(p / Wp) - py, xx = (int)(p % Wp) - px;
+        const bool in = yy >= 0 && yy < Ho && xx >= 0 && xx < Wo;
+        const long src = in ? (((long)yy * Wo + xx) * Cs + g * V) : 0;
+        const vec yv = *reinterpret_cast<const vec*>(y + src), gv = *reinterpret_cast<const vec*>(dy + src);
+        vec o;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          const float yf = (float)yv[e], gf = (float)gv[e];
+          const T t = (T)(in && g * V + e < K ? (act ? gf * (1.f - yf * yf) : gf) : 0.f);
+          o[e] = t;
+          s[e] += (float)t;
+        }
+        *reinterpret_cast<vec*>(dz + p * Cs + g * V) = o;
+      }
     }
-    part[(long)c * gridDim.x + blockIdx.x] = s;
+#pragma unroll
+    for (int e = 0; e < V; ++e) sh[threadIdx.x * V + e] = s[e];
+    __syncthreads();
+    for (int i = threadIdx.x; i < Gb * V; i += 256) {
+      float t = 0.f;
+      for (int l = 0; l < lanes; ++l) t += sh[l * Gb * V + i];
+      if (g0 * V + i < Cs) part[(long)(g0 * V + i) * gridDim.x + blockIdx.x] = t;
+    }
+    __syncthreads();
   }
 }
 
@@ -81,7 +118,7 @@ __global__ void k_reduce_rows(const float* __restrict__ part, int nb, int n, flo
 // per SIMD, so two 7-wave blocks share a CU (LDS: 2 x 57 KB for 7 x 7 tiles).
 template <typename TX, typename T, int KT, int CT>
 __global__ __launch_bounds__(64 * KT, 4) void k_dw_mfma(const TX* __restrict__ x, int Win, int Csx,
-                                                        const T* __restrict__ dz, int Ho, int Wo, int Csk, int KW,
+                                                        const T* __restrict__ dz, int zpitch, int Wo, int Csk, int KW,
                                                         int taps, int nch, int segs_per_row, long nseg, long spc,
                                                         float* __restrict__ part) {
   constexpr int KP = 16 * KT, CP = 16 * CT, NTH = 64 * KT, SEG = 64;
@@ -127,7 +164,7 @@ __global__ __launch_bounds__(64 * KT, 4) void k_dw_mfma(const TX* __restrict__ x
   u32x4 reg[NVMAX];
   auto load = [&](long s) {
     const int ho = (int)(s / segs_per_row), wo0 = (int)(s % segs_per_row) * SEG;
-    const T* zrow = dz + ((long)ho * Wo + wo0) * Csk;
+    const T* zrow = dz + ((long)ho * zpitch + wo0) * Csk;
     const TX* xrow = x + ((long)(ho + ti) * Win + wo0 + tj) * Csx;
 #pragma unroll
     for (int i = 0; i < NVMAX; ++i) {
@@ -183,152 +220,31 @@ __global__ __launch_bounds__(64 * KT, 4) void k_dw_mfma(const TX* __restrict__ x
     for (int e = 0; e < 4; ++e) out[(k0 + 4 * lk + e) * CP + 16 * t + lrow] = acc[t][e];
 }
 
-// Weight gradient of one tap row on bf16 MFMA (bf16 input and dz): the block
-// handles the KW taps (i, 0 .. KW-1) of tap row i for a chunk of 64-pixel
-// segments, one wave per 16-channel tile of K (KT waves), KW x CT accumulator
-// tiles per wave.  A segment's dz and its input row go to LDS transposed
-// (channel-major, pixel-minor bf16), the input once per tap shift j (so every
-// fragment is a 16-byte aligned read): per 32 pixels a wave issues KW x CT
-// v_mfma_f32_16x16x32_bf16 with A[m][p] = dz[p][k0+m], B[p][n] = x[p + j][16t+n].
-// Two LDS buffers alternate: while the MFMAs run on one segment, the next one's
-// vectors (loaded a segment earlier) are written into the other.  The K x C
-// sums of tap (i, j) go to part[chunk][tap], the layout of k_dw_mfma.
-template <int KT, int CT, int KW>
-__global__ __launch_bounds__(64 * KT, 1) void k_dw_bf16(const bf16* __restrict__ x, int Win, int Csx,
-                                                        const bf16* __restrict__ dz, int Ho, int Wo, int Csk, int KH,
-                                                        int nch, int segs_per_row, long nseg, long spc,
-                                                        float* __restrict__ part) {
-  constexpr int KP = 16 * KT, CP = 16 * CT, NTH = 64 * KT, SEG = 64, XPX = SEG + KW - 1;
-  constexpr int ZB = KP * SEG, XB = KW * CP * SEG;  // bf16 elements of one buffer's dz and x parts
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16* lds = reinterpret_cast<bf16*>(lds_raw);  // [buf][ZB + XB]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int b = blockIdx.x, xcd = b & 7, local = b >> 3;
-  const int ti = local % KH, chunk = (local / KH) * 8 + xcd;
-  if (chunk >= nch) return;  // the grid is rounded up to whole groups of 8 chunks
-  const long s0 = (long)chunk * spc;
-  const long s1 = s0 + spc < nseg ? s0 + spc : nseg;
-  for (int i = tid; i < 2 * (ZB + XB) / 2; i += NTH) reinterpret_cast<unsigned*>(lds)[i] = 0u;  // pad channels stay 0
-  const int zvp = Csk / 8, xvp = Csx / 8;  // 16-byte vectors per pixel
-  const int nzv = SEG * zvp, nv = nzv + XPX * xvp;
-  constexpr int NVMAX = (SEG * (KP / 8) + XPX * (CP / 8) + NTH - 1) / NTH;
-  // Per vector slot: pixel, channel group, operand (0 dz, 1 x, -1 none).
-  // Consecutive slots take consecutive pixels of one channel group, so the
-  // transposed 16-bit stores of a wave fill contiguous 128-byte row pieces (no
-  // bank conflicts); the group's strided global reads hit the L1 lines that the
-  // segment's other groups bring in.
-  int vpx[NVMAX], vg[NVMAX], vkind[NVMAX];
-#pragma unroll
-  for (int i = 0; i < NVMAX; ++i) {
-    const int v = tid + i * NTH;
-    if (v < nzv) {
-      vpx[i] = v % SEG; vg[i] = v / SEG; vkind[i] = 0;
-    } else if (v < nv) {
-      vpx[i] = (v - nzv) % XPX; vg[i] = (v - nzv) / XPX; vkind[i] = 1;
-    } else {
-      vpx[i] = vg[i] = 0; vkind[i] = -1;
-    }
-  }
-  u32x4 reg[NVMAX];
-  auto load = [&](long s) {
-    const int ho = (int)(s / segs_per_row), wo0 = (int)(s % segs_per_row) * SEG;
-    const bf16* zrow = dz + ((long)ho * Wo + wo0) * Csk;
-    const bf16* xrow = x + ((long)(ho + ti) * Win + wo0) * Csx;
-#pragma unroll
-    for (int i = 0; i < NVMAX; ++i) {
-      u32x4 r = {0u, 0u, 0u, 0u};
-      if (vkind[i] == 0) {
-        if (wo0 + vpx[i] < Wo) r = *reinterpret_cast<const u32x4*>(zrow + (long)vpx[i] * Csk + vg[i] * 8);
-      } else if (vkind[i] == 1) {
-        if (wo0 + vpx[i] < Win) r = *reinterpret_cast<const u32x4*>(xrow + (long)vpx[i] * Csx + vg[i] * 8);
-      }
-      reg[i] = r;
-    }
-  };
-  // Transposed stores: element e of a vector (channel 8 g + e) goes to row
-  // 8 g + e at the vector's pixel; an input vector at pixel p' goes to shift
-  // copy j at pixel p' - j.
-  auto store = [&](int buf) {
-    bf16* zb = lds + buf * (ZB + XB);
-    bf16* xb = zb + ZB;
-#pragma unroll
-    for (int i = 0; i < NVMAX; ++i) {
-      const unsigned short* e16 = reinterpret_cast<const unsigned short*>(&reg[i]);
-      if (vkind[i] == 0) {
-        unsigned short* d = reinterpret_cast<unsigned short*>(zb) + (vg[i] * 8) * SEG + vpx[i];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) d[e * SEG] = e16[e];
-      } else if (vkind[i] == 1) {
-#pragma unroll
-        for (int j = 0; j < KW; ++j) {
-          const int p = vpx[i] - j;
-          if (p >= 0 && p < SEG) {
-            unsigned short* d = reinterpret_cast<unsigned short*>(xb) + (j * CP + vg[i] * 8) * SEG + p;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) d[e * SEG] = e16[e];
-          }
-        }
-      }
-    }
-  };
-  f32x4 acc[KW][CT];
-#pragma unroll
-  for (int j = 0; j < KW; ++j)
-#pragma unroll
-    for (int t = 0; t < CT; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int lrow = lane & 15, kg = lane >> 4, k0 = 16 * wave;
-  __syncthreads();  // the zero fill is done
-  if (s0 < s1) {
-    load(s0);
-    store(0);
-    if (s0 + 1 < s1) load(s0 + 1);
-  }
-  __syncthreads();
-  for (long s = s0; s < s1; ++s) {
-    const int buf = (int)((s - s0) & 1);
-    const bf16* zb = lds + buf * (ZB + XB);
-    const bf16* xb = zb + ZB;
-    // the next segment into the other buffer (its previous readers finished
-    // before the barrier that ended the last iteration)
-    if (s + 1 < s1) {
-      store(buf ^ 1);
-      if (s + 2 < s1) load(s + 2);
-    }
-#pragma unroll
-    for (int h = 0; h < SEG / 32; ++h) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(zb + (k0 + lrow) * SEG + 32 * h + 8 * kg);
-#pragma unroll
-      for (int j = 0; j < KW; ++j)
-#pragma unroll
-        for (int t = 0; t < CT; ++t) {
-          const bf16x8 bv = *reinterpret_cast<const bf16x8*>(xb + (j * CP + 16 * t + lrow) * SEG + 32 * h + 8 * kg);
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[j][t], 0, 0, 0);
-        }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < KW; ++j) {
-    float* out = part + ((long)chunk * KH * KW + ti * KW + j) * KP * CP;
-#pragma unroll
-    for (int t = 0; t < CT; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[(k0 + 4 * kg + e) * CP + 16 * t + lrow] = acc[j][t][e];
-  }
-}
-
-// dW[k][c][KH-1-i][KW-1-j] = sum over chunks of the (tap = i KW + j) partials.
-__global__ void k_dw_reduce(const float* __restrict__ part, int nch, int taps, int KP, int CP, int K, int C, int KH,
-                            int KW, float* __restrict__ dw) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)K * C * taps) return;
+// dW[k][c][KH-1-i][KW-1-j] = sum over chunks of the (tap = i KW + j) partials:
+// a block takes 64 outputs (consecutive c), four threads each, which sum a
+// quarter of the chunks and are added in order.  (One thread per output left
+// 80 strided loads in a row: 24 us for 80 chunks of a 3x3 layer, 9.5 us now.)
+__global__ __launch_bounds__(256) void k_dw_reduce(const float* __restrict__ part, int nch, int taps, int KP, int CP,
+                                                   int K, int C, int KH, int KW, float* __restrict__ dw) {
+  const long idx = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+  const int quarter = threadIdx.x >> 6;
+  const bool in = idx < (long)K * C * taps;
   const int c = (int)(idx % C);
   const int k = (int)((idx / C) % K);
-  const int tap = (int)(idx / ((long)C * K));
+  const int tap = in ? (int)(idx / ((long)C * K)) : 0;
+  const int per = (nch + 3) / 4, ch0 = quarter * per, ch1 = ch0 + per < nch ? ch0 + per : nch;
+  const float* p = part + ((long)tap * KP + k) * CP + c;
+  const long step = (long)taps * KP * CP;
   float s = 0.f;
-  for (int ch = 0; ch < nch; ++ch) s += part[(((long)ch * taps + tap) * KP + k) * CP + c];
-  const int i = tap / KW, j = tap % KW;
-  dw[(((long)k * C + c) * KH + (KH - 1 - i)) * KW + (KW - 1 - j)] = s;
+  if (in)
+    for (int ch = ch0; ch < ch1; ++ch) s += p[ch * step];
+  __shared__ float sh[4][64];
+  sh[quarter][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (quarter == 0 && in) {
+    const int l = threadIdx.x, i = tap / KW, j = tap % KW;
+    dw[(((long)k * C + c) * KH + (KH - 1 - i)) * KW + (KW - 1 - j)] = (sh[0][l] + sh[1][l]) + (sh[2][l] + sh[3][l]);
+  }
 }
 
 // Partial weight gradient on the VALU, for channel counts beyond the MFMA
@@ -337,8 +253,9 @@ __global__ void k_dw_reduce(const float* __restrict__ part, int nch, int taps, i
 // block's pixel range.  Pixels go through LDS 64 at a time.
 template <typename TX, typename T>
 __global__ __launch_bounds__(256) void k_dw_partial(const TX* __restrict__ x, int Win, int Csx,
-                                                    const T* __restrict__ dz, int Ho, int Wo, int Csk, int K,
-                                                    int C, int KH, int KW, long chunk, float* __restrict__ part) {
+                                                    const T* __restrict__ dz, int zpitch, int Ho, int Wo, int Csk,
+                                                    int K, int C, int KH, int KW, long chunk,
+                                                    float* __restrict__ part) {
   const int tk = threadIdx.x & 15, tc = threadIdx.x >> 4;
   const int k0 = blockIdx.x * 16;
   const int cblocks = (C + 15) / 16;
@@ -356,7 +273,7 @@ __global__ __launch_bounds__(256) void k_dw_partial(const TX* __restrict__ x, in
       float zv = 0.f, xv = 0.f;
       if (p < p1) {
         const int ho = (int)(p / Wo), wo = (int)(p % Wo);
-        if (k0 + e < K) zv = ldf(dz, p * Csk + k0 + e);
+        if (k0 + e < K) zv = ldf(dz, ((long)ho * zpitch + wo) * Csk + k0 + e);
         if (c0 + e < C) xv = ldf(x, ((long)(ho + i) * Win + wo + j) * Csx + c0 + e);
       }
       zs[pl][e] = zv;
@@ -370,17 +287,6 @@ __global__ __launch_bounds__(256) void k_dw_partial(const TX* __restrict__ x, in
   const int k = k0 + tk, c = c0 + tc;
   if (k < K && c < C)
     part[(long)blockIdx.z * K * C * KH * KW + (((long)k * C + c) * KH + (KH - 1 - i)) * KW + (KW - 1 - j)] = acc;
-}
-
-template <typename T>
-__global__ void k_pad_dz(const T* __restrict__ dz, int Ho, int Wo, int Cs, int py, int px, T* __restrict__ out) {
-  const int Hp = Ho + 2 * py, Wp = Wo + 2 * px;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)Hp * Wp * Cs) return;
-  const int c = (int)(idx % Cs);
-  const long p = idx / Cs;
-  const int yy = (int)(p / Wp) - py, xx = (int)(p % Wp) - px;
-  out[idx] = (yy >= 0 && yy < Ho && xx >= 0 && xx < Wo) ? dz[((long)yy * Wo + xx) * Cs + c] : (T)0.f;
 }
 
 // Wt[c][k][a][b] = W[k][c][KH-1-a][KW-1-b]
@@ -402,10 +308,10 @@ using namespace ccs;
 namespace {
 
 template <typename TX, typename T, int KT, int CT>
-void launch_dw_mfma(const TX* x, int W, int Csx, const T* z, int Ho, int Wo, int Csk, int KW, int taps,
+void launch_dw_mfma(const TX* x, int W, int Csx, const T* z, int zpitch, int Wo, int Csk, int KW, int taps,
                     int segs_row, long nseg, long spc, int nch, float* part, hipStream_t st) {
   const unsigned blocks = (unsigned)(8 * taps * ((nch + 7) / 8));  // whole groups of 8 chunks, one per XCD
-  k_dw_mfma<TX, T, KT, CT><<<blocks, 64 * KT, 0, st>>>(x, W, Csx, z, Ho, Wo, Csk, KW, taps, nch, segs_row, nseg, spc,
+  k_dw_mfma<TX, T, KT, CT><<<blocks, 64 * KT, 0, st>>>(x, W, Csx, z, zpitch, Wo, Csk, KW, taps, nch, segs_row, nseg, spc,
                                                       part);
 }
 
@@ -413,11 +319,11 @@ void launch_dw_mfma(const TX* x, int W, int Csx, const T* z, int Ho, int Wo, int
 int dw_tiles(int n) { return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : n <= 7 ? 7 : 0; }
 
 template <typename TX, typename T>
-bool dw_mfma(int KT, int CT, const TX* x, int W, int Csx, const T* z, int Ho, int Wo, int Csk, int KW, int taps,
+bool dw_mfma(int KT, int CT, const TX* x, int W, int Csx, const T* z, int zpitch, int Wo, int Csk, int KW, int taps,
              int segs_row, long nseg, long spc, int nch, float* part, hipStream_t st) {
 #define CCS_DW(kt, ct)                                                                                      \
   if (KT == kt && CT == ct) {                                                                               \
-    launch_dw_mfma<TX, T, kt, ct>(x, W, Csx, z, Ho, Wo, Csk, KW, taps, segs_row, nseg, spc, nch, part, st); \
+    launch_dw_mfma<TX, T, kt, ct>(x, W, Csx, z, zpitch, Wo, Csk, KW, taps, segs_row, nseg, spc, nch, part, st); \
     return true;                                                                                            \
   }
   CCS_DW(7, 7) CCS_DW(7, 1) CCS_DW(4, 4) CCS_DW(4, 1) CCS_DW(1, 1) CCS_DW(2, 2) CCS_DW(2, 1) CCS_DW(1, 2)
@@ -426,29 +332,9 @@ bool dw_mfma(int KT, int CT, const TX* x, int W, int Csx, const T* z, int Ho, in
   return false;
 }
 
-constexpr int kDwSeg = 64;            // output pixels per segment of k_dw_mfma and k_dw_bf16
+constexpr int kDwSeg = 64;            // output pixels per segment of k_dw_mfma
 constexpr int kDwTargetBlocks = 512;  // two resident blocks per CU of the 256: one round
-constexpr int kDwBf16Blocks = 256;    // k_dw_bf16: one 114 KB block per CU
-
-void launch_dw_bf16(const bf16* x, int W, int Csx, const bf16* z, int Ho, int Wo, int Csk, int KH, int KW,
-                    int segs_row, long nseg, long spc, int nch, float* part, hipStream_t st) {
-  const unsigned blocks = (unsigned)(8 * KH * ((nch + 7) / 8));  // whole groups of 8 chunks, one per XCD
-  auto go = [&](auto kwc) {
-    constexpr int kw = decltype(kwc)::value;
-    constexpr size_t lds = 2 * sizeof(bf16) * (112 * 64 + kw * 112 * 64);
-    const auto kern = k_dw_bf16<7, 7, kw>;
-    static bool configured = false;
-    if (!configured) {
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      configured = true;
-    }
-    kern<<<blocks, 64 * 7, lds, st>>>(x, W, Csx, z, Ho, Wo, Csk, KH, nch, segs_row, nseg, spc, part);
-  };
-  if (KW == 3)
-    go(std::integral_constant<int, 3>{});
-  else
-    go(std::integral_constant<int, 2>{});
-}
+constexpr int kDwSplitBlocks = 256;   // k_dw_split: one block per CU (each writes KW tap partials of 50 KB)
 
 // The backward of one layer from its input x (element type TX) and output y
 // (element type T of the precision); dy has y's shape and type, dx x's shape
@@ -459,66 +345,68 @@ int conv_backward(ccs_handle_t h, const TX* x, const T* y, int H, int W, int C, 
   const int Ho = H - KH + 1, Wo = W - KW + 1;
   const int Csx = feature_stride(C), Csk = feature_stride(K);
   const long P = (long)Ho * Wo;
-  const long nz = P * Csk;
   const int taps = KH * KW;
   const size_t wcount = (size_t)K * C * KH * KW;
-  const int Hp = Ho + 2 * (KH - 1), Wp = Wo + 2 * (KW - 1);
   const int KT = dw_tiles((K + 15) / 16), CT = dw_tiles((C + 15) / 16);
   const bool mfma = KT && CT && Csk <= 16 * KT && Csx <= 16 * CT;
-  const int segs_row = (Wo + kDwSeg - 1) / kDwSeg;
+  // Equal types and 65 to 112 channels on both sides: the split kernel (one
+  // block per tap row and chunk); other MFMA shapes: one block per tap and chunk.
+  const bool split = std::is_same<TX, T>::value && KT == 7 && CT == 7 && dw_split_supported(Csx, Csk, KW);
+  const int seg = split ? dw_split_segment(precision) : kDwSeg;
+  const int segs_row = (Wo + seg - 1) / seg;
   const long nseg = (long)Ho * segs_row;
-  // bf16 input and dz with 7 x 7 channel tiles: the tap-row kernel on bf16 MFMA
-  // (one block per tap row and chunk, about one block per CU in all).
-  const bool dw_bf16 = std::is_same<TX, bf16>::value && std::is_same<T, bf16>::value && mfma && KT == 7 &&
-                       CT == 7 && (KW == 2 || KW == 3);
-  const int dw_units = dw_bf16 ? KH : taps;  // blocks per chunk
-  int nch = (int)std::min<long>(nseg, std::max(8, (dw_bf16 ? kDwBf16Blocks : kDwTargetBlocks) / dw_units / 8 * 8));
+  const int dw_units = split ? KH : taps;  // blocks per chunk
+  int nch = (int)std::min<long>(nseg, std::max(8, (split ? kDwSplitBlocks : kDwTargetBlocks) / dw_units / 8 * 8));
   const long spc = (nseg + nch - 1) / nch;
   nch = (int)((nseg + spc - 1) / spc);
   const int nb = 64;  // pixel blocks of the VALU weight gradient
   const long chunk = (P + nb - 1) / nb;
-  const int dz_chunk = 64;  // pixels per block of the bias-gradient partials
-  const int nbz = (int)((P + dz_chunk - 1) / dz_chunk);
-  size_t part_n = (size_t)nbz * Csk + Csk;
-  part_n = std::max(part_n, mfma ? (size_t)nch * taps * 256 * KT * CT : (size_t)nb * wcount);
-  const size_t pad_n = dx ? (size_t)Hp * Wp * Csk : 0;
+  // dz goes into a map padded for the input gradient (unpadded without it).
+  const int py = dx ? KH - 1 : 0, px = dx ? KW - 1 : 0;
+  const int Hp = Ho + 2 * py, Wp = Wo + 2 * px;
+  const long Pp = (long)Hp * Wp;
+  const int dz_chunk = 64;  // padded pixels per block of k_dz_pad
+  const int nbz = (int)((Pp + dz_chunk - 1) / dz_chunk);
+  const size_t part_n =
+      std::max((size_t)nbz * Csk, mfma ? (size_t)nch * taps * 256 * KT * CT : (size_t)nb * wcount);
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-  const size_t need = al(sizeof(T) * nz) + al(sizeof(float) * part_n) + al(sizeof(T) * pad_n) + sizeof(float) * wcount;
+  const size_t need = al(sizeof(T) * Pp * Csk) + al(sizeof(float) * part_n) + sizeof(float) * wcount;
   int rc = h->misc2.reserve(need, h->stream);
   if (rc) return rc;
-  char* base = (char*)h->misc2.ptr;
-  T* z = (T*)base;
-  float* part = (float*)(base + al(sizeof(T) * nz));
-  T* zpad = (T*)((char*)part + al(sizeof(float) * part_n));
-  float* wt = (float*)((char*)zpad + al(sizeof(T) * pad_n));
+  T* zpad = (T*)h->misc2.ptr;
+  float* part = (float*)((char*)zpad + al(sizeof(T) * Pp * Csk));
+  float* wt = (float*)((char*)part + al(sizeof(float) * part_n));
+  const T* z = zpad + ((long)py * Wp + px) * Csk;  // output pixel 0, rows Wp pixels apart
 
-  k_dz_db<T><<<nbz, Csk <= 256 ? (Csk + 63) / 64 * 64 : 256, 0, h->stream>>>(y, dy, P, Csk, K, act, dz_chunk, z,
-                                                                                part);
-  if (db) {
-    k_reduce_cols<<<Csk, 256, 0, h->stream>>>(part, nbz, part + (size_t)nbz * Csk);
-    CCS_HIP(hipMemcpyAsync(db, part + (size_t)nbz * Csk, sizeof(float) * K, hipMemcpyDeviceToDevice, h->stream));
-  }
-  if (dw_bf16) {
-    if constexpr (std::is_same<TX, bf16>::value && std::is_same<T, bf16>::value)
-      launch_dw_bf16(x, W, Csx, z, Ho, Wo, Csk, KH, KW, segs_row, nseg, spc, nch, part, h->stream);
-    k_dw_reduce<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(part, nch, taps, 16 * KT, 16 * CT, K, C, KH, KW,
-                                                                  dw);
-  } else if (mfma) {
-    dw_mfma<TX, T>(KT, CT, x, W, Csx, z, Ho, Wo, Csk, KW, taps, segs_row, nseg, spc, nch, part, h->stream);
-    k_dw_reduce<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(part, nch, taps, 16 * KT, 16 * CT, K, C, KH, KW,
-                                                                  dw);
+  constexpr int V = 16 / (int)sizeof(T);
+  if (((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0)
+    k_dz_pad<T, V><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, part);
+  else
+    k_dz_pad<T, 1><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, part);
+  if (db) k_reduce_cols<<<K, 256, 0, h->stream>>>(part, nbz, db);
+  if (mfma) {
+    if (split)
+      dw_split({x, z, part, W, Csx, Wp, Ho, Wo, Csk, nch, segs_row, nseg, spc}, precision, KH, KW, h->stream);
+    else
+      dw_mfma<TX, T>(KT, CT, x, W, Csx, z, Wp, Wo, Csk, KW, taps, segs_row, nseg, spc, nch, part, h->stream);
+    k_dw_reduce<<<ceil_div((long)wcount, 64), 256, 0, h->stream>>>(part, nch, taps, 16 * KT, 16 * CT, K, C, KH, KW,
+                                                                 dw);
   } else {
     dim3 grid(ceil_div(K, 16), ceil_div(C, 16) * KH * KW, nb);
-    k_dw_partial<TX, T><<<grid, 256, 0, h->stream>>>(x, W, Csx, z, Ho, Wo, Csk, K, C, KH, KW, chunk, part);
+    k_dw_partial<TX, T><<<grid, 256, 0, h->stream>>>(x, W, Csx, z, Wp, Ho, Wo, Csk, K, C, KH, KW, chunk, part);
     k_reduce_rows<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(part, nb, (int)wcount, dw);
   }
   if (dx) {
-    k_pad_dz<T><<<ceil_div((long)Hp * Wp * Csk, 256), 256, 0, h->stream>>>(z, Ho, Wo, Csk, KH - 1, KW - 1, zpad);
-    k_transpose_flip<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(w, K, C, KH, KW, wt);
-    CCS_LAUNCH_CHECK();
-    // dx has C output channels from K input channels.
-    if ((rc = ccs_conv2d_forward(h, zpad, CCS_LAYOUT_NHWC, Hp, Wp, K, wt, nullptr, C, KH, KW, 0, precision, dx)))
-      return rc;
+    // dx has C output channels from K input channels; the MFMA shapes pack the
+    // transposed filters straight from w.
+    bool done = false;
+    if ((rc = conv_input_gradient(h, zpad, Hp, Wp, K, w, C, KH, KW, precision, dx, &done))) return rc;
+    if (!done) {
+      k_transpose_flip<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(w, K, C, KH, KW, wt);
+      CCS_LAUNCH_CHECK();
+      if ((rc = ccs_conv2d_forward(h, zpad, CCS_LAYOUT_NHWC, Hp, Wp, K, wt, nullptr, C, KH, KW, 0, precision, dx)))
+        return rc;
+    }
   }
   CCS_LAUNCH_CHECK();
   return CCS_OK;

@@ -1,0 +1,74 @@
+"""The layer adjoint on split products at the edges of its segments, channel
+tiles and padding, against float64.
+
+dz is formed and rounded in the maps' type, and the reference starts from that
+dz.  Products are exact (float32: but for 2^-26 of each).  A chunk sums n steps
+of 32 pixels, at most six roundings each at the size of its partial sums and
+one more in the running sum, then at most 128 chunks are added:
+|error| <= (8 + n + 128) 2^-24 sum |dz x| for n = ceil(pixels of a chunk / 32).
+"""
+import pytest
+import torch
+
+from cnn_crf_stereo_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def maps(g, H, W, C, dtype, scale=1.0):
+    f = torch.zeros((H, W, capi.feature_stride(C)), device="cuda")
+    f[:, :, :C] = scale * torch.tanh(torch.randn((H, W, C), generator=g, device="cuda"))
+    return f.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,K,k,H,W,aligned", [
+    (100, 100, 3, 3, 3, True),       # one output pixel
+    (100, 100, 3, 5, 34, True),      # one float32 segment
+    (100, 100, 3, 5, 35, True),      # a pixel over
+    (100, 100, 3, 12, 66, True),     # one bfloat16 segment
+    (100, 100, 3, 12, 67, True),
+    (100, 100, 2, 70, 130, True),    # many chunks
+    (65, 112, 3, 9, 40, True),       # fewest and most channels
+    (112, 65, 2, 9, 40, True),
+    (100, 100, 3, 9, 70, False),     # y and dy off 16 bytes: the scalar dz pass
+    (40, 100, 3, 9, 70, True),       # not on the split kernel
+])
+def test_conv_adjoint(handle, C, K, k, H, W, aligned, dtype):
+    g = torch.Generator(device="cuda").manual_seed(C + K + k + H + W)
+    Ho, Wo = H - k + 1, W - k + 1
+    x, y = maps(g, H, W, C, dtype), maps(g, Ho, Wo, K, dtype)
+    dy = maps(g, Ho, Wo, K, dtype, 1e-3)
+    w = torch.randn((K, C, k, k), generator=g, device="cuda") * 0.05
+    if not aligned:
+        shift = lambda t: torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)  # noqa: E731
+        y, dy = shift(y), shift(dy)
+        assert y.data_ptr() % 16 and dy.data_ptr() % 16
+    dx, dw, db = ops.conv2d_backward_stored(handle, x, y, w, dy)
+    dz = (dy.float() * (1.0 - y.float() * y.float())).to(dtype)[:, :, :K].double()  # fused or not: 2^-23 below
+    xd = x[:, :, :C].double()
+    want, size = torch.empty_like(w, dtype=torch.float64), torch.empty_like(w, dtype=torch.float64)
+    for i in range(k):
+        for j in range(k):
+            xs, z = xd[i:i + Ho, j:j + Wo].reshape(-1, C), dz.reshape(-1, K)
+            want[:, :, k - 1 - i, k - 1 - j] = z.t() @ xs
+            size[:, :, k - 1 - i, k - 1 - j] = z.abs().t() @ xs.abs()
+    n = -(-Ho * Wo // 32)
+    unit = 2.0**-23 if dtype == torch.float32 else 2.0**-8  # dz's own rounding may differ by one unit
+    tol = ((8 + n + 128) * 2.0**-24 + (unit if dtype == torch.float32 else 2.0**-20)) * size
+    assert ((dw.double() - want).abs() <= tol).all()
+    assert ((db.double() - dz.sum((0, 1))).abs() <= (n * 32 * 2.0**-24 + unit) * dz.abs().sum((0, 1))).all()
+    # dx: the full correlation of dz with the filters
+    pad = torch.nn.functional.pad(dz.permute(2, 0, 1), (k - 1,) * 4)
+    wantx = torch.zeros((C, H, W), dtype=torch.float64, device="cuda")
+    sizex = torch.zeros_like(wantx)
+    wd = (w if dtype == torch.float32 else w.bfloat16()).double()
+    for i in range(k):
+        for j in range(k):
+            f = wd[:, :, k - 1 - i, k - 1 - j]  # x[p + (i, j)] met this filter entry
+            src = pad[:, k - 1 - i:k - 1 - i + H, k - 1 - j:k - 1 - j + W].reshape(K, -1)
+            wantx += (f.t() @ src).view(C, H, W)
+            sizex += (f.abs().t() @ src.abs()).view(C, H, W)
+    tolx = (64 * 2.0**-24 + unit) * sizex + (2.0**-8 * wantx.abs() if dtype == torch.bfloat16 else 0)
+    assert ((dx[:, :, :C].permute(2, 0, 1).double() - wantx).abs() <= tolx).all()
+    assert torch.count_nonzero(dx[:, :, C:]).item() == 0
