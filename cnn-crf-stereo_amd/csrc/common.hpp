@@ -82,10 +82,7 @@ constexpr int kXentBlocks = 4096;
 // Half-steps of a CRF run whose per-chain sums are kept before one launch adds
 // them up, and the doubles that takes (minima and constants of max(H, W) chains).
 constexpr int kSumSlots = 64;
-inline size_t run_chain_doubles(int nmax, int iters) {
-  const long steps = 2 * (long)iters + 1;
-  return 2 * (size_t)nmax * (steps < kSumSlots ? steps : kSumSlots);
-}
+inline size_t run_chain_doubles(int nmax) { return 2 * (size_t)nmax * kSumSlots; }
 
 inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) / b); }
 

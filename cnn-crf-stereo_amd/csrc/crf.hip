@@ -312,13 +312,15 @@ static int run(ccs_handle_t h, const float* cost, const float* wx, const float* 
   CCS_CHECK(iters >= 0 && iters <= 10000, CCS_ERR_ARG, "ccs_slackprop: bad iteration count %d", iters);
   const size_t vol = (size_t)H * W * D, bytes = vol * sizeof(float);
   // The state lives in unaries_out where the caller wants the final unaries
-  // (no copy at the end), unless that overlaps the costs every sweep reads.
+  // (no copy at the end), unless that overlaps the costs every sweep reads.  The
+  // handle's own volume is reserved either way, so that after one run any call
+  // of these sizes can be captured.
   const uintptr_t u0 = (uintptr_t)unaries_out, c0 = (uintptr_t)cost;
   const bool own = !unaries_out || (u0 < c0 + bytes && c0 < u0 + bytes);
-  if (own && (rc = h->crf_a.reserve(bytes, h->stream))) return rc;
+  if ((rc = h->crf_a.reserve(bytes, h->stream))) return rc;
   if ((rc = h->crf_sums.reserve(sizeof(double) * (4 * (size_t)iters + 2), h->stream))) return rc;
   const int nmax = H > W ? H : W;
-  if ((rc = h->crf_small.reserve(sizeof(double) * run_chain_doubles(nmax, iters), h->stream))) return rc;
+  if ((rc = h->crf_small.reserve(sizeof(double) * run_chain_doubles(nmax), h->stream))) return rc;
   float* A = own ? (float*)h->crf_a.ptr : unaries_out;
   double* S = sums ? sums : (double*)h->crf_sums.ptr;  // S_0 .. S_{2 iters}
   double* K = S + 2 * iters + 1;                       // K_0 .. K_{2 iters - 1}

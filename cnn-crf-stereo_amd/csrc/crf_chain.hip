@@ -37,6 +37,23 @@ static long seg_min_bytes() {
   return v;
 }
 
+template <int LPL>
+static int launch_mode(ChainMode mode, ChainArgs& a, bool seg, hipStream_t st) {
+  switch (mode) {
+    case kRowsMinorant: return launch_labels<LPL, kRowsMinorant>(a, seg, st);
+    case kColsMinorant: return launch_labels<LPL, kColsMinorant>(a, seg, st);
+    case kRowsDecode: return launch_labels<LPL, kRowsDecode>(a, seg, st);
+  }
+  return fail(CCS_ERR_ARG, "unknown chain mode %d", (int)mode);
+}
+
+// The sweeps stream the costs where the cost and the state volume together are
+// larger than the last-level cache: a sweep reads the costs once and the unaries
+// twice, so keeping costs there only displaces unaries (measured, a row and a
+// column sweep: 450 -> 432 us at 1242x375x128, 2763 -> 2710 us at 1488x992x256;
+// where both fit, streaming costs 2-3 %: 185 -> 190 us at 320x240x256).
+constexpr long kStreamMinBytes = 128l << 20;
+
 int launch_chain(ChainMode mode, ChainArgs& a, hipStream_t st) {
   if (mode != kColsMinorant) {  // row chains are addressed with 32-bit byte offsets
     const long extent = ((long)(a.n - 1) * a.pns * a.D + a.D) * (long)sizeof(float);
@@ -46,6 +63,7 @@ int launch_chain(ChainMode mode, ChainArgs& a, hipStream_t st) {
   }
   bool seg = false;
   const long vol = (long)a.n_chains * a.n * a.D * (long)sizeof(float);
+  a.stream = vol > kStreamMinBytes;
   if (mode == kColsMinorant && kSeg > 0) {
     // A segment's nodes are addressed with 32-bit byte offsets from its first node.
     const long span = ((long)(kSeg - 1) * a.pns * a.D + a.D) * (long)sizeof(float);
@@ -59,9 +77,9 @@ int launch_chain(ChainMode mode, ChainArgs& a, hipStream_t st) {
   const size_t row_lds = row_seg_lds(lpl, pe, a.n);
   const bool row_seg = kSeg > 0 && vol >= seg_min_bytes() && row_lds <= kLdsPerCu;
   seg = mode == kColsMinorant ? seg : mode == kRowsMinorant && row_seg;
-  if (a.D <= 64) return launch_labels<1>(mode, a, seg, st);
-  if (a.D <= 128) return launch_labels<2>(mode, a, seg, st);
-  return launch_labels<4>(mode, a, seg, st);
+  if (a.D <= 64) return launch_mode<1>(mode, a, seg, st);
+  if (a.D <= 128) return launch_mode<2>(mode, a, seg, st);
+  return launch_mode<4>(mode, a, seg, st);
 }
 
 }  // namespace ccs

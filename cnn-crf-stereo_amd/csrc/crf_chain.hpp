@@ -26,6 +26,7 @@ struct ChainArgs {
   long pcs, pns;       // pixel index = chain * pcs + node * pns
   int n_chains, n, D, delta;
   float L1, L2;
+  bool stream = false;  // the costs are read without being kept in the caches (set by launch_chain)
 };
 
 // Column sweeps of large volumes keep the backward messages of every
@@ -56,9 +57,9 @@ constexpr size_t row_seg_lds(int lpl, bool per_edge, int n) {
 // Compute units of the current device.
 int cu_count();
 
-// One sweep for LPL (1, 2 or 4) labels per lane; seg: the checkpointed schemes.
-template <int LPL>
-int launch_labels(ChainMode mode, ChainArgs& a, bool seg, hipStream_t st);
+// One sweep of MODE for LPL (1, 2 or 4) labels per lane; seg: the checkpointed schemes.
+template <int LPL, int MODE>
+int launch_labels(ChainArgs& a, bool seg, hipStream_t st);
 
 // Launches one sweep of `mode` over all chains of `a` on `st`.
 int launch_chain(ChainMode mode, ChainArgs& a, hipStream_t st);

@@ -42,6 +42,9 @@
 // value it reads, which the host turns into a status code.
 #pragma once
 
+#include <type_traits>
+#include <utility>
+
 #include "crf_chain.hpp"
 
 namespace ccs {
@@ -225,13 +228,23 @@ __device__ __forceinline__ void pin(Vec<LPL>& x) {
   for (int j = 0; j < LPL; ++j) asm volatile("" : "+v"(x.v[j]));
 }
 
+// f(integral_constant 0) ... f(integral_constant N-1): steps whose position is a
+// compile-time constant.
+template <int... I, typename F>
+__device__ __forceinline__ void unroll_seq(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unroll_steps(F&& f) {
+  unroll_seq(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
+}
+
 // Minimum over the 64 lanes of a value, left in every lane.  A wave alone on
-// its SIMD takes 8 cycles per dependent VALU instruction and 4 per issue slot
-// (measured, stand-alone), so the tree's length is what a sweep's step costs:
-// four DPP levels inside each row of 16 lanes (16 cycles each with their wait
-// states), then the four rows' minima through v_readlane (36 cycles in all;
-// v_permlane16_swap and v_permlane32_swap, with their copies and wait states,
-// take 57).
+// its SIMD takes 4 cycles per instruction (measured, stand-alone), wait states
+// included, so the tree's length is what a sweep's step costs: four DPP levels
+// inside each row of 16 lanes (two wait states before each), then the four rows'
+// minima through v_readlane: 9 instructions against 10 with v_permlane16_swap
+// and v_permlane32_swap, whose copies and wait states cannot be filled.
 __device__ __forceinline__ float rows_min(float x) {
   auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); };
   const float s0 = row(0), s1 = row(16), s2 = row(32), s3 = row(48);
@@ -548,22 +561,26 @@ __device__ __forceinline__ Rsrc chain_rsrc(const float* base, long nfloats) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(nfloats * 4), 0x00020000);
 }
 
-template <int LPL, int FIT>
+// AUX: cache policy of the access (0, or kStream for costs that a sweep reads
+// once and that do not stay in the cache until the next one: they then leave the
+// cached part to the unaries, which every sweep reads twice).
+constexpr int kStream = 2;  // non-temporal
+template <int LPL, int FIT, int AUX = 0>
 __device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D, float fill) {
   Vec<LPL> out;
   if constexpr (FIT != kFitAny) {
     const bool ok = FIT == kFitFull || lane * LPL < D;
     const int voff = (FIT == kFitFull ? lane * LPL : min(lane * LPL, D - LPL)) * 4;
     if constexpr (LPL == 4) {
-      const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+      const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, AUX);
 #pragma unroll
       for (int j = 0; j < 4; ++j) out.v[j] = __uint_as_float(t[j]);
     } else if constexpr (LPL == 2) {
-      const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+      const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, AUX);
       out.v[0] = __uint_as_float(t[0]);
       out.v[1] = __uint_as_float(t[1]);
     } else {
-      out.v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+      out.v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, AUX));
     }
 #pragma unroll
     for (int j = 0; j < LPL; ++j) out.v[j] = ok ? out.v[j] : fill;
@@ -571,7 +588,7 @@ __device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D, fl
 #pragma unroll
     for (int j = 0; j < LPL; ++j) {
       const int s = lane * LPL + j;
-      const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (s < D ? s : D - 1) * 4, soff, 0));
+      const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (s < D ? s : D - 1) * 4, soff, AUX));
       out.v[j] = s < D ? v : fill;
     }
   }
@@ -673,7 +690,9 @@ __device__ double chain_kept(const float* v, const double* b, int n, int lane, d
 // of registers and the load for node s + P is issued right after slot s is read
 // (clamped to the last node, so it never leaves the chain).  The last partial
 // block is an unrolled tail that issues no loads.
-template <int LPL, int MODE, int P, int FIT, int DC, bool SEG, bool NANCHK, bool PE>
+//
+// SEG: 0 every message is stored; 1 checkpointed; 2 checkpointed, costs streamed.
+template <int LPL, int MODE, int P, int FIT, int DC, int SEG, bool NANCHK, bool PE>
 __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_chain(ChainArgs a) {
   extern __shared__ double lds_all[];
   constexpr bool kCols = MODE == kColsMinorant;
@@ -682,7 +701,8 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
   // 256 threads runs two chains (waves 0-1 and 2-3, each with its own LDS), so
   // that between one and two times as many chains as CUs need not put two
   // workgroups on a CU.
-  constexpr bool kRowSeg = !kCols && SEG;
+  constexpr bool kRowSeg = !kCols && SEG != 0;
+  constexpr int kCostAux = SEG == 2 ? kStream : 0;
   constexpr int KR = kRowSeg ? seg_len<LPL>() : 1;
   static_assert(!kRowSeg || P == kRowRing * KR, "the forward ring spans the message ring");
   static_assert(P <= 64, "one weight per lane and step of a block");
@@ -897,7 +917,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 #pragma unroll
     for (int k = 0; k < LPL; ++k) bh.v[k] = keep(k) ? m.v[k] - u : 0.f;
     if constexpr (kCols) {
-      constexpr int K = SEG ? seg_len<LPL>() : 0;
+      constexpr int K = SEG != 0 ? seg_len<LPL>() : 0;
       if (K == 0 || i % K == 0) st_node<LPL, FIT>(msg + (long)i * D, lane, D, bh);  // i is wave-uniform
     } else if constexpr (kRowSeg) {
       if (ck) st_buf<LPL, FIT>(rM, i * D * 4, lane, D, bh);
@@ -1063,7 +1083,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 #pragma unroll
         for (int j = 0; j < P; ++j) {
           ra[j] = ld_buf<LPL, FIT>(rA, node_a(j < P - 1 ? j : -1) * strideB, lane, D, kInfF);
-          rc[j] = ld_buf<LPL, FIT>(rC, node_c(j) * strideB, lane, D, kInfF);
+          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, node_c(j) * strideB, lane, D, kInfF);
         }
         lds_barrier();  // segments 0 and 1 are in the ring
         bm[0] = ld_ring<LPL>(ring, lane);
@@ -1094,7 +1114,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
         if (!TAIL) {
           // C_i and A_i are read: their slots take C of step ip + P and A of
           // step ip - 1 + P.
-          rc[j] = ld_buf<LPL, FIT>(rC, __builtin_amdgcn_readlane(ao, j) - strideB, lane, D, kInfF);
+          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, __builtin_amdgcn_readlane(ao, j) - strideB, lane, D, kInfF);
           ra[jp] = ld_buf<LPL, FIT>(rA, j > 0 ? __builtin_amdgcn_readlane(ao, j - 1) : __builtin_amdgcn_readlane(aop, P - 1),
                                      lane, D, kInfF);
         }
@@ -1125,7 +1145,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 #pragma unroll
       for (int j = 0; j < P; ++j) fstep(i0p, 0, 0, j, true, true);
     } else
-    if constexpr (kCols && SEG && seg_len<LPL>() > 0) {
+    if constexpr (kCols && SEG != 0 && seg_len<LPL>() > 0) {
       // Segments of K forward steps i0 .. i0+K-1.  Their nodes i0+1 .. i0+K
       // (unaries and costs), the checkpoint Bh_{min(i0+K, n-1)} (Bh_{n-1} = 0
       // is stored) and the segment's minima u_i and weights w_i (one per lane)
@@ -1153,7 +1173,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
         for (int t = 0; t < K; ++t) {
           const int off = min(t, n - 1 - first) * strideB;
           B.a[t] = ld_buf<LPL, FIT>(sA, off, lane, D, kInfF);
-          B.c[t] = ld_buf<LPL, FIT>(sC, off, lane, D, kInfF);
+          B.c[t] = ld_buf<LPL, FIT, kCostAux>(sC, off, lane, D, kInfF);
         }
         B.m = ld_node<LPL, FIT>(msg + (long)min(i0 + K, nb) * D, lane, D, 0.f);
         const int e = max(min(i0 + lane, n - 2), 0);
@@ -1259,6 +1279,412 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
       a.lam[c] = Lambda;
       a.kept[c] = kept;
     }
+  }
+}
+
+// Chain sweep on three waves per chain (delta = 2), for the sweeps whose time is
+// the steps of one resident set of chains and not the bytes they move
+// (use_line()).
+//
+// A wave alone on its SIMD pays 4 cycles for every instruction, dependent or
+// not, but 16-24 for a global load or store, 16-20 for an LDS store and 12 for
+// an LDS read (measured, stand-alone).  A forward step of k_chain spends 100 of
+// its 304 cycles on its memory instructions (two loads, a store, an LDS read and
+// an LDS store; 128 ns measured at 1242 x 375 x 128).  Here the chain wave
+// touches no global memory in its forward pass: 47 instructions, one LDS read
+// and one LDS store per step (103 ns).
+//
+//   Backward pass (chain wave): theta through a register ring, every K-th
+//     message stored as a checkpoint (end-aligned, at nodes n-1 - m K).  The
+//     per-node minimum is kept in a register: one DPP move writes it to the
+//     step's quad of lanes, and 16 steps' values go to LDS at once.
+//   Forward pass, in segments of K steps (forward step i' = i + g of node i, g
+//     virtual steps align the segments with the checkpoints).  Between barriers
+//     q and q + 1
+//       the chain wave runs segment q: it reads (Bh_i, theta_{i+1}) as one vector
+//         from an LDS ring of three segments, two steps ahead, and writes its
+//         result (rows: A'_i = A_i - g_i; columns: g_i) to a ring of two;
+//       the output wave stores segment q - 1 (rows: C_i - A'_i; columns:
+//         (C_i - B_i) + g_i);
+//       the message wave recomputes the messages of segment q + 2 from the
+//         checkpoint at its end into the slot that segment q - 1 has left, with
+//         the backward step's own operations and operands, so they are the
+//         messages it formed, bit for bit.
+//
+// Loads run 4 (costs) and 6 segments (theta) ahead: 1242 x 256 chains of 128
+// labels 242 -> 237 us against 2 and 3.  Up to two chains per CU share a
+// workgroup of eight waves, two of them idle: waves go to the four SIMDs in turn,
+// so that each chain wave keeps a SIMD to itself.
+//
+// Measured, one sweep (us, k_chain -> this): rows 320 x 240 x 32 72 -> 54,
+// 744 x 496 x 64 141 -> 120, 1242 x 128 x 128 261 -> 217 (88 of them backward),
+// 1242 x 375 x 128 270 -> 257 (streaming the costs; 954 MB, 3.7 TB/s); columns
+// 320 x 240 x 32 73 -> 43, 744 x 496 x 64 126 -> 100.
+constexpr int kLineK = 8;
+constexpr int kLineRing = 3 * 2 + 2;  // segments of node vectors in the two rings
+enum LineRole { kChain = 0, kMessages = 1, kOut = 2, kIdle = 3 };
+
+// LDS of one chain: b, w, u, v, [w2], rounded to 16 bytes, then the rings.
+constexpr size_t line_lds(int lpl, bool per_edge, int n) {
+  return sizeof(float) *
+         ((((per_edge ? 6 : 5) * (size_t)n + 3) & ~(size_t)3) + (size_t)kLineRing * kLineK * 64 * lpl);
+}
+
+template <int LPL, int FIT, bool PE, bool COLS, bool NANCHK>
+__global__ __launch_bounds__(512) void k_line(ChainArgs a) {
+  extern __shared__ double lds_line[];
+  constexpr int K = kLineK, DC = 2, P = 32, NS = 64 * LPL;
+  const int n = a.n, D = a.D;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool two = blockDim.x > 256;  // two chains in the workgroup
+  const int cs = two ? (wave >> 1) & 1 : 0;
+  const int role = !two ? wave : wave < 4 ? wave & 1 : wave & 1 ? kOut : kIdle;
+  const int c_slot = blockIdx.x * (two ? 2 : 1) + cs;
+  const int c = min(c_slot, a.n_chains - 1);
+  // per chain: b (doubles), w, u, v, [w2], then the rings at a 16-byte boundary
+  const int head = ((PE ? 6 : 5) * n + 3) & ~3;
+  const int chain_floats = head + kLineRing * K * NS;
+  double* b_lds = lds_line + cs * (chain_floats / 2);
+  float* w_lds = reinterpret_cast<float*>(b_lds + n);
+  float* u_lds = w_lds + n;
+  float* v_lds = u_lds + n;
+  float* w2_lds = v_lds + n;  // PE only
+  float* msg_ring = reinterpret_cast<float*>(b_lds) + head;  // [3][K] nodes of 64 x (Bh, theta)
+  float* out_ring = msg_ring + 3 * K * 2 * NS;               // [3][K] nodes
+  ShiftCarry cc;
+  const float L1v = in_vgpr(a.L1), L2v = in_vgpr(a.L2);
+  const long pbase = (long)c * a.pcs;
+  const int strideB = (int)(a.pns * D * 4);
+  const long span = (long)(n - 1) * a.pns * D + D;
+  const Rsrc rT = chain_rsrc((COLS ? a.A : a.A_in) + pbase * D, span);  // theta: the sweep's unaries
+  const Rsrc rC = chain_rsrc(a.cost + pbase * D, span);
+  const Rsrc rW = chain_rsrc(a.A + pbase * D, span);
+  const Rsrc rM = chain_rsrc(a.msg + (long)c * n * D, (long)n * D);
+  const bool valid = FIT == kFitFull || lane * LPL < D;  // this lane has labels
+  const float* __restrict__ wb = a.w + pbase * a.wmul;
+  const float* __restrict__ wb2 = PE ? a.w2 + pbase * a.wmul : nullptr;
+  const long wstep = a.pns * a.wmul;
+  if (role <= kMessages)
+    for (int i = role * 64 + lane; i < n - 1; i += 128) {
+      w_lds[i] = wb[(long)i * wstep];
+      if constexpr (PE) w2_lds[i] = wb2[(long)i * wstep];
+    }
+  const int nb = n - 1, M = (nb + K - 1) / K, g = M * K - nb;
+  __syncthreads();
+  if (role == kIdle || c_slot >= a.n_chains) {  // the same barriers, no work
+    __syncthreads();
+    if (M > 0)
+      for (int q = 0; q <= M; ++q) lds_barrier();
+    return;
+  }
+  auto ld_theta = [&](int node) { return ld_buf<LPL, FIT>(rT, node * strideB, lane, D, kInfF); };
+
+  auto ib = [&](int q) { return q * K - g; };  // node of a segment's first step
+
+  if (role == kOut) {
+    // ---- output wave: the costs run four segments ahead
+    constexpr int F = 4;
+    Vec<LPL> C[F][K], B[COLS ? F : 1][K];
+    auto load = [&](int q, auto k) {
+      constexpr int kk = decltype(k)::value;
+      auto off = [&](int t) { return min(max(ib(min(q, M - 1)) + t, 0), n - 1) * strideB; };
+      if (a.stream) {
+#pragma unroll
+        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT, kStream>(rC, off(t), lane, D, kInfF);
+      } else {
+#pragma unroll
+        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT>(rC, off(t), lane, D, kInfF);
+      }
+      if constexpr (COLS) {
+#pragma unroll
+        for (int t = 0; t < K; ++t) B[kk][t] = ld_buf<LPL, FIT>(rT, off(t), lane, D, kInfF);
+      }
+    };
+    // Stores segment q (q % F = k) after barrier q + 1, then loads segment q + F.
+    auto store = [&](int q, auto k) {
+      constexpr int kk = decltype(k)::value;
+      const float* src = out_ring + (kk % 2) * K * NS;
+      Vec<LPL> r[K];
+#pragma unroll
+      for (int t = 0; t < K; ++t) r[t] = ld_ring<LPL>(src + t * NS, lane);
+#pragma unroll
+      for (int t = 0; t < K; ++t) {
+#pragma unroll
+        for (int e = 0; e < LPL; ++e)
+          r[t].v[e] = COLS ? (C[kk][t].v[e] - B[COLS ? kk : 0][t].v[e]) + r[t].v[e] : C[kk][t].v[e] - r[t].v[e];
+        const int i = ib(q) + t;
+        if (kk != 0 || i >= 0) st_buf<LPL, FIT>(rW, i * strideB, lane, D, r[t]);
+      }
+      load(q + F, k);
+    };
+    __syncthreads();
+    if (M == 0) return;
+    unroll_steps<F>([&](auto k) { load(decltype(k)::value, k); });
+    lds_barrier();  // 0
+    for (int q = 0; q < M; q += F)
+      unroll_steps<F>([&](auto k) {
+        const int qk = q + decltype(k)::value;
+        if (qk < M) {
+          lds_barrier();  // qk + 1
+          store(qk, k);
+        }
+      });
+    return;
+  }
+  if (role == kMessages) {
+    // ---- message wave
+    struct Seg {
+      Vec<LPL> a[K], m;
+      float u, w, w2;
+    };
+    constexpr int F = 6;  // segments in flight
+    Seg T[F];
+    auto load_t = [&](int q, Seg& S) {           // theta of nodes ib + 1 .. ib + K
+#pragma unroll
+      for (int t = 0; t < K; ++t) S.a[t] = ld_theta(min(max(ib(min(q, M - 1)) + t + 1, 1), n - 1));
+    };
+    auto load_m = [&](int q, Seg& S) {  // the checkpoint and the segment's minima and weights, one per lane
+      S.m = ld_buf<LPL, FIT>(rM, min(ib(q) + K, n - 1) * D * 4, lane, D, 0.f);
+      const int e = max(min(ib(q) + lane, n - 2), 0);
+      S.u = u_lds[e];
+      S.w = w_lds[e];
+      S.w2 = PE ? w2_lds[e] : 0.f;
+    };
+    bool nan1 = NANCHK && any_nan(ld_theta(0));
+    if (M > 0) {
+#pragma unroll
+      for (int k = 0; k < F; ++k) load_t(k, T[k]);
+    }
+    __syncthreads();  // the checkpoints and u_lds are visible
+    if (M == 0) {
+      if constexpr (NANCHK) {
+        const bool any = __ballot(nan1) != 0;
+        if (lane == 0) a.nan_flags[c] = any ? 1 : 0;
+      }
+      return;
+    }
+    // The messages of segment q into ring slot q % 3; low: segment 0, which may
+    // start with virtual steps.
+    auto messages = [&](int q, const Seg& S, int slot, bool low) {
+      float* dst = msg_ring + slot * K * 2 * NS + lane * 2 * LPL;
+      Vec<LPL> X = S.m;
+#pragma unroll
+      for (int t = K - 1; t >= 0; --t) {
+        if (!low || ib(q) + t >= 0) {
+          if constexpr (NANCHK) nan1 |= any_nan(S.a[t]);
+          const float u = lane_weight(S.u, t);
+          Vec<LPL> U, nr;
+          near_only<LPL, DC, PE>(U, S.a[t], X, lane_weight(S.w, t), L1v, 2, cc, nr);
+          const Vec<LPL> m =
+              minconv<LPL, PE>(U, nr, u, lane_weight(S.w, t), PE ? lane_weight(S.w2, t) : 0.f, L2v);
+#pragma unroll
+          for (int k = 0; k < LPL; ++k) X.v[k] = m.v[k] - u;
+          float* d = dst + t * 2 * NS;
+          if constexpr (LPL == 2) {  // (64-bit stores, as everywhere)
+            *reinterpret_cast<float2*>(d) = make_float2(X.v[0], X.v[1]);
+            asm volatile("" ::: "memory");
+            *reinterpret_cast<float2*>(d + 2) = make_float2(S.a[t].v[0], S.a[t].v[1]);
+          } else {
+            *reinterpret_cast<float2*>(d) = make_float2(X.v[0], S.a[t].v[0]);
+          }
+        }
+      }
+    };
+    // Segment q (q % F = k), then the checkpoint of segment q + 3 and theta of q + F.
+    auto run = [&](int q, auto k, bool low) {
+      constexpr int kk = decltype(k)::value;
+      messages(q, T[kk], kk % 3, low);
+      load_m(q + 3, T[(kk + 3) % F]);
+      load_t(q + F, T[kk]);
+    };
+    unroll_steps<3>([&](auto k) { load_m(decltype(k)::value, T[decltype(k)::value]); });
+    run(0, std::integral_constant<int, 0>{}, true);
+    if (M > 1) run(1, std::integral_constant<int, 1>{}, false);
+    lds_barrier();  // 0
+    // Segment q before barrier q - 1.
+    for (int q0 = 0; q0 < M; q0 += F)
+      unroll_steps<F>([&](auto k) {
+        constexpr int kk = decltype(k)::value;
+        const int q = q0 + kk;
+        if ((kk >= 2 || q0 > 0) && q < M) {
+          run(q, k, false);
+          lds_barrier();  // q - 1
+        }
+      });
+    lds_barrier();  // M - 1 (M > 1), else M
+    if (M > 1) lds_barrier();  // M
+    if constexpr (NANCHK) {
+      const bool any = __ballot(nan1) != 0;  // all lanes take part
+      if (lane == 0) a.nan_flags[c] = any ? 1 : 0;
+    }
+    return;
+  }
+
+  // ---- chain wave, backward pass: step s handles i = n-2-s
+  Vec<LPL> bh;
+#pragma unroll
+  for (int k = 0; k < LPL; ++k) bh.v[k] = 0.f;
+  st_buf<LPL, FIT>(rM, (n - 1) * D * 4, lane, D, bh);  // Bh_{n-1} = 0, the last segment's checkpoint
+  auto wlane_b = [&](int s0) { return w_lds[max(n - 2 - (s0 + lane), 0)]; };
+  auto wlane_b2 = [&](int s0) { return PE ? w2_lds[max(n - 2 - (s0 + lane), 0)] : 0.f; };
+  // Returns the minimum; refill() re-issues the ring slot th came from.
+  auto step_b = [&](const Vec<LPL>& th, float wi, float wi2, auto&& refill) {
+    Vec<LPL> U, nr;
+    const float lm = near_block<LPL, DC, PE, 1>(U, th, bh, wi, L1v, 2, cc, nr);
+    __builtin_amdgcn_sched_barrier(kSchedValu);
+    refill();
+    const float u = near_min_rest<LPL, DC>(lm);
+    const Vec<LPL> m = minconv<LPL, PE>(U, nr, u, wi, wi2, L2v);
+#pragma unroll
+    for (int k = 0; k < LPL; ++k) bh.v[k] = m.v[k] - u;
+    return u;
+  };
+  // Puts a uniform value into the lanes 4 slot .. 4 slot + 3 of col.
+  auto collect = [&](float& col, float x, auto slot) {
+    constexpr int S = decltype(slot)::value;
+    col = dpp_f<0xe4, 1 << (S >> 2), 1 << (S & 3), false>(col, x);
+  };
+  Vec<LPL> ra[P];
+  if (nb > 0) {
+#pragma unroll
+    for (int j = 0; j < P; ++j) ra[j] = ld_theta(j < nb ? n - 1 - j : 1);
+  }
+  int s0 = 0;
+  float wv = wlane_b(0), wv2 = wlane_b2(0);
+  for (; s0 + P <= nb; s0 += P) {
+    const float wnext = wlane_b(s0 + P), wnext2 = wlane_b2(s0 + P);
+    const int bo = (s0 + P + lane < nb ? n - 1 - (s0 + P + lane) : 1) * strideB;  // refill offsets, one per lane
+    float uc = 0.f;
+    unroll_steps<P>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const float u = step_b(ra[j], lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, [&]() {
+        ra[j] = ld_buf<LPL, FIT>(rT, __builtin_amdgcn_readlane(bo, j), lane, D, kInfF);
+      });
+      collect(uc, u, std::integral_constant<int, j % 16>{});
+      if constexpr (j % 16 == 15) u_lds[n - 2 - (s0 + j - 15 + (lane >> 2))] = uc;
+      if constexpr ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (n - 2 - (s0 + j)) * D * 4, lane, D, bh);
+    });
+    wv = wnext;
+    wv2 = wnext2;
+  }
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+    if (s0 + j < nb) {
+      u_lds[n - 2 - (s0 + j)] = step_b(ra[j], lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, []() {});
+      if ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (n - 2 - (s0 + j)) * D * 4, lane, D, bh);
+    }
+  const double bsum = chain_offsets(u_lds, b_lds, n, lane);
+  const Vec<LPL> a0 = ld_theta(0);
+  const Vec<LPL> c_end = ld_buf<LPL, FIT>(rC, (n - 1) * strideB, lane, D, kInfF);
+  __syncthreads();
+  Vec<LPL> M0;
+#pragma unroll
+  for (int k = 0; k < LPL; ++k) M0.v[k] = a0.v[k] + bh.v[k];
+  const double Lambda = bsum + (double)chain_min(local_min(M0));
+
+  // ---- chain wave, forward pass
+  Vec<LPL> R = a0, t_cur = a0;  // theta of the current node
+  struct Pair {
+    Vec<LPL> b, t;
+  };
+  auto rd = [&](int slot) {  // node slot 0 .. 3K-1 of the message ring
+    const float* p = msg_ring + slot * 2 * NS + lane * 2 * LPL;
+    Pair r;
+    if constexpr (LPL == 2) {
+      const float4 x = *reinterpret_cast<const float4*>(p);
+      r.b.v[0] = x.x; r.b.v[1] = x.y; r.t.v[0] = x.z; r.t.v[1] = x.w;
+    } else {
+      const float2 x = *reinterpret_cast<const float2*>(p);
+      r.b.v[0] = x.x; r.t.v[0] = x.y;
+    }
+    return r;
+  };
+  auto wl = [&](int q) { return w_lds[max(min(q * K - g + lane, n - 2), 0)]; };
+  auto wl2 = [&](int q) { return PE ? w2_lds[max(min(q * K - g + lane, n - 2), 0)] : 0.f; };
+  if (M > 0) {
+    Pair pr[3];
+    lds_barrier();  // 0: segments 0 and 1 are in the ring
+    pr[0] = rd(0);
+    pr[1] = rd(1);
+    float wf = wl(0), wf2 = wl2(0);
+    // Segment q in ring slots q % 3 (messages) and q % 2 (results); low: it may
+    // start with virtual steps.
+    auto segment = [&](int q, auto slotc, auto outc, bool low) {
+      constexpr int slot = decltype(slotc)::value, oslot = decltype(outc)::value;
+      const float wn = wl(q + 1), wn2 = wl2(q + 1);
+      float vc = 0.f;
+      unroll_steps<K>([&](auto tc) {
+        constexpr int t = decltype(tc)::value, j = slot * K + t;
+        const Pair x = pr[j % 3];
+        auto next = [&]() { pr[(j + 2) % 3] = rd((j + 2) % (3 * K)); };
+        if (!low || q * K + t >= g) {
+          const float wi = lane_weight(wf, t), wi2 = PE ? lane_weight(wf2, t) : 0.f;
+          Vec<LPL> V, nr;
+          float lm;
+          if constexpr (FIT == kFitFull) {
+            lm = near_block<LPL, DC, PE, 2>(V, R, x.b, wi, L1v, 2, cc, nr);
+          } else {
+#pragma unroll
+            for (int k = 0; k < LPL; ++k) V.v[k] = valid ? fmaf(-kGamma, R.v[k] + x.b.v[k], R.v[k]) : kInfF;
+            lm = near_block<LPL, DC, PE, 0>(V, V, V, wi, L1v, 2, cc, nr);
+          }
+          __builtin_amdgcn_sched_barrier(kSchedValu);
+          next();
+          const float v = near_min_rest<LPL, DC>(lm);
+          collect(vc, v, tc);
+          const Vec<LPL> m = minconv<LPL, PE>(V, nr, v, wi, wi2, L2v);
+          Vec<LPL> mm, nx, am, o;
+#pragma unroll
+          for (int k = 0; k < LPL; ++k) mm.v[k] = FIT == kFitFull || valid ? m.v[k] : -kInfF;
+          near_max_minus<LPL, DC, PE>(mm, m, x.t, wi, L1v, 2, cc, nx, am);
+#pragma unroll
+          for (int k = 0; k < LPL; ++k) {
+            const float gk = R.v[k] - fmaxf(m.v[k], nx.v[k]);
+            o.v[k] = COLS ? gk : t_cur.v[k] - gk;
+            R.v[k] = am.v[k] - v;
+          }
+          st_ring<LPL>(out_ring + (oslot * K + t) * NS, lane, o);
+          t_cur = x.t;
+        } else {
+          next();
+        }
+      });
+      // lanes 4 t .. 4 t + 3 hold step t's minimum
+      const int i = q * K - g + (lane >> 2);
+      if (lane < 4 * K && i >= 0) v_lds[i] = vc;
+      wf = wn;
+      wf2 = wn2;
+      lds_barrier();  // q + 1
+    };
+    // six segments bring both rings back to their first slots
+    constexpr std::integral_constant<int, 0> s0c;
+    constexpr std::integral_constant<int, 1> s1c;
+    constexpr std::integral_constant<int, 2> s2c;
+    segment(0, s0c, s0c, true);
+    for (int q = 1;; q += 6) {
+      if (q >= M) break;
+      segment(q, s1c, s1c, false);
+      if (q + 1 >= M) break;
+      segment(q + 1, s2c, s0c, false);
+      if (q + 2 >= M) break;
+      segment(q + 2, s0c, s1c, false);
+      if (q + 3 >= M) break;
+      segment(q + 3, s1c, s0c, false);
+      if (q + 4 >= M) break;
+      segment(q + 4, s2c, s1c, false);
+      if (q + 5 >= M) break;
+      segment(q + 5, s0c, s0c, false);
+    }
+  }
+  Vec<LPL> out;
+#pragma unroll
+  for (int k = 0; k < LPL; ++k)
+    out.v[k] = COLS ? (c_end.v[k] - t_cur.v[k]) + R.v[k] : c_end.v[k] - (t_cur.v[k] - R.v[k]);
+  st_buf<LPL, FIT>(rW, (n - 1) * strideB, lane, D, out);
+  const double kept = chain_kept(v_lds, b_lds, n, lane, kGammaD);
+  if (lane == 0) {
+    a.lam[c] = Lambda;
+    a.kept[c] = kept;
   }
 }
 
@@ -1526,9 +1952,9 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
   }
 }
 
-template <int LPL, int MODE, int P, int FIT, int DC, bool SEG, bool NANCHK, bool PE>
+template <int LPL, int MODE, int P, int FIT, int DC, int SEG, bool NANCHK, bool PE>
 static void launch_sweep(ChainArgs& a, size_t lds, hipStream_t st) {
-  constexpr bool kRowSeg = MODE != kColsMinorant && SEG;
+  constexpr bool kRowSeg = MODE != kColsMinorant && SEG != 0;
   int cpw = 1;
   if constexpr (kRowSeg) {
     lds = row_seg_lds(LPL, PE, a.n);
@@ -1540,6 +1966,34 @@ static void launch_sweep(ChainArgs& a, size_t lds, hipStream_t st) {
     (void)hipFuncSetAttribute((const void*)k_chain<LPL, MODE, P, FIT, DC, SEG, NANCHK, PE>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   k_chain<LPL, MODE, P, FIT, DC, SEG, NANCHK, PE><<<(a.n_chains + cpw - 1) / cpw, kRowSeg ? 128 * cpw : 64, lds, st>>>(a);
+}
+
+template <int LPL, int FIT, bool PE, bool COLS, bool NANCHK>
+static void launch_line(ChainArgs& a, hipStream_t st) {
+  size_t lds = line_lds(LPL, PE, a.n);
+  const bool two = a.n_chains > cu_count() && 2 * lds <= kLdsPerCu;
+  if (two) lds *= 2;
+  if (lds > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)k_line<LPL, FIT, PE, COLS, NANCHK>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  k_line<LPL, FIT, PE, COLS, NANCHK><<<two ? (a.n_chains + 1) / 2 : a.n_chains, two ? 512 : 192, lds, st>>>(a);
+}
+
+// Whether a sweep runs on k_line: where its time is the steps of one resident
+// set of chains.  With more chains than LINE_ROUNDS per CU the sweep is bound by
+// what it moves, and the three waves of a chain only take the CUs' wave slots
+// from other chains.  Measured, k_line against k_chain (us):
+//   rows, D = 64:  320 x 240 53 / 62, 640 x 480 102 / 119, 1000 x 1000 232 / 217
+//   rows, D = 128: 320 x 240 63 / 72, 744 x 496 166 / 169, 1000 x 1000 458 / 414
+//   columns, D = 64:  320 x 240 43 / 63, 1000 x 1000 238 / 281, 1242 x 375 141 / 129
+//   columns, D = 128: 320 x 240 50 / 66, 512 x 256 62 / 74, 640 x 480 206 / 154
+template <int LPL, int MODE>
+static bool use_line(const ChainArgs& a) {
+  constexpr int kRounds = MODE == kColsMinorant && LPL == 1 ? 4 : 2;
+  const long extent = ((long)(a.n - 1) * a.pns * a.D + a.D) * (long)sizeof(float);  // 32-bit byte offsets
+  const long msg = (long)a.n * a.D * (long)sizeof(float);
+  return a.n_chains <= kRounds * cu_count() && line_lds(LPL, a.w2 != nullptr, a.n) <= kLdsPerCu &&
+         extent <= 0x7fffffffL && msg <= 0x7fffffffL;
 }
 
 // Register-ring depth of the row sweeps with a message wave: three segments.
@@ -1565,20 +2019,26 @@ static void launch_one(ChainArgs& a, size_t lds, bool seg, hipStream_t st) {
       k_decode4<LPL, PD, FIT, DC, true, PE><<<a.n_chains, 256, lds2, st>>>(a);
     else
       k_decode4<LPL, PD, FIT, DC, false, PE><<<a.n_chains, 256, lds2, st>>>(a);
-  } else if constexpr (MODE == kColsMinorant) {
-    if (seg)
-      launch_sweep<LPL, MODE, P, FIT, DC, true, false, PE>(a, lds, st);
-    else
-      launch_sweep<LPL, MODE, P, FIT, DC, false, false, PE>(a, lds, st);
-  } else if (seg) {
-    if (a.nan_flags)
-      launch_sweep<LPL, MODE, row_seg_p<LPL>(), FIT, DC, true, true, PE>(a, lds, st);
-    else
-      launch_sweep<LPL, MODE, row_seg_p<LPL>(), FIT, DC, true, false, PE>(a, lds, st);
-  } else if (a.nan_flags) {
-    launch_sweep<LPL, MODE, P, FIT, DC, false, true, PE>(a, lds, st);
   } else {
-    launch_sweep<LPL, MODE, P, FIT, DC, false, false, PE>(a, lds, st);
+    constexpr bool kCols = MODE == kColsMinorant;
+    constexpr int PS = kCols ? P : row_seg_p<LPL>();  // ring depth of the checkpointed sweep
+    if constexpr (DC == 2 && LPL <= 2) {
+      if (use_line<LPL, MODE>(a)) {
+        if constexpr (!kCols)
+          if (a.nan_flags) return launch_line<LPL, FIT, PE, false, true>(a, st);
+        return launch_line<LPL, FIT, PE, kCols, false>(a, st);
+      }
+    }
+    auto sweep = [&](auto nan) {
+      constexpr bool NAN_ = decltype(nan)::value;
+      if (!seg) return launch_sweep<LPL, MODE, P, FIT, DC, 0, NAN_, PE>(a, lds, st);
+      if constexpr (DC == 2)
+        if (a.stream) return launch_sweep<LPL, MODE, PS, FIT, DC, 2, NAN_, PE>(a, lds, st);
+      launch_sweep<LPL, MODE, PS, FIT, DC, 1, NAN_, PE>(a, lds, st);
+    };
+    if constexpr (!kCols)
+      if (a.nan_flags) return sweep(std::true_type{});
+    sweep(std::false_type{});
   }
 }
 
@@ -1615,19 +2075,14 @@ static void launch_lpl(ChainArgs& a, size_t lds, bool seg, hipStream_t st) {
 #define CCS_CRF_P_COLS 16
 #endif
 
-// One sweep of `mode` over all chains for LPL labels per lane.  Defined for
-// LPL = 1, 2 and 4 (up to 64, 128 and 256 labels), each in a translation unit
-// of its own (crf_sweeps_*.hip).
-template <int LPL>
-int launch_labels(ChainMode mode, ChainArgs& a, bool seg, hipStream_t st) {
+// One sweep over all chains for LPL labels per lane.  Defined for LPL = 1, 2
+// and 4 (up to 64, 128 and 256 labels), the row sweeps and the others each in a
+// translation unit of their own (crf_sweeps_*.hip).
+template <int LPL, int MODE>
+int launch_labels(ChainArgs& a, bool seg, hipStream_t st) {
   const size_t lds = (sizeof(double) + (a.w2 ? 3 : 2) * sizeof(float)) * (size_t)a.n;
-  constexpr int PR = LPL < 4 ? CCS_CRF_P_ROWS : CCS_CRF_P_ROWS / 2, PC = LPL < 4 ? CCS_CRF_P_COLS : CCS_CRF_P_COLS / 2;
-  switch (mode) {
-    case kRowsMinorant: launch_lpl<kRowsMinorant, LPL, PR>(a, lds, seg, st); break;
-    case kColsMinorant: launch_lpl<kColsMinorant, LPL, PC>(a, lds, seg, st); break;
-    case kRowsDecode: launch_lpl<kRowsDecode, LPL, PR>(a, lds, seg, st); break;
-    default: return fail(CCS_ERR_ARG, "unknown chain mode %d", (int)mode);
-  }
+  constexpr int P = MODE == kColsMinorant ? CCS_CRF_P_COLS : CCS_CRF_P_ROWS;
+  launch_lpl<MODE, LPL, LPL < 4 ? P : P / 2>(a, lds, seg, st);
   CCS_LAUNCH_CHECK();
   return CCS_OK;
 }

@@ -1,6 +1,7 @@
-// The chain sweeps of up to 64 labels (1 per lane).
+// The column sweeps and the decode of up to 64 labels (1 per lane).
 #include "crf_sweeps.hpp"
 
 namespace ccs {
-template int launch_labels<1>(ChainMode mode, ChainArgs& a, bool seg, hipStream_t st);
+template int launch_labels<1, kColsMinorant>(ChainArgs& a, bool seg, hipStream_t st);
+template int launch_labels<1, kRowsDecode>(ChainArgs& a, bool seg, hipStream_t st);
 }  // namespace ccs

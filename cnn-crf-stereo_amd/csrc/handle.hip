@@ -127,7 +127,7 @@ extern "C" int ccs_reserve(ccs_handle_t h, int H, int W, int D, int C, int iters
   if ((rc = h->misc2.reserve(misc2, h->stream))) return rc;
   if ((rc = h->crf_a.reserve(vol * sizeof(float), h->stream))) return rc;
   if ((rc = h->crf_msg.reserve(vol * sizeof(float), h->stream))) return rc;
-  if ((rc = h->crf_small.reserve(sizeof(double) * ccs::run_chain_doubles((int)big, iters), h->stream))) return rc;
+  if ((rc = h->crf_small.reserve(sizeof(double) * ccs::run_chain_doubles((int)big), h->stream))) return rc;
   if ((rc = h->crf_nan.reserve(sizeof(int) * (size_t)H, h->stream))) return rc;
   if ((rc = h->crf_sums.reserve(sizeof(double) * (4 * (size_t)iters + 2), h->stream))) return rc;
   return CCS_OK;
