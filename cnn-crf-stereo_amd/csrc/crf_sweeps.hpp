@@ -84,8 +84,10 @@ struct Vec {
 // kFitLanes: D is a multiple of LPL, so a lane's labels all exist or none does:
 // a node is one vector access per lane, as with kFitFull, and the lanes without
 // labels only need +inf unaries (their messages are never stored and never
-// reach a label).  kFitAny: element-wise accesses and a mask per label.
-enum { kFitAny = 0, kFitLanes = 1, kFitFull = 2 };
+// reach a label).  kFitHalf: kFitLanes with labels in two of the wave's four rows
+// only, whose minimum over the labels is five instructions shorter.  kFitAny:
+// element-wise accesses and a mask per label.
+enum { kFitAny = 0, kFitLanes = 1, kFitFull = 2, kFitHalf = 3 };
 
 // Row sweeps with a message wave (SEG rows): the backward pass keeps every
 // seg_len()-th message in the scratch volume, and a second wave of the
@@ -245,18 +247,22 @@ __device__ __forceinline__ void unroll_steps(F&& f) {
 // inside each row of 16 lanes (two wait states before each), then the four rows'
 // minima through v_readlane: 9 instructions against 10 with v_permlane16_swap
 // and v_permlane32_swap, whose copies and wait states cannot be filled.
+// ROWS = 2: the other two rows hold +inf (32 labels, kFitHalf: 4 instructions).
+template <int ROWS = 4>
 __device__ __forceinline__ float rows_min(float x) {
   auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); };
+  if constexpr (ROWS == 2) return fminf(fminf(x, row(0)), row(16));
   const float s0 = row(0), s1 = row(16), s2 = row(32), s3 = row(48);
   // (one scalar operand per instruction, so no value has to be moved first)
   return fminf(fminf(fminf(s0, x), fminf(s1, x)), fminf(fminf(s2, x), fminf(s3, x)));
 }
+template <int ROWS = 4>
 __device__ __forceinline__ float chain_min(float x) {
   x = fminf(x, dpp_rot<0xb1>(x));
   x = fminf(x, dpp_rot<0x4e>(x));
   x = fminf(x, dpp_rot<0x124>(x));
   x = fminf(x, dpp_rot<0x128>(x));
-  return rows_min(x);
+  return rows_min<ROWS>(x);
 }
 
 // A kernel-uniform value kept in a VGPR.  The steps multiply the edge weight
@@ -402,12 +408,12 @@ __device__ __forceinline__ float near_block(Vec<LPL>& U, const Vec<LPL>& x, cons
 }
 
 // The rest of the minimum's tree, from near_block's partial minimum.
-template <int LPL, int DC>
+template <int LPL, int DC, int ROWS = 4>
 __device__ __forceinline__ float near_min_rest(float lm) {
-  if constexpr (!(LPL == 2 && DC == 2)) return chain_min(lm);
+  if constexpr (!(LPL == 2 && DC == 2)) return chain_min<ROWS>(lm);
   lm = fminf(lm, dpp_rot<0x124>(lm));
   lm = fminf(lm, dpp_rot<0x128>(lm));
-  return rows_min(lm);
+  return rows_min<ROWS>(lm);
 }
 
 // U = x + y and its neighbour terms alone (the recomputed messages, whose
@@ -500,13 +506,24 @@ __device__ __forceinline__ Vec<LPL> minconv(const Vec<LPL>& U, const Vec<LPL>& n
 // Node loads never sit under divergent control flow (that would make the
 // compiler drain every outstanding load at the join): with kFitFull every lane
 // owns LPL labels and loads them as one vector, with kFitLanes the lanes without
-// labels load the last lane's again and replace them by the fill; with kFitAny
-// the lane loads clamped addresses element by element and masks the labels >= D.
+// labels load the last lane's again; with kFitAny the lane loads clamped
+// addresses element by element.  What the places without a label load is replaced
+// where it is used (masked()), never beside the load: a select there is scheduled
+// with the load and waits for it, which empties the register rings (320 x 240 x 32
+// rows 58 us, x 64 52 us; a streamed wave waits once per segment).
 template <int LPL, int FIT>
-__device__ __forceinline__ Vec<LPL> ld_node(const float* __restrict__ base, int lane, int D, float fill) {
+__device__ __forceinline__ Vec<LPL> masked(const Vec<LPL>& x, int lane, int D, float fill) {
+  Vec<LPL> o;
+#pragma unroll
+  for (int j = 0; j < LPL; ++j)
+    o.v[j] = FIT == kFitFull || lane * LPL + (FIT == kFitAny ? j : 0) < D ? x.v[j] : fill;
+  return o;
+}
+
+template <int LPL, int FIT>
+__device__ __forceinline__ Vec<LPL> ld_node(const float* __restrict__ base, int lane, int D) {
   Vec<LPL> out;
   if constexpr (FIT != kFitAny) {
-    const bool ok = FIT == kFitFull || lane * LPL < D;
     const int l = FIT == kFitFull ? lane * LPL : min(lane * LPL, D - LPL);
     if constexpr (LPL == 4) {
       const float4 t = *reinterpret_cast<const float4*>(base + l);
@@ -517,14 +534,11 @@ __device__ __forceinline__ Vec<LPL> ld_node(const float* __restrict__ base, int 
     } else {
       out.v[0] = base[l];
     }
-#pragma unroll
-    for (int j = 0; j < LPL; ++j) out.v[j] = ok ? out.v[j] : fill;
   } else {
 #pragma unroll
     for (int j = 0; j < LPL; ++j) {
       const int s = lane * LPL + j;
-      const float v = base[s < D ? s : D - 1];
-      out.v[j] = s < D ? v : fill;
+      out.v[j] = base[s < D ? s : D - 1];
     }
   }
   return out;
@@ -533,7 +547,7 @@ __device__ __forceinline__ Vec<LPL> ld_node(const float* __restrict__ base, int 
 template <int LPL, int FIT>
 __device__ __forceinline__ void st_node(float* __restrict__ base, int lane, int D, const Vec<LPL>& x) {
   if constexpr (FIT != kFitAny) {
-    if (FIT == kFitLanes && lane * LPL >= D) return;
+    if (FIT != kFitFull && lane * LPL >= D) return;
     if constexpr (LPL == 4) {  // two 64-bit stores (see kNoWideStores)
       *reinterpret_cast<float2*>(base + lane * 4) = make_float2(x.v[0], x.v[1]);
       asm volatile("" ::: "memory");
@@ -566,10 +580,9 @@ __device__ __forceinline__ Rsrc chain_rsrc(const float* base, long nfloats) {
 // cached part to the unaries, which every sweep reads twice).
 constexpr int kStream = 2;  // non-temporal
 template <int LPL, int FIT, int AUX = 0>
-__device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D, float fill) {
+__device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D) {
   Vec<LPL> out;
   if constexpr (FIT != kFitAny) {
-    const bool ok = FIT == kFitFull || lane * LPL < D;
     const int voff = (FIT == kFitFull ? lane * LPL : min(lane * LPL, D - LPL)) * 4;
     if constexpr (LPL == 4) {
       const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, AUX);
@@ -582,14 +595,11 @@ __device__ __forceinline__ Vec<LPL> ld_buf(Rsrc r, int soff, int lane, int D, fl
     } else {
       out.v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, AUX));
     }
-#pragma unroll
-    for (int j = 0; j < LPL; ++j) out.v[j] = ok ? out.v[j] : fill;
   } else {
 #pragma unroll
     for (int j = 0; j < LPL; ++j) {
       const int s = lane * LPL + j;
-      const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (s < D ? s : D - 1) * 4, soff, AUX));
-      out.v[j] = s < D ? v : fill;
+      out.v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (s < D ? s : D - 1) * 4, soff, AUX));
     }
   }
   return out;
@@ -741,12 +751,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
   auto keep = [&](int j) { return FIT != kFitAny || valid[j]; };
 
   // The chain unaries: what the sweep reads (A for rows, B for columns).
-  auto theta_of = [&](const Vec<LPL>& av) {
-    Vec<LPL> th;
-#pragma unroll
-    for (int j = 0; j < LPL; ++j) th.v[j] = keep(j) ? av.v[j] : kInfF;
-    return th;
-  };
+  auto theta_of = [&](const Vec<LPL>& av) { return masked<LPL, FIT>(av, lane, D, kInfF); };
   // Columns: the row unaries C - B of a node.
   auto row_unaries = [&](const Vec<LPL>& bv, const Vec<LPL>& cv) {
     Vec<LPL> r;
@@ -823,7 +828,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
       const int M = (nb + K - 1) / K;
       // NANCHK: this wave tests node 0 and every unary its segments consume
       // (nodes 1 .. n-1) and sets the chain's flag, off the forward wave.
-      bool nan1 = NANCHK && any_nan(ld_buf<LPL, FIT>(rA, 0, lane, D, kInfF));
+      bool nan1 = NANCHK && any_nan(ld_buf<LPL, FIT>(rA, 0, lane, D));
       auto put_flag = [&]() {
         if constexpr (NANCHK) {
           const bool any = __ballot(nan1) != 0;  // all lanes take part
@@ -844,8 +849,8 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
         const int ib = s * K - g;            // node of t = 0 (negative only in segment 0)
 #pragma unroll
         for (int t = 0; t < K; ++t)
-          B.a[t] = ld_buf<LPL, FIT>(rA, min(max(ib + t + 1, 1), n - 1) * strideB, lane, D, kInfF);
-        B.m = ld_buf<LPL, FIT>(rM, (ib + K) * D * 4, lane, D, 0.f);
+          B.a[t] = ld_buf<LPL, FIT>(rA, min(max(ib + t + 1, 1), n - 1) * strideB, lane, D);
+        B.m = ld_buf<LPL, FIT>(rM, (ib + K) * D * 4, lane, D);
         const int e = max(min(ib + lane, n - 2), 0);
         B.u = u_lds[e];
         B.w = w_lds[e];
@@ -894,9 +899,9 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
   auto load_b = [&](int s, Vec<LPL>& av) {
     const int node = s < nb ? n - 1 - s : 1;  // clamped: beyond the chain re-read node 1
     if constexpr (kCols)
-      av = ld_node<LPL, FIT>(Ab + node * nstride, lane, D, kInfF);
+      av = ld_node<LPL, FIT>(Ab + node * nstride, lane, D);
     else
-      av = ld_buf<LPL, FIT>(rA, node * strideB, lane, D, kInfF);
+      av = ld_buf<LPL, FIT>(rA, node * strideB, lane, D);
   };
   // weights of steps s0 .. s0+63 of the backward pass (edge n-2-s)
   auto wlane_b = [&](int s0) { return w_lds[max(n - 2 - (s0 + lane), 0)]; };
@@ -944,7 +949,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
       // refill reuses the slot's registers.
       step_b(s0 + j, theta_of(ra[j]), lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, (j + 1) % KR == 0, [&]() {
         if constexpr (kRowSeg)
-          ra[j] = ld_buf<LPL, FIT>(rA, __builtin_amdgcn_readlane(bo, j), lane, D, kInfF);
+          ra[j] = ld_buf<LPL, FIT>(rA, __builtin_amdgcn_readlane(bo, j), lane, D);
         else
           load_b(s0 + j + P, ra[j]);
       });
@@ -961,13 +966,13 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
   bsum = chain_offsets(u_lds, b_lds, n, lane);  // b_0 = sum of all minima
 
   // bh holds Bh[0]; theta[0] is read directly.
-  a0 = ld_node<LPL, FIT>(Ab, lane, D, kInfF);
+  a0 = ld_node<LPL, FIT>(Ab, lane, D);
   if constexpr (NANCHK && !kRowSeg) {  // (kRowSeg: the message wave tests the unaries)
     nan_seen |= any_nan(a0);
     const bool any = __ballot(nan_seen) != 0;  // all lanes take part
     if (lane == 0) a.nan_flags[c] = any ? 1 : 0;
   }
-  if constexpr (MODE != kRowsDecode) c0 = ld_node<LPL, FIT>(Cb, lane, D, kInfF);
+  if constexpr (MODE != kRowsDecode) c0 = ld_node<LPL, FIT>(Cb, lane, D);
   th0 = theta_of(a0);
   }
   __syncthreads();  // kRowSeg: the checkpoints and u_lds are now visible to wave 1
@@ -991,13 +996,13 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
     auto load_f = [&](int i, Vec<LPL>& bv, Vec<LPL>& av, Vec<LPL>& cv) {
       const int node = i < nb ? i : nb - 1;
       if constexpr (kCols) {
-        bv = ld_node<LPL, FIT>(msg + (long)node * D, lane, D, 0.f);
-        av = ld_node<LPL, FIT>(Ab + (node + 1) * nstride, lane, D, kInfF);
-        cv = ld_node<LPL, FIT>(Cb + (node + 1) * nstride, lane, D, kInfF);
+        bv = ld_node<LPL, FIT>(msg + (long)node * D, lane, D);
+        av = ld_node<LPL, FIT>(Ab + (node + 1) * nstride, lane, D);
+        cv = ld_node<LPL, FIT>(Cb + (node + 1) * nstride, lane, D);
       } else {
-        bv = ld_buf<LPL, FIT>(rM, node * D * 4, lane, D, 0.f);
-        av = ld_buf<LPL, FIT>(rA, (node + 1) * strideB, lane, D, kInfF);
-        cv = ld_buf<LPL, FIT>(rC, node * strideB, lane, D, kInfF);
+        bv = ld_buf<LPL, FIT>(rM, node * D * 4, lane, D);
+        av = ld_buf<LPL, FIT>(rA, (node + 1) * strideB, lane, D);
+        cv = ld_buf<LPL, FIT>(rC, node * strideB, lane, D);
       }
     };
     // weights of steps i0 .. i0+63 of the forward pass (edge i)
@@ -1007,7 +1012,7 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
     Vec<LPL> a_cur = kCols ? row_unaries(a0, c0) : a0;  // A_0
     // Rows: the costs of the last node, for its stored C - A'.
     Vec<LPL> c_last;
-    if constexpr (!kCols) c_last = ld_buf<LPL, FIT>(rC, (n - 1) * strideB, lane, D, kInfF);
+    if constexpr (!kCols) c_last = ld_buf<LPL, FIT>(rC, (n - 1) * strideB, lane, D);
     // The float64 kept constant (the chain minimum this pass leaves behind) is
     // formed from the per-node minima v_i after the pass: chain_kept().
     // step_f takes Bh_i, A_{i+1} and theta_{i+1} (the read unaries) and returns
@@ -1082,8 +1087,8 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
         // step's own unaries), its C that of step P-1
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-          ra[j] = ld_buf<LPL, FIT>(rA, node_a(j < P - 1 ? j : -1) * strideB, lane, D, kInfF);
-          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, node_c(j) * strideB, lane, D, kInfF);
+          ra[j] = ld_buf<LPL, FIT>(rA, node_a(j < P - 1 ? j : -1) * strideB, lane, D);
+          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, node_c(j) * strideB, lane, D);
         }
         lds_barrier();  // segments 0 and 1 are in the ring
         bm[0] = ld_ring<LPL>(ring, lane);
@@ -1114,9 +1119,9 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
         if (!TAIL) {
           // C_i and A_i are read: their slots take C of step ip + P and A of
           // step ip - 1 + P.
-          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, __builtin_amdgcn_readlane(ao, j) - strideB, lane, D, kInfF);
+          rc[j] = ld_buf<LPL, FIT, kCostAux>(rC, __builtin_amdgcn_readlane(ao, j) - strideB, lane, D);
           ra[jp] = ld_buf<LPL, FIT>(rA, j > 0 ? __builtin_amdgcn_readlane(ao, j - 1) : __builtin_amdgcn_readlane(aop, P - 1),
-                                     lane, D, kInfF);
+                                     lane, D);
         }
       };
       int i0p = 0;
@@ -1172,10 +1177,10 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 #pragma unroll
         for (int t = 0; t < K; ++t) {
           const int off = min(t, n - 1 - first) * strideB;
-          B.a[t] = ld_buf<LPL, FIT>(sA, off, lane, D, kInfF);
-          B.c[t] = ld_buf<LPL, FIT, kCostAux>(sC, off, lane, D, kInfF);
+          B.a[t] = ld_buf<LPL, FIT>(sA, off, lane, D);
+          B.c[t] = ld_buf<LPL, FIT, kCostAux>(sC, off, lane, D);
         }
-        B.m = ld_node<LPL, FIT>(msg + (long)min(i0 + K, nb) * D, lane, D, 0.f);
+        B.m = ld_node<LPL, FIT>(msg + (long)min(i0 + K, nb) * D, lane, D);
         const int e = max(min(i0 + lane, n - 2), 0);
         B.u = u_lds[e];
         B.w = w_lds[e];
@@ -1297,7 +1302,9 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 //   Backward pass (chain wave): theta through a register ring, every K-th
 //     message stored as a checkpoint (end-aligned, at nodes n-1 - m K).  The
 //     per-node minimum is kept in a register: one DPP move writes it to the
-//     step's quad of lanes, and 16 steps' values go to LDS at once.
+//     step's quad of lanes, and 16 steps' values go to LDS at once.  The messages
+//     of the first three segments, the pass's last, go straight to the ring, so
+//     that the forward pass starts without waiting for a recomputation.
 //   Forward pass, in segments of K steps (forward step i' = i + g of node i, g
 //     virtual steps align the segments with the checkpoints).  Between barriers
 //     q and q + 1
@@ -1306,10 +1313,10 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 //         result (rows: A'_i = A_i - g_i; columns: g_i) to a ring of two;
 //       the output wave stores segment q - 1 (rows: C_i - A'_i; columns:
 //         (C_i - B_i) + g_i);
-//       the message wave recomputes the messages of segment q + 2 from the
-//         checkpoint at its end into the slot that segment q - 1 has left, with
-//         the backward step's own operations and operands, so they are the
-//         messages it formed, bit for bit.
+//       the message wave (first: the float64 offsets b_i) recomputes the messages
+//         of segment q + 2 from the checkpoint at its end into the slot that
+//         segment q - 1 has left, with the backward step's own operations and
+//         operands, so they are the messages it formed, bit for bit.
 //
 // Loads run 4 (costs) and 6 segments (theta) ahead: 1242 x 256 chains of 128
 // labels 242 -> 237 us against 2 and 3.  Up to two chains per CU share a
@@ -1324,10 +1331,10 @@ constexpr int kLineK = 8;
 constexpr int kLineRing = 3 * 2 + 2;  // segments of node vectors in the two rings
 enum LineRole { kChain = 0, kMessages = 1, kOut = 2, kIdle = 3 };
 
-// LDS of one chain: b, w, u, v, [w2], rounded to 16 bytes, then the rings.
+// LDS of one chain: b and their sum, w, u, v, [w2], rounded to 16 bytes, then the rings.
 constexpr size_t line_lds(int lpl, bool per_edge, int n) {
   return sizeof(float) *
-         ((((per_edge ? 6 : 5) * (size_t)n + 3) & ~(size_t)3) + (size_t)kLineRing * kLineK * 64 * lpl);
+         ((((per_edge ? 6 : 5) * (size_t)n + 5) & ~(size_t)3) + (size_t)kLineRing * kLineK * 64 * lpl);
 }
 
 template <int LPL, int FIT, bool PE, bool COLS, bool NANCHK>
@@ -1341,11 +1348,11 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
   const int role = !two ? wave : wave < 4 ? wave & 1 : wave & 1 ? kOut : kIdle;
   const int c_slot = blockIdx.x * (two ? 2 : 1) + cs;
   const int c = min(c_slot, a.n_chains - 1);
-  // per chain: b (doubles), w, u, v, [w2], then the rings at a 16-byte boundary
-  const int head = ((PE ? 6 : 5) * n + 3) & ~3;
+  // per chain: b and their sum (doubles), w, u, v, [w2], then the rings at a 16-byte boundary
+  const int head = ((PE ? 6 : 5) * n + 5) & ~3;
   const int chain_floats = head + kLineRing * K * NS;
   double* b_lds = lds_line + cs * (chain_floats / 2);
-  float* w_lds = reinterpret_cast<float*>(b_lds + n);
+  float* w_lds = reinterpret_cast<float*>(b_lds + n + 1);
   float* u_lds = w_lds + n;
   float* v_lds = u_lds + n;
   float* w2_lds = v_lds + n;  // PE only
@@ -1364,22 +1371,38 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
   const float* __restrict__ wb = a.w + pbase * a.wmul;
   const float* __restrict__ wb2 = PE ? a.w2 + pbase * a.wmul : nullptr;
   const long wstep = a.pns * a.wmul;
-  if (role <= kMessages)
-    for (int i = role * 64 + lane; i < n - 1; i += 128) {
+  const int nb = n - 1, M = (nb + K - 1) / K, g = M * K - nb;
+  auto fill_weights = [&]() {  // by the message and the output wave
+    for (int i = (role - kMessages) * 64 + lane; i < nb; i += 128) {
       w_lds[i] = wb[(long)i * wstep];
       if constexpr (PE) w2_lds[i] = wb2[(long)i * wstep];
     }
-  const int nb = n - 1, M = (nb + K - 1) / K, g = M * K - nb;
-  __syncthreads();
+  };
   if (role == kIdle || c_slot >= a.n_chains) {  // the same barriers, no work
     __syncthreads();
-    if (M > 0)
-      for (int q = 0; q <= M; ++q) lds_barrier();
+    __syncthreads();
+    for (int q = 1; q <= M; ++q) lds_barrier();
     return;
   }
-  auto ld_theta = [&](int node) { return ld_buf<LPL, FIT>(rT, node * strideB, lane, D, kInfF); };
+  auto theta_of = [&](const Vec<LPL>& x) { return masked<LPL, FIT>(x, lane, D, kInfF); };
+  auto ld_theta = [&](int node) { return ld_buf<LPL, FIT>(rT, node * strideB, lane, D); };
 
   auto ib = [&](int q) { return q * K - g; };  // node of a segment's first step
+  // The two halves of a lane's vector in the message ring (64-bit stores, as everywhere).
+  auto put_msg = [&](float* d, const Vec<LPL>& x) {
+    if constexpr (LPL == 2) {
+      *reinterpret_cast<float2*>(d) = make_float2(x.v[0], x.v[1]);
+      asm volatile("" ::: "memory");
+    } else {
+      d[0] = x.v[0];
+    }
+  };
+  auto put_theta = [&](float* d, const Vec<LPL>& x) {
+    if constexpr (LPL == 2)
+      *reinterpret_cast<float2*>(d + 2) = make_float2(x.v[0], x.v[1]);
+    else
+      d[1] = x.v[0];
+  };
 
   if (role == kOut) {
     // ---- output wave: the costs run four segments ahead
@@ -1390,14 +1413,14 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
       auto off = [&](int t) { return min(max(ib(min(q, M - 1)) + t, 0), n - 1) * strideB; };
       if (a.stream) {
 #pragma unroll
-        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT, kStream>(rC, off(t), lane, D, kInfF);
+        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT, kStream>(rC, off(t), lane, D);
       } else {
 #pragma unroll
-        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT>(rC, off(t), lane, D, kInfF);
+        for (int t = 0; t < K; ++t) C[kk][t] = ld_buf<LPL, FIT>(rC, off(t), lane, D);
       }
       if constexpr (COLS) {
 #pragma unroll
-        for (int t = 0; t < K; ++t) B[kk][t] = ld_buf<LPL, FIT>(rT, off(t), lane, D, kInfF);
+        for (int t = 0; t < K; ++t) B[kk][t] = ld_buf<LPL, FIT>(rT, off(t), lane, D);
       }
     };
     // Stores segment q (q % F = k) after barrier q + 1, then loads segment q + F.
@@ -1417,10 +1440,10 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
       }
       load(q + F, k);
     };
-    __syncthreads();
-    if (M == 0) return;
     unroll_steps<F>([&](auto k) { load(decltype(k)::value, k); });
-    lds_barrier();  // 0
+    fill_weights();
+    __syncthreads();
+    __syncthreads();
     for (int q = 0; q < M; q += F)
       unroll_steps<F>([&](auto k) {
         const int qk = q + decltype(k)::value;
@@ -1444,75 +1467,59 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
       for (int t = 0; t < K; ++t) S.a[t] = ld_theta(min(max(ib(min(q, M - 1)) + t + 1, 1), n - 1));
     };
     auto load_m = [&](int q, Seg& S) {  // the checkpoint and the segment's minima and weights, one per lane
-      S.m = ld_buf<LPL, FIT>(rM, min(ib(q) + K, n - 1) * D * 4, lane, D, 0.f);
+      S.m = ld_buf<LPL, FIT>(rM, min(ib(q) + K, n - 1) * D * 4, lane, D);
       const int e = max(min(ib(q) + lane, n - 2), 0);
       S.u = u_lds[e];
       S.w = w_lds[e];
       S.w2 = PE ? w2_lds[e] : 0.f;
     };
-    bool nan1 = NANCHK && any_nan(ld_theta(0));
-    if (M > 0) {
+    fill_weights();
+    bool nan1 = false;
+    if constexpr (NANCHK) {  // the nodes that its segments do not read
 #pragma unroll
-      for (int k = 0; k < F; ++k) load_t(k, T[k]);
+      for (int i = 0; i <= 3 * K; ++i) nan1 |= any_nan(ld_theta(min(i, n - 1)));
     }
-    __syncthreads();  // the checkpoints and u_lds are visible
-    if (M == 0) {
-      if constexpr (NANCHK) {
-        const bool any = __ballot(nan1) != 0;
-        if (lane == 0) a.nan_flags[c] = any ? 1 : 0;
-      }
-      return;
-    }
-    // The messages of segment q into ring slot q % 3; low: segment 0, which may
-    // start with virtual steps.
-    auto messages = [&](int q, const Seg& S, int slot, bool low) {
+    unroll_steps<F>([&](auto k) { load_t(3 + decltype(k)::value, T[(3 + decltype(k)::value) % F]); });
+    __syncthreads();  // the weights are in LDS
+    __syncthreads();  // the checkpoints, the minima and segments 0 .. 2 are visible
+    // The messages of segment q >= 3 into ring slot q % 3.
+    auto messages = [&](int q, const Seg& S, int slot) {
       float* dst = msg_ring + slot * K * 2 * NS + lane * 2 * LPL;
       Vec<LPL> X = S.m;
 #pragma unroll
       for (int t = K - 1; t >= 0; --t) {
-        if (!low || ib(q) + t >= 0) {
-          if constexpr (NANCHK) nan1 |= any_nan(S.a[t]);
-          const float u = lane_weight(S.u, t);
-          Vec<LPL> U, nr;
-          near_only<LPL, DC, PE>(U, S.a[t], X, lane_weight(S.w, t), L1v, 2, cc, nr);
-          const Vec<LPL> m =
-              minconv<LPL, PE>(U, nr, u, lane_weight(S.w, t), PE ? lane_weight(S.w2, t) : 0.f, L2v);
+        if constexpr (NANCHK) nan1 |= any_nan(S.a[t]);
+        const Vec<LPL> th = theta_of(S.a[t]);
+        const float u = lane_weight(S.u, t);
+        Vec<LPL> U, nr;
+        near_only<LPL, DC, PE>(U, th, X, lane_weight(S.w, t), L1v, 2, cc, nr);
+        const Vec<LPL> m = minconv<LPL, PE>(U, nr, u, lane_weight(S.w, t), PE ? lane_weight(S.w2, t) : 0.f, L2v);
 #pragma unroll
-          for (int k = 0; k < LPL; ++k) X.v[k] = m.v[k] - u;
-          float* d = dst + t * 2 * NS;
-          if constexpr (LPL == 2) {  // (64-bit stores, as everywhere)
-            *reinterpret_cast<float2*>(d) = make_float2(X.v[0], X.v[1]);
-            asm volatile("" ::: "memory");
-            *reinterpret_cast<float2*>(d + 2) = make_float2(S.a[t].v[0], S.a[t].v[1]);
-          } else {
-            *reinterpret_cast<float2*>(d) = make_float2(X.v[0], S.a[t].v[0]);
-          }
-        }
+        for (int k = 0; k < LPL; ++k) X.v[k] = m.v[k] - u;
+        float* d = dst + t * 2 * NS;
+        put_msg(d, X);
+        put_theta(d, th);
       }
     };
-    // Segment q (q % F = k), then the checkpoint of segment q + 3 and theta of q + F.
-    auto run = [&](int q, auto k, bool low) {
-      constexpr int kk = decltype(k)::value;
-      messages(q, T[kk], kk % 3, low);
-      load_m(q + 3, T[(kk + 3) % F]);
-      load_t(q + F, T[kk]);
-    };
-    unroll_steps<3>([&](auto k) { load_m(decltype(k)::value, T[decltype(k)::value]); });
-    run(0, std::integral_constant<int, 0>{}, true);
-    if (M > 1) run(1, std::integral_constant<int, 1>{}, false);
-    lds_barrier();  // 0
-    // Segment q before barrier q - 1.
+    unroll_steps<3>([&](auto k) { load_m(3 + decltype(k)::value, T[3 + decltype(k)::value]); });
+    const double bsum = chain_offsets(u_lds, b_lds, n, lane);  // b_0 = sum of all minima
+    if (lane == 0) b_lds[n] = bsum;
+    // Segment q (q % F = k) between barriers q - 2 and q - 1, then the checkpoint
+    // of segment q + 3 and theta of q + F.
+    for (int q = 1; q <= min(M, 2); ++q)
+      if (q < 2 || M < 4) lds_barrier();
     for (int q0 = 0; q0 < M; q0 += F)
       unroll_steps<F>([&](auto k) {
         constexpr int kk = decltype(k)::value;
         const int q = q0 + kk;
-        if ((kk >= 2 || q0 > 0) && q < M) {
-          run(q, k, false);
+        if ((kk >= 3 || q0 > 0) && q < M) {
+          messages(q, T[kk], kk % 3);
+          load_m(q + 3, T[(kk + 3) % F]);
+          load_t(q + F, T[kk]);
           lds_barrier();  // q - 1
         }
       });
-    lds_barrier();  // M - 1 (M > 1), else M
-    if (M > 1) lds_barrier();  // M
+    for (int q = max(M - 1, 3); q <= M; ++q) lds_barrier();
     if constexpr (NANCHK) {
       const bool any = __ballot(nan1) != 0;  // all lanes take part
       if (lane == 0) a.nan_flags[c] = any ? 1 : 0;
@@ -1533,7 +1540,7 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
     const float lm = near_block<LPL, DC, PE, 1>(U, th, bh, wi, L1v, 2, cc, nr);
     __builtin_amdgcn_sched_barrier(kSchedValu);
     refill();
-    const float u = near_min_rest<LPL, DC>(lm);
+    const float u = near_min_rest<LPL, DC, FIT == kFitHalf ? 2 : 4>(lm);
     const Vec<LPL> m = minconv<LPL, PE>(U, nr, u, wi, wi2, L2v);
 #pragma unroll
     for (int k = 0; k < LPL; ++k) bh.v[k] = m.v[k] - u;
@@ -1545,42 +1552,58 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
     col = dpp_f<0xe4, 1 << (S >> 2), 1 << (S & 3), false>(col, x);
   };
   Vec<LPL> ra[P];
-  if (nb > 0) {
 #pragma unroll
-    for (int j = 0; j < P; ++j) ra[j] = ld_theta(j < nb ? n - 1 - j : 1);
-  }
+  for (int j = 0; j < P; ++j) ra[j] = ld_theta(j < nb ? n - 1 - j : min(1, nb));
+  const Vec<LPL> a0 = theta_of(ld_theta(0)), c_end = ld_buf<LPL, FIT>(rC, nb * strideB, lane, D);
+  __syncthreads();  // the weights are in LDS
   int s0 = 0;
   float wv = wlane_b(0), wv2 = wlane_b2(0);
-  for (; s0 + P <= nb; s0 += P) {
+  // A block of P steps; low: it may reach the first three segments.
+  auto block_b = [&](bool low) {
     const float wnext = wlane_b(s0 + P), wnext2 = wlane_b2(s0 + P);
     const int bo = (s0 + P + lane < nb ? n - 1 - (s0 + P + lane) : 1) * strideB;  // refill offsets, one per lane
     float uc = 0.f;
     unroll_steps<P>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      const float u = step_b(ra[j], lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, [&]() {
-        ra[j] = ld_buf<LPL, FIT>(rT, __builtin_amdgcn_readlane(bo, j), lane, D, kInfF);
+      const int ip = nb - 1 - (s0 + j) + g;  // the node's forward step
+      const bool ring = low && ip < 3 * K;
+      float* d = msg_ring + ip * 2 * NS + lane * 2 * LPL;
+      const Vec<LPL> th = theta_of(ra[j]);
+      const float u = step_b(th, lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, [&]() {
+        if (ring) put_theta(d, th);
+        ra[j] = ld_buf<LPL, FIT>(rT, __builtin_amdgcn_readlane(bo, j), lane, D);
       });
       collect(uc, u, std::integral_constant<int, j % 16>{});
-      if constexpr (j % 16 == 15) u_lds[n - 2 - (s0 + j - 15 + (lane >> 2))] = uc;
-      if constexpr ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (n - 2 - (s0 + j)) * D * 4, lane, D, bh);
+      if constexpr (j % 16 == 15) u_lds[nb - 1 - (s0 + j - 15 + (lane >> 2))] = uc;
+      if (ring)
+        put_msg(d, bh);
+      else if ((j + 1) % K == 0)
+        st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
     });
     wv = wnext;
     wv2 = wnext2;
-  }
+    s0 += P;
+  };
+  while (s0 + P <= nb - 3 * K) block_b(false);
+  while (s0 + P <= nb) block_b(true);
 #pragma unroll
   for (int j = 0; j < P; ++j)
     if (s0 + j < nb) {
-      u_lds[n - 2 - (s0 + j)] = step_b(ra[j], lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, []() {});
-      if ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (n - 2 - (s0 + j)) * D * 4, lane, D, bh);
+      const int ip = nb - 1 - (s0 + j) + g;
+      float* d = msg_ring + ip * 2 * NS + lane * 2 * LPL;
+      const Vec<LPL> th = theta_of(ra[j]);
+      if (ip < 3 * K) put_theta(d, th);
+      u_lds[nb - 1 - (s0 + j)] = step_b(th, lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, []() {});
+      if (ip < 3 * K)
+        put_msg(d, bh);
+      else if ((j + 1) % K == 0)
+        st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
     }
-  const double bsum = chain_offsets(u_lds, b_lds, n, lane);
-  const Vec<LPL> a0 = ld_theta(0);
-  const Vec<LPL> c_end = ld_buf<LPL, FIT>(rC, (n - 1) * strideB, lane, D, kInfF);
   __syncthreads();
   Vec<LPL> M0;
 #pragma unroll
   for (int k = 0; k < LPL; ++k) M0.v[k] = a0.v[k] + bh.v[k];
-  const double Lambda = bsum + (double)chain_min(local_min(M0));
+  const float m0 = chain_min(local_min(M0));
 
   // ---- chain wave, forward pass
   Vec<LPL> R = a0, t_cur = a0;  // theta of the current node
@@ -1603,7 +1626,6 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
   auto wl2 = [&](int q) { return PE ? w2_lds[max(min(q * K - g + lane, n - 2), 0)] : 0.f; };
   if (M > 0) {
     Pair pr[3];
-    lds_barrier();  // 0: segments 0 and 1 are in the ring
     pr[0] = rd(0);
     pr[1] = rd(1);
     float wf = wl(0), wf2 = wl2(0);
@@ -1630,7 +1652,7 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
           }
           __builtin_amdgcn_sched_barrier(kSchedValu);
           next();
-          const float v = near_min_rest<LPL, DC>(lm);
+          const float v = near_min_rest<LPL, DC, FIT == kFitHalf ? 2 : 4>(lm);
           collect(vc, v, tc);
           const Vec<LPL> m = minconv<LPL, PE>(V, nr, v, wi, wi2, L2v);
           Vec<LPL> mm, nx, am, o;
@@ -1683,7 +1705,7 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
   st_buf<LPL, FIT>(rW, (n - 1) * strideB, lane, D, out);
   const double kept = chain_kept(v_lds, b_lds, n, lane, kGammaD);
   if (lane == 0) {
-    a.lam[c] = Lambda;
+    a.lam[c] = (M > 0 ? b_lds[n] : 0.0) + (double)m0;  // (n = 1: nothing orders the waves)
     a.kept[c] = kept;
   }
 }
@@ -1711,8 +1733,8 @@ __device__ __forceinline__ void ring_pass(Rsrc rA, int strideB, Rsrc rM, const f
   Vec<LPL> ra[P], rm[P];
   auto load = [&](int s, Vec<LPL>& av, Vec<LPL>& mv) {
     const int i = first + dir * (s < cnt ? s : cnt - 1);
-    av = ld_buf<LPL, FIT>(rA, (i + aoff) * strideB, lane, D, kInfF);
-    if constexpr (MSG) mv = ld_buf<LPL, FIT>(rM, i * D * 4, lane, D, 0.f);
+    av = ld_buf<LPL, FIT>(rA, (i + aoff) * strideB, lane, D);
+    if constexpr (MSG) mv = ld_buf<LPL, FIT>(rM, i * D * 4, lane, D);
   };
   auto wlane = [&](int s0) { return w_lds[max(min(first + dir * (s0 + lane) + woff, n - 2), 0)]; };
   auto wlane2 = [&](int s0) { return PE ? w2_lds[max(min(first + dir * (s0 + lane) + woff, n - 2), 0)] : 0.f; };
@@ -1755,6 +1777,7 @@ template <int LPL, int P, int FIT, int DC, bool GAP, bool PE>
 __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
   extern __shared__ double lds2[];
   constexpr int K = seg_len<LPL>();
+  constexpr int ROWS = FIT == kFitHalf ? 2 : 4;
   static_assert(P == kRowRing * K, "the message waves' register ring spans three segments");
   static_assert(P <= 64, "one weight per lane and step of a block");
   constexpr int kNS = 64 * LPL;  // ring stride per node, floats
@@ -1795,16 +1818,16 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
   Vec<LPL> X;  // wave 0: F_i, wave 1: Bh_i
   auto fwd = [&](const Vec<LPL>& an, float w, float w2) {  // F_i = A_i + minconv(F_{i-1}; w_{i-1}) - min F_{i-1}
     Vec<LPL> nr;
-    const float f = near_min_rest<LPL, DC>(near_block<LPL, DC, PE, 0>(X, X, X, w, L1v, a.delta, cc, nr));
+    const float f = near_min_rest<LPL, DC, ROWS>(near_block<LPL, DC, PE, 0>(X, X, X, w, L1v, a.delta, cc, nr));
     const Vec<LPL> m = minconv<LPL, PE>(X, nr, f, w, w2, L2v);
 #pragma unroll
-    for (int k = 0; k < LPL; ++k) X.v[k] = keep(k) ? an.v[k] + m.v[k] - f : kInfF;
+    for (int k = 0; k < LPL; ++k) X.v[k] = an.v[k] + m.v[k] - f;
+    X = masked<LPL, FIT>(X, lane, D, kInfF);
   };
   auto bwd = [&](int i, const Vec<LPL>& an1, float w, float w2) {  // Bh_i from Bh_{i+1}, A_{i+1} and w_i
-    Vec<LPL> th, U, nr;
-#pragma unroll
-    for (int k = 0; k < LPL; ++k) th.v[k] = keep(k) ? an1.v[k] : kInfF;
-    const float u = near_min_rest<LPL, DC>(near_block<LPL, DC, PE, 1>(U, th, X, w, L1v, a.delta, cc, nr));
+    Vec<LPL> U, nr;
+    const Vec<LPL> th = masked<LPL, FIT>(an1, lane, D, kInfF);
+    const float u = near_min_rest<LPL, DC, ROWS>(near_block<LPL, DC, PE, 1>(U, th, X, w, L1v, a.delta, cc, nr));
     const Vec<LPL> m = minconv<LPL, PE>(U, nr, u, w, w2, L2v);
 #pragma unroll
     for (int k = 0; k < LPL; ++k) X.v[k] = keep(k) ? m.v[k] - u : 0.f;
@@ -1818,7 +1841,7 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
     float best = kInfF;
 #pragma unroll
     for (int k = 0; k < LPL; ++k) best = fminf(best, valid[k] ? F.v[k] + b.v[k] : kInfF);
-    const float gbest = chain_min(best);
+    const float gbest = chain_min<ROWS>(best);
     const float thr = gbest + kTieEps * fmaxf(1.f, fabsf(gbest));
     int bj = LPL;
 #pragma unroll
@@ -1834,14 +1857,14 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
         const float mm = valid[k] ? F.v[k] + b.v[k] : kInfF;
         if (lane * LPL + k != label) second = fminf(second, mm);
       }
-      a.gap[p] = chain_min(second) - gbest;
+      a.gap[p] = chain_min<ROWS>(second) - gbest;
     }
     a.labels[p] = label;
   };
 
   // Phase 1: waves 0 and 1 walk to the midpoint, storing their messages.
   if (wv == 0) {
-    X = ld_node<LPL, FIT>(Ab, lane, D, kInfF);  // F_0 = A_0
+    X = masked<LPL, FIT>(ld_node<LPL, FIT>(Ab, lane, D), lane, D, kInfF);  // F_0 = A_0
     if (mid > 0) st_node<LPL, FIT>(msg, lane, D, X);
     ring_pass<LPL, FIT, P, false, PE>(rA, strideB, rM, w_lds, w2_lds, n, D, lane, 1, mid - 1, 1, 0, -1,
                                        [&](int i, const Vec<LPL>& an, const Vec<LPL>&, float w, float w2) {
@@ -1873,7 +1896,7 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
     auto wnode = [&](int j) { return max(min(wv == 0 ? mid + j - 1 : mid - 1 - j, n - 2), 0); };
     Vec<LPL> ra[P];
 #pragma unroll
-    for (int t = 0; t < P; ++t) ra[t] = ld_buf<LPL, FIT>(rA, anode(t) * strideB, lane, D, kInfF);
+    for (int t = 0; t < P; ++t) ra[t] = ld_buf<LPL, FIT>(rA, anode(t) * strideB, lane, D);
     for (int jb = 0; jb < S * K; jb += P) {
       const float wl = w_lds[wnode(jb + lane)];
       const float wl2 = PE ? w2_lds[wnode(jb + lane)] : 0.f;
@@ -1884,7 +1907,7 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
         const int j = jb + t;
         const Vec<LPL> an = fresh(ra[t]);
         __builtin_amdgcn_sched_barrier(kSchedValu);
-        ra[t] = ld_buf<LPL, FIT>(rA, __builtin_amdgcn_readlane(ao, t), lane, D, kInfF);
+        ra[t] = ld_buf<LPL, FIT>(rA, __builtin_amdgcn_readlane(ao, t), lane, D);
         if (j < len) {
           if (wv == 0) {
             if (j > 0 || mid > 0) fwd(an, lane_weight(wl, t), PE ? lane_weight(wl2, t) : 0.f);
@@ -1899,11 +1922,11 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
     lds_barrier();  // round S (the decision waves' last segment)
     if (wv == 1) {
       // Chain minimum: sum of the backward minima + min(A_0 + Bh_0).
-      const Vec<LPL> a0 = ld_node<LPL, FIT>(Ab, lane, D, kInfF);
+      const Vec<LPL> a0 = masked<LPL, FIT>(ld_node<LPL, FIT>(Ab, lane, D), lane, D, kInfF);
       Vec<LPL> M0;
 #pragma unroll
       for (int k = 0; k < LPL; ++k) M0.v[k] = a0.v[k] + X.v[k];
-      const double Lambda = chain_total(u_lds, n, lane) + (double)chain_min(local_min(M0));
+      const double Lambda = chain_total(u_lds, n, lane) + (double)chain_min<ROWS>(local_min(M0));
       if (lane == 0) a.lam[c] = Lambda;
     }
   } else {
@@ -1919,7 +1942,7 @@ __global__ __launch_bounds__(256) void k_decode4(ChainArgs a) {
 #pragma unroll
       for (int t = 0; t < K; ++t) {
         const int i = min(max(node_of(s * K + t), 0), n - 1);
-        o[t] = ld_buf<LPL, FIT>(rM, i * D * 4, lane, D, 0.f);
+        o[t] = ld_buf<LPL, FIT>(rM, i * D * 4, lane, D);
       }
     };
     auto decide_seg = [&](int s, const Vec<LPL> (&o)[K]) {
@@ -2009,24 +2032,32 @@ static void launch_one(ChainArgs& a, size_t lds, bool seg, hipStream_t st) {
     const size_t lds2 = sizeof(float) * ((((PE ? 3 : 2) * (size_t)a.n + 3) & ~(size_t)3) +
                                          (size_t)2 * 2 * seg_len<LPL>() * 64 * LPL);
     constexpr int PD = row_seg_p<LPL>();
-    if (lds2 > 64 * 1024) {
-      (void)hipFuncSetAttribute((const void*)k_decode4<LPL, PD, FIT, DC, true, PE>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2);
-      (void)hipFuncSetAttribute((const void*)k_decode4<LPL, PD, FIT, DC, false, PE>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2);
-    }
-    if (a.gap)
-      k_decode4<LPL, PD, FIT, DC, true, PE><<<a.n_chains, 256, lds2, st>>>(a);
-    else
-      k_decode4<LPL, PD, FIT, DC, false, PE><<<a.n_chains, 256, lds2, st>>>(a);
+    auto decode = [&](auto fit, auto gap) {
+      constexpr int F = decltype(fit)::value;
+      constexpr bool GAP = decltype(gap)::value;
+      if (lds2 > 64 * 1024)
+        (void)hipFuncSetAttribute((const void*)k_decode4<LPL, PD, F, DC, GAP, PE>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2);
+      k_decode4<LPL, PD, F, DC, GAP, PE><<<a.n_chains, 256, lds2, st>>>(a);
+    };
+    auto either = [&](auto fit) { a.gap ? decode(fit, std::true_type{}) : decode(fit, std::false_type{}); };
+    if constexpr (LPL == 1 && FIT == kFitLanes)
+      if (a.D <= 32) return either(std::integral_constant<int, kFitHalf>{});
+    either(std::integral_constant<int, FIT>{});
   } else {
     constexpr bool kCols = MODE == kColsMinorant;
     constexpr int PS = kCols ? P : row_seg_p<LPL>();  // ring depth of the checkpointed sweep
     if constexpr (DC == 2 && LPL <= 2) {
       if (use_line<LPL, MODE>(a)) {
-        if constexpr (!kCols)
-          if (a.nan_flags) return launch_line<LPL, FIT, PE, false, true>(a, st);
-        return launch_line<LPL, FIT, PE, kCols, false>(a, st);
+        auto line = [&](auto fit) {
+          constexpr int F = decltype(fit)::value;
+          if constexpr (!kCols)
+            if (a.nan_flags) return launch_line<LPL, F, PE, false, true>(a, st);
+          launch_line<LPL, F, PE, kCols, false>(a, st);
+        };
+        if constexpr (LPL == 1 && FIT == kFitLanes)
+          if (a.D <= 32) return line(std::integral_constant<int, kFitHalf>{});
+        return line(std::integral_constant<int, FIT>{});
       }
     }
     auto sweep = [&](auto nan) {

@@ -51,6 +51,20 @@ def test_bands_equal_whole(handle, D, n):
         assert torch.allclose(total, sums, rtol=0, atol=chains * 2.0 ** -52 * float(chains * n))
 
 
+@pytest.mark.parametrize("D", [2, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize("H,W", [(5, 1), (3, 2), (9, 40), (4, 77)])
+def test_decode_ignores_infinite_labels(handle, D, H, W):
+    """Labels and gaps of D labels, and of 64 of which all but D cost +inf."""
+    g = torch.Generator(device="cuda").manual_seed(D + W)
+    A = -torch.softmax(3 * torch.randn((H, W, D), generator=g, device="cuda"), dim=2)
+    wx = torch.rand((H, W), generator=g, device="cuda")
+    full = torch.full((H, W, 64), float("inf"), device="cuda")
+    full[:, :, :D] = A
+    got, want = (ops.slackprop_decode_gap(handle, x, wx, 0.5, 2.0, 2) for x in (A, full))
+    assert torch.equal(got[0], want[0])
+    assert torch.equal(bits(got[1]), bits(want[1]))
+
+
 @pytest.mark.parametrize("D", [66, 128])
 @pytest.mark.parametrize("H,W", [(7, 41), (300, 10), (1, 20), (20, 1)])
 def test_per_edge_equals_element_path(handle, D, H, W):
