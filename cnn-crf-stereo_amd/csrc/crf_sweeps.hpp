@@ -1440,10 +1440,10 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
       }
       load(q + F, k);
     };
-    unroll_steps<F>([&](auto k) { load(decltype(k)::value, k); });
     fill_weights();
     __syncthreads();
     __syncthreads();
+    unroll_steps<F>([&](auto k) { load(decltype(k)::value, k); });
     for (int q = 0; q < M; q += F)
       unroll_steps<F>([&](auto k) {
         const int qk = q + decltype(k)::value;
@@ -1551,54 +1551,60 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
     constexpr int S = decltype(slot)::value;
     col = dpp_f<0xe4, 1 << (S >> 2), 1 << (S & 3), false>(col, x);
   };
-  Vec<LPL> ra[P];
+  // The steps down to the first three segments run through the register ring;
+  // those of the first three segments, the last, have their unaries from the start.
+  const int nhi = max(nb - (3 * K - g), 0);
+  Vec<LPL> ra[P], lo[3 * K];
 #pragma unroll
-  for (int j = 0; j < P; ++j) ra[j] = ld_theta(j < nb ? n - 1 - j : min(1, nb));
+  for (int j = 0; j < P; ++j) ra[j] = ld_theta(j < nhi ? n - 1 - j : min(1, nb));
+#pragma unroll
+  for (int t = 0; t < 3 * K; ++t) lo[t] = ld_theta(max(min(t - g, nb - 1) + 1, 0));
   const Vec<LPL> a0 = theta_of(ld_theta(0)), c_end = ld_buf<LPL, FIT>(rC, nb * strideB, lane, D);
   __syncthreads();  // the weights are in LDS
   int s0 = 0;
   float wv = wlane_b(0), wv2 = wlane_b2(0);
-  // A block of P steps; low: it may reach the first three segments.
-  auto block_b = [&](bool low) {
+  for (; s0 + P <= nhi; s0 += P) {
     const float wnext = wlane_b(s0 + P), wnext2 = wlane_b2(s0 + P);
-    const int bo = (s0 + P + lane < nb ? n - 1 - (s0 + P + lane) : 1) * strideB;  // refill offsets, one per lane
+    const int bo = (s0 + P + lane < nhi ? n - 1 - (s0 + P + lane) : 1) * strideB;  // refill offsets, one per lane
     float uc = 0.f;
     unroll_steps<P>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      const int ip = nb - 1 - (s0 + j) + g;  // the node's forward step
-      const bool ring = low && ip < 3 * K;
-      float* d = msg_ring + ip * 2 * NS + lane * 2 * LPL;
-      const Vec<LPL> th = theta_of(ra[j]);
-      const float u = step_b(th, lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, [&]() {
-        if (ring) put_theta(d, th);
+      const float u = step_b(theta_of(ra[j]), lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, [&]() {
         ra[j] = ld_buf<LPL, FIT>(rT, __builtin_amdgcn_readlane(bo, j), lane, D);
       });
       collect(uc, u, std::integral_constant<int, j % 16>{});
       if constexpr (j % 16 == 15) u_lds[nb - 1 - (s0 + j - 15 + (lane >> 2))] = uc;
-      if (ring)
-        put_msg(d, bh);
-      else if ((j + 1) % K == 0)
-        st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
+      if constexpr ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
     });
     wv = wnext;
     wv2 = wnext2;
-    s0 += P;
-  };
-  while (s0 + P <= nb - 3 * K) block_b(false);
-  while (s0 + P <= nb) block_b(true);
+  }
 #pragma unroll
   for (int j = 0; j < P; ++j)
-    if (s0 + j < nb) {
-      const int ip = nb - 1 - (s0 + j) + g;
-      float* d = msg_ring + ip * 2 * NS + lane * 2 * LPL;
-      const Vec<LPL> th = theta_of(ra[j]);
-      if (ip < 3 * K) put_theta(d, th);
-      u_lds[nb - 1 - (s0 + j)] = step_b(th, lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, []() {});
-      if (ip < 3 * K)
-        put_msg(d, bh);
-      else if ((j + 1) % K == 0)
-        st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
+    if (s0 + j < nhi) {
+      u_lds[nb - 1 - (s0 + j)] = step_b(theta_of(ra[j]), lane_weight(wv, j), PE ? lane_weight(wv2, j) : 0.f, []() {});
+      if ((j + 1) % K == 0) st_buf<LPL, FIT>(rM, (nb - 1 - (s0 + j)) * D * 4, lane, D, bh);
     }
+  {
+    const int e = max(min(lane - g, nb - 1), 0);
+    const float wlow = w_lds[e], wlow2 = PE ? w2_lds[e] : 0.f;
+    float* d = msg_ring + lane * 2 * LPL;
+    float uc = 0.f;
+    unroll_steps<3 * K>([&](auto tc) {
+      constexpr int t = 3 * K - 1 - decltype(tc)::value;  // the node's forward step
+      if (t < M * K && t >= g) {
+        const Vec<LPL> th = theta_of(lo[t]);
+        const float u = step_b(th, lane_weight(wlow, t), PE ? lane_weight(wlow2, t) : 0.f, []() {});
+        collect(uc, u, std::integral_constant<int, t % 16>{});
+        put_msg(d + t * 2 * NS, bh);
+        put_theta(d + t * 2 * NS, th);
+      }
+      if constexpr (t % 16 == 0) {
+        const int i = t - g + (lane >> 2);
+        if (i >= 0 && i < nb - nhi) u_lds[i] = uc;  // (a quad writes its step's value)
+      }
+    });
+  }
   __syncthreads();
   Vec<LPL> M0;
 #pragma unroll
