@@ -18,8 +18,8 @@
 // k_conv_bf16: the same GEMM for the other channel counts (64 and 8): 4-row x
 //   TW-pixel tiles, the whole input tile in LDS, weights in chunk groups
 //   staged through registers, output staged through LDS.
-// k_conv_split (conv_split.hip): the float32 layers of 100 and 64 channels, as
-//   six bf16 products of exactly split operands.
+// k_conv_split (conv_split.hip): the float32 layers of 100 and 64 channels, on
+//   16-bit products of split operands.
 // k_conv_f32: 8-channel float32 layers on v_mfma_f32_16x16x4_f32 (2-row tile),
 //   whose reduction is too short to fill a 32-deep step's four groups.
 // k_conv_generic: VALU direct convolution for the 1- and 3-channel input layer
@@ -999,7 +999,7 @@ extern "C" int ccs_conv_forward_packed(ccs_handle_t h, const void* x, int x_layo
 // GPU (held until the process ends) instead of the handle's scratch.  The
 // array's name is a host-side stand-in, not a device address: host code uses
 // only the address hipGetSymbolAddress returns on each device.
-constexpr size_t kNoAllocScratchBytes = 640u << 10;  // the largest MFMA pack is 645,120 bytes
+constexpr size_t kNoAllocScratchBytes = 512u << 10;  // the largest MFMA pack is 452,032 bytes
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -1,36 +1,40 @@
-// float32 feature layers (fused valid convolution + bias + tanh) on the bf16
+// float32 feature layers (fused valid convolution + bias + tanh) on the 16-bit
 // matrix cores.
 //
-// gfx950 runs v_mfma_f32_16x16x32_bf16 at 16 times the rate of
-// v_mfma_f32_16x16x4_f32.  Both operands are split exactly into three bfloat16
-// terms, x = xh + xm + xl and w = wh + wm + wl (split3), and a product is formed
-// from six of the nine partial products,
-//   xh wh + (xh wm + xm wh) + (xm wm + xh wl + xl wh),
-// each exact in the matrix core and accumulated in float32.  The three products
-// left out (xm wl, xl wm, xl wl) are below 2^-26 |x w| together, under
-// float32's own rounding of a single product.  A 32-deep reduction step is
-// summed from zero and added to the accumulator once, so an output takes 30
+// gfx950 runs v_mfma_f32_16x16x32_f16 (and _bf16) at 16 times the rate of
+// v_mfma_f32_16x16x4_f32.  Both operands are split into two float16 terms,
+// x s = xh + xl and w t = wh + wl (split2: one rounding of at most 2^-24), with a
+// power of two s for each pixel's 32 channels of a stage and t for each output
+// channel, and a product is formed from
+//   wl xh + wh xl + wh xh,
+// each exact in the matrix core and accumulated in float32; wl xl, the one left
+// out, is below 2^-24 |x w|.  Channels past the last multiple of 32 take an exact
+// three-way bfloat16 split (split3) and six of its nine products instead: their
+// reduction steps hold several taps, hence several pixels, in one instruction, so
+// no scale fits.  A 32-deep step is summed from zero and added to the accumulator
+// once (by the fma that takes the pixel's scale back), so an output takes 30
 // roundings at its own size (the float32 instruction took 225): the relative
-// error of a layer against 64 bits is 1.2e-7 (3x3) and 0.8e-7 (2x2), where
+// error of a layer against 64 bits is 1.3e-7 (3x3) and 1.1e-7 (2x2), where
 // v_mfma_f32_16x16x4_f32 left 5.4e-7 and 3.6e-7 (tanh off, 200 x 300 maps).
 //
 // k_conv_split: a workgroup of 4 waves computes a 16 x 16-pixel output tile for
 // all output channels; a wave owns four rows of 16 pixels (MT = 4) times NT
 // 16-channel tiles of accumulators.  The (16+KH-1) x (16+KW-1) input halo tile
 // is staged in LDS one stage of four 8-channel groups at a time, split into its
-// three planes on the way (324 pixels x 64 bytes x 3 = 61 KB for 3x3, so two
-// workgroups share a CU and one's staging runs under the other's MFMAs).  A
-// square tile has the least halo and wastes least at the edges of odd frames.
-// The weights are packed in fragment order and read straight from L2 into
-// registers, one channel tile ahead: per reduction step a wave issues
-// 6 * 4 * NT MFMAs (168 for 100 channels, 2688 cycles) on 12 LDS fragments and
-// 3 NT weight fragments, so the loop has no barrier and is bound by the matrix
-// cores.  Measured (100 channels, against the float32-MFMA kernel it replaces):
-// 3x3 at 1256 x 389 1456 -> 482 us (181 TFLOP/s of the layer, 1.09 PFLOP/s of
-// bf16 products, the rate a large bf16 matrix product reaches on this card),
-// 2x2 at 749 x 501 530 -> 217 us, 2x2 at 325 x 245 140 -> 65 us.  Reading the
-// weights two tiles ahead, or adding a step's sums one tile later, changed
-// nothing (476-485 us).
+// planes on the way (324 pixels x 64 bytes x 2 = 41 KB for 3x3); a step's weights
+// (14 KB for 100 channels) are copied to LDS once per workgroup while the step
+// before runs.  Two workgroups share a CU, and one's staging and epilogue run
+// under the other's MFMAs.  A square tile has the least halo and wastes least at
+// the edges of odd frames.  A step issues 3 * 4 * NT MFMAs (84, 1400 cycles);
+// its additions are spread between the next tile's MFMAs.
+//
+// Measured (100 channels; the float32-MFMA kernel -> six bfloat16 products with
+// the weights read from L2 by every wave -> this): 3x3 at 1256 x 389
+// 1456 -> 565 -> 400 us, 3x3 at 524 x 268 - -> 175 -> 128 us, 2x2 at 749 x 501
+// 530 -> 205 -> 159 us, 2x2 at 325 x 245 140 -> 65 -> 50 us.  At 400 us the
+// matrix cores are busy half of the time at 1.9 GHz; a tile spends 66 % of its
+// time in the steps, 18 % staging and 11 % in the epilogue's tanh.  Four waves per
+// SIMD (half the rows per wave) took 449 us, two steps' loads in flight 439 us.
 #include <type_traits>
 
 #include "conv_split.hpp"
@@ -40,15 +44,24 @@ namespace ccs {
 template <int KH_, int KW_, int CG_, int NT_>
 struct SplitCfg {
   static constexpr int KH = KH_, KW = KW_, CG = CG_, NT = NT_;
-  static constexpr int Cs = CG * 8, MT = 4, TS = 16;
+  static constexpr int Cs = CG * 8, MT = 4, TS = 16, threads = 256;
   static constexpr int taps = KH * KW;
   static constexpr int FULL = CG / 4, REM = CG % 4;  // stages of four groups, groups of the last stage
   static constexpr int REM_NQ = (taps * REM + 3) / 4;
   static constexpr int NQ = FULL * taps + REM_NQ;  // 32-deep reduction steps
   static constexpr int AR = TS + KH - 1, AC = TS + KW - 1, NPX = AR * AC;
-  static constexpr int plane = NPX * 64;  // bytes of one plane of a stage
-  static constexpr int zero_off = 3 * plane;
+  static constexpr int plane = NPX * 64;  // bytes of one plane of a four-group stage
+  static constexpr int rplane = NPX * REM * 16;  // and of the last stage
+  static constexpr int scale_off = 2 * plane > 3 * rplane ? 2 * plane : 3 * rplane;
+  // two steps' weights (two planes; in the last stage three, behind its smaller planes)
+  static constexpr int w2 = NT * 2048, w3 = NT * 3072;
+  static constexpr int w2_off = (scale_off + NPX * 4 + 1023) & ~1023;
+  static constexpr int w3_off = (3 * rplane + 1023) & ~1023;
+  static constexpr int zero_off = w2_off + 2 * w2 > w3_off + 2 * w3 ? w2_off + 2 * w2 : w3_off + 2 * w3;
   static constexpr int lds_bytes = zero_off + 16;
+  // packed weights: two-plane fragments, three-plane fragments, row scales
+  static constexpr size_t frag_bytes = (size_t)NT * 1024 * (2 * FULL * taps + 3 * REM_NQ);
+  static constexpr size_t packed_bytes = frag_bytes + NT * 16 * sizeof(float);
 };
 
 // Reduction step q of the packed weights, lane group lgrp: the tap and the
@@ -68,35 +81,64 @@ __host__ __device__ inline void split_step(int q, int lgrp, int* tap, int* c0) {
   }
 }
 
-// Packed layout: [q][t][plane][lane][8], the fragment of channel tile t, with
-// lane (lrow, lgrp) holding output channel 16 t + lrow.  One thread per lane.
+// Packed layout: step q < FULL * taps as [q][t][2][lane][8] float16, the others
+// as [q][t][3][lane][8] bfloat16, the fragment of channel tile t with lane
+// (lrow, lgrp) holding output channel 16 t + lrow; then the row scales.  All
+// weights of a row are divided by its scale.  Block (t, y) packs a share of tile
+// t's steps; its 16 groups of 16 lanes each look at one row first.
+constexpr int kPackShares = 8;
 template <class Cfg>
-__global__ void k_pack_split(const float* __restrict__ w, int K, int C, int adj, bf16* __restrict__ out) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= Cfg::NQ * Cfg::NT * 64) return;
-  const int lane = idx & 63, t = (idx >> 6) % Cfg::NT, q = (idx >> 6) / Cfg::NT;
-  const int n = 16 * t + (lane & 15);
-  int tap, c0;
-  split_step<Cfg>(q, lane >> 4, &tap, &c0);
-  float v[8];
-  bf16 p[3][8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int c = c0 + e;
-    const int i = tap / Cfg::KW, j = tap % Cfg::KW;
-    // adj: Wt[n][c] flipped, Wt[n][c][a][b] = w[c][n][KH-1-a][KW-1-b]
-    v[e] = n < K && c0 >= 0 && c < C
-               ? w[adj ? (((long)c * K + n) * Cfg::KH + i) * Cfg::KW + j
-                       : (((long)n * C + c) * Cfg::KH + (Cfg::KH - 1 - i)) * Cfg::KW + (Cfg::KW - 1 - j)]
-               : 0.f;
+__global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w, int K, int C, int adj,
+                                                    unsigned char* __restrict__ out) {
+  __shared__ int exps[16];
+  const int tid = threadIdx.x, t = blockIdx.x;
+  // adj: Wt[n][c] flipped, Wt[n][c][a][b] = w[c][n][KH-1-a][KW-1-b]
+  auto at = [&](int n, int c, int tap) {
+    return w[adj ? ((long)c * K + n) * Cfg::taps + tap : ((long)n * C + c) * Cfg::taps + (Cfg::taps - 1 - tap)];
+  };
+  {
+    const int n = 16 * t + (tid >> 4);
+    unsigned mx = 0;
+    if (n < K)
+      for (int i = tid & 15; i < C * Cfg::taps; i += 16) mx = max(mx, finite_bits(at(n, i / Cfg::taps, i % Cfg::taps)));
+    for (int o = 1; o < 16; o <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 16));
+    if ((tid & 15) == 0) {
+      exps[tid >> 4] = split_exp(mx);
+      if (blockIdx.y == 0)
+        reinterpret_cast<float*>(out + Cfg::frag_bytes)[n] = __uint_as_float((unsigned)split_exp(mx) << 23);
+    }
   }
-  split3(v, p[0], p[1], p[2]);
+  __syncthreads();
+  for (int u = blockIdx.y * 256 + tid; u < Cfg::NQ * 64; u += kPackShares * 256) {
+    const int q = u >> 6, lane = u & 63, n = 16 * t + (lane & 15);
+    const int eb = exps[lane & 15];
+    int tap, c0;
+    split_step<Cfg>(q, lane >> 4, &tap, &c0);
+    float v[8];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    bf16x8 o;
+    for (int e = 0; e < 8; ++e) v[e] = n < K && c0 >= 0 && c0 + e < C ? at(n, c0 + e, tap) : 0.f;
+    constexpr int NQ2 = Cfg::FULL * Cfg::taps;
+    if (q < NQ2) {
+      f16x8 p[2];
+      split2<false>(v, split_scale(eb), p[0], p[1]);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = p[k][e];
-    *reinterpret_cast<bf16x8*>(out + (((long)(q * Cfg::NT + t) * 3 + k) * 64 + lane) * 8) = o;
+      for (int k = 0; k < 2; ++k)
+        *reinterpret_cast<f16x8*>(out + ((long)((q * Cfg::NT + t) * 2 + k) * 64 + lane) * 16) = p[k];
+    } else {
+      const float unit = __uint_as_float(eb < 254 ? (unsigned)(254 - eb) << 23 : 0x400000u);  // 1 / the row's scale
+      bf16 p[3][8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= unit;
+      split3(v, p[0], p[1], p[2]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = p[k][e];
+        *reinterpret_cast<bf16x8*>(out + (size_t)NQ2 * Cfg::NT * 2048 +
+                                   ((long)(((q - NQ2) * Cfg::NT + t) * 3 + k) * 64 + lane) * 16) = o;
+      }
+    }
   }
 }
 
@@ -104,9 +146,14 @@ __global__ void k_pack_split(const float* __restrict__ w, int K, int C, int adj,
 // eight consecutive pixels land in eight distinct bank groups.
 __device__ __forceinline__ int split_swz(int px, int g) { return g ^ ((px >> 1) & 3); }
 
+// Each lane's 16 bytes from src go to dst + 16 lane (dst is uniform), counted by vmcnt.
+__device__ __forceinline__ void load_lds16(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
 template <class Cfg>
 __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__ x, int Hin, int Win,
-                                                       const bf16* __restrict__ wpk, const float* __restrict__ bias,
+                                                       const unsigned char* __restrict__ wpk, const float* __restrict__ bias,
                                                        int K, int act, float* __restrict__ y, int Ho, int Wo,
                                                        int tiles_x, int tiles) {
   constexpr int MT = Cfg::MT, NT = Cfg::NT, AC = Cfg::AC, NPX = Cfg::NPX, Cs = Cfg::Cs;
@@ -128,154 +175,236 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   // past Ho x Wo).
   auto stage = [&](auto gc, int cg0) {
     constexpr int G = decltype(gc)::value;
-    constexpr int NU = NPX * G, PER = (NU + 255) / 256;
-    u32x4 r[PER][2];
+    constexpr int NU = NPX * G, PER = (NU + Cfg::threads - 1) / Cfg::threads;
+    f32x4 r[PER][2];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int v = min(tid + 256 * i, NU - 1);
+      const int v = min(tid + Cfg::threads * i, NU - 1);
       const int px = v / G, g = v % G;
       const int hi = min(h0 + px / AC, Hin - 1), wi = min(w0 + px % AC, Win - 1);
-      const u32x4* src = reinterpret_cast<const u32x4*>(x + ((long)hi * Win + wi) * Cs + (cg0 + g) * 8);
+      const f32x4* src = reinterpret_cast<const f32x4*>(x + ((long)hi * Win + wi) * Cs + (cg0 + g) * 8);
       r[i][0] = src[0];
       r[i][1] = src[1];
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int v = tid + 256 * i;
+      const int v = tid + Cfg::threads * i;
       const int px = v / G, g = v % G;
       float f[8];
-      bf16 p[3][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = __uint_as_float(r[i][e >> 2][e & 3]);
-      split3(f, p[0], p[1], p[2]);
-      const int off = G == 4 ? px * 64 + split_swz(px, g) * 16 : (px * G + g) * 16;
-      if (v < NU) {
+      for (int e = 0; e < 8; ++e) f[e] = r[i][e >> 2][e & 3];
+      if constexpr (G == 4) {
+        // A pixel's four units lie in a quad of lanes: one scale for its 32 channels.
+        auto quad_max = [](unsigned m) {
+          m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0xb1, 0xf, 0xf, true));
+          return max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x4e, 0xf, 0xf, true));
+        };
+        unsigned mx = 0;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          bf16x8 o;
+        for (int e = 0; e < 8; ++e) mx = max(mx, __float_as_uint(f[e]) & 0x7fffffffu);
+        const bool finite = !__any(mx >= 0x7f800000u);
+        if (!finite) {
+          mx = 0;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = p[k][e];
-          *reinterpret_cast<bf16x8*>(lds + k * Cfg::plane + off) = o;
+          for (int e = 0; e < 8; ++e) mx = max(mx, finite_bits(f[e]));
+        }
+        const int eb = split_exp(quad_max(mx));
+        f16x8 p[2];
+        if (finite)
+          split2<true>(f, split_scale(eb), p[0], p[1]);
+        else
+          split2<false>(f, split_scale(eb), p[0], p[1]);
+        if (v < NU) {
+          const int off = px * 64 + split_swz(px, g) * 16;
+#pragma unroll
+          for (int k = 0; k < 2; ++k) *reinterpret_cast<f16x8*>(lds + k * Cfg::plane + off) = p[k];
+          if (g == 0) *reinterpret_cast<float*>(lds + Cfg::scale_off + px * 4) = split_unscale(eb);
+        }
+      } else {
+        bf16 p[3][8];
+        split3(f, p[0], p[1], p[2]);
+        if (v < NU) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = p[k][e];
+            *reinterpret_cast<bf16x8*>(lds + k * Cfg::rplane + (px * G + g) * 16) = o;
+          }
         }
       }
     }
   };
 
-  // Accumulators start at the bias: lane (lrow, lgrp) holds pixel lrow of row
-  // 4 wave + m and channels 16 t + 4 lgrp .. +3 (the weights are the A operand).
+  // Lane (lrow, lgrp) holds pixel lrow of row 4 wave + m and channels
+  // 16 t + 4 lgrp .. +3 (the weights are the A operand), over the rows' scales.
   f32x4 acc[MT][NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    f32x4 bn;
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int n = 16 * t + 4 * lgrp + e;
-      bn[e] = (n < K && bias) ? bias[n] : 0.f;
+    for (int m = 0; m < MT; ++m) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // A step's weight fragments (1 KB each: one load of a wave, straight to LDS)
+  // are copied once per workgroup, a step ahead, to the buffer the step before
+  // has left.
+  auto copy_w = [&](const unsigned char* src, int off, int frags) {
+#pragma unroll 1
+    for (int f = wave; f < frags; f += 4) load_lds16(src + (long)f * 1024 + lane * 16, lds + off + f * 1024);
+  };
+  auto copy2 = [&](int q) { copy_w(wpk + (long)q * Cfg::w2, Cfg::w2_off + (q & 1) * Cfg::w2, 2 * NT); };
+  auto copy3 = [&](int ql) {
+    copy_w(wpk + (long)Cfg::FULL * Cfg::taps * Cfg::w2 + (long)ql * Cfg::w3, Cfg::w3_off + (ql & 1) * Cfg::w3, 3 * NT);
+  };
+  // The copies of this wave have arrived, and so have everyone's.
+  auto step_barrier = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+
+  // The step's products are summed from zero and added to the accumulators
+  // once, in the vector unit: the matrix core's roundings then happen at the
+  // size of 32 products, and only the additions at that of the whole sum.
+  auto step2 = [&](int q, int ti, int tj) {
+    f16x8 a[2][MT];
+    float sc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int px = (MT * wave + m + ti) * AC + tj + lrow;
+      const int o = px * 64 + split_swz(px, lgrp) * 16;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) a[k][m] = *reinterpret_cast<const f16x8*>(lds + o + k * Cfg::plane);
+      sc[m] = *reinterpret_cast<const float*>(lds + Cfg::scale_off + px * 4);
+    }
+    const f16x8* wb = reinterpret_cast<const f16x8*>(lds + Cfg::w2_off + (q & 1) * Cfg::w2) + lane;
+    f16x8 b0[2] = {wb[0], wb[64]}, b1[2];
+    f32x4 cur[2][MT];
+    auto add = [&](int t, int m) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[m][t][e] = fmaf(cur[t & 1][m][e], sc[m], acc[m][t][e]);
+    };
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      f32x4(&c)[MT] = cur[t & 1];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        c[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[1], a[0][m], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      // (the next tile's fragments are read behind these: the wait before a
+      // tile's first product is for every LDS read issued so far)
+      __builtin_amdgcn_sched_barrier(0);
+      b1[0] = wb[128 * min(t + 1, NT - 1)];
+      b1[1] = wb[128 * min(t + 1, NT - 1) + 64];
+      if (t > 0) add(t - 1, 0);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        c[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[0], a[1][m], c[m], 0, 0, 0);
+        if (t > 0 && m > 0) add(t - 1, m);
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) c[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[0], a[0][m], c[m], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      b0[0] = b1[0];
+      b0[1] = b1[1];
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m][t] = bn;
-  }
-
-  // Weight fragments: three planes of a channel tile, 1 KB apart.  Fragment
-  // f = q * NT + t; a read past the last one is clamped to it.
-  const bf16x8* wl = reinterpret_cast<const bf16x8*>(wpk) + lane;
-  auto load_w = [&](int f, bf16x8 (&b)[3]) {
-    const bf16x8* p = wl + (long)min(f, Cfg::NQ * NT - 1) * 3 * 64;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) b[k] = p[64 * k];
+    for (int m = 0; m < MT; ++m) add(NT - 1, m);
   };
-  bf16x8 b0[3], b1[3];
-  load_w(0, b0);
-
-  // One reduction step: offs(m) is the LDS byte offset of row tile m's fragment
-  // in plane 0, poff the plane distance (0 for the zero vector).
-  auto step = [&](int q, auto&& offs, int poff) {
+  // A step of the last stage (ql of REM_NQ): its lane groups hold different taps,
+  // hence different pixels, so it takes the exact three-way split without scales.
+  auto step3 = [&](int ql) {
+    constexpr int R = Cfg::REM > 0 ? Cfg::REM : 1;
+    const int kg = 4 * ql + lgrp;
+    const bool ok = kg < Cfg::taps * R;
+    const int tap = ok ? kg / R : 0, g = ok ? kg % R : 0;
+    const int ti = tap / Cfg::KW, tj = tap % Cfg::KW;
     bf16x8 a[3][MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const int o = offs(m);
+      const int px = (MT * wave + m + ti) * AC + tj + lrow;
+      const int o = ok ? (px * R + g) * 16 : Cfg::zero_off;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) a[k][m] = *reinterpret_cast<const bf16x8*>(lds + o + k * poff);
+      for (int k = 0; k < 3; ++k) a[k][m] = *reinterpret_cast<const bf16x8*>(lds + o + (ok ? k * Cfg::rplane : 0));
     }
-    // The step's products are summed from zero and added to the accumulators
-    // once, in the vector unit: the matrix core's roundings then happen at the
-    // size of 32 products, and only the additions at that of the whole sum.
+    const bf16x8* p = reinterpret_cast<const bf16x8*>(lds + Cfg::w3_off + (ql & 1) * Cfg::w3) + lane;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      load_w(q * NT + t + 1, b1);
-      __builtin_amdgcn_sched_barrier(0);
+      bf16x8 b[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) b[k] = p[t * 192 + 64 * k];
       f32x4 cur[MT];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        cur[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0[0], a[2][m], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        cur[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0], a[2][m], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
       auto mm = [&](int kw, int kx) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          cur[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0[kw], a[kx][m], cur[m], 0, 0, 0);
+          cur[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kw], a[kx][m], cur[m], 0, 0, 0);
       };
       mm(2, 0);
       mm(1, 1);
       mm(0, 1);
       mm(1, 0);
       mm(0, 0);
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) acc[m][t] += cur[m];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) b0[k] = b1[k];
+      for (int m = 0; m < MT; ++m) {
+        acc[m][t] += cur[m];
+        asm volatile("" : "+v"(acc[m][t]));  // added here, not behind the step (the sums of all tiles would spill)
+      }
     }
   };
 
+  copy2(0);
 #pragma unroll 1
   for (int s = 0; s < Cfg::FULL; ++s) {
-    if (s > 0) __syncthreads();  // every wave has read the previous stage
     stage(std::integral_constant<int, 4>{}, 4 * s);
-    __syncthreads();
+    step_barrier();
 #pragma unroll 1
     for (int tap = 0; tap < Cfg::taps; ++tap) {
-      const int ti = tap / Cfg::KW, tj = tap % Cfg::KW;
-      step(
-          s * Cfg::taps + tap,
-          [&](int m) {
-            const int px = (4 * wave + m + ti) * AC + tj + lrow;
-            return px * 64 + split_swz(px, lgrp) * 16;
-          },
-          Cfg::plane);
+      const int q = s * Cfg::taps + tap;
+      if (q + 1 < Cfg::FULL * Cfg::taps) copy2(q + 1);
+      step2(q, tap / Cfg::KW, tap % Cfg::KW);
+      step_barrier();
     }
   }
   if constexpr (Cfg::REM > 0) {
-    __syncthreads();
+    copy3(0);
     stage(std::integral_constant<int, Cfg::REM>{}, 4 * Cfg::FULL);
-    __syncthreads();
+    step_barrier();
 #pragma unroll 1
     for (int ql = 0; ql < Cfg::REM_NQ; ++ql) {
-      const int kg = 4 * ql + lgrp;
-      const bool ok = kg < Cfg::taps * Cfg::REM;
-      const int tap = ok ? kg / Cfg::REM : 0, g = ok ? kg % Cfg::REM : 0;
-      const int ti = tap / Cfg::KW, tj = tap % Cfg::KW;
-      step(
-          Cfg::FULL * Cfg::taps + ql,
-          [&](int m) {
-            const int px = (4 * wave + m + ti) * AC + tj + lrow;
-            return ok ? (px * Cfg::REM + g) * 16 : Cfg::zero_off;
-          },
-          ok ? Cfg::plane : 0);
+      if (ql + 1 < Cfg::REM_NQ) copy3(ql + 1);
+      step3(ql);
+      if (ql + 1 < Cfg::REM_NQ) step_barrier();
     }
   }
 
-  // Epilogue: tanh, four channels of one pixel per lane and store (16 bytes).
-  // Padding channels are stored as zeros (an infinite input times their zero
-  // weights is NaN).
+  // Epilogue: row scale, bias, tanh, four channels of one pixel per lane and
+  // store (16 bytes).  Padding channels are stored as zeros (an infinite input
+  // times their zero weights is NaN).
+  __builtin_amdgcn_sched_barrier(0);  // (its loads stay behind the last step: registers)
+  const f32x4* rows = reinterpret_cast<const f32x4*>(wpk + Cfg::frag_bytes);
+  f32x4 rs[NT], bn[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    rs[t] = rows[4 * t + lgrp];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int n = 16 * t + 4 * lgrp + e;
+      bn[t][e] = (n < K && bias) ? bias[n] : 0.f;
+    }
+  }
   auto epilogue = [&](auto f) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const int ho = h0 + 4 * wave + m, wo = w0 + lrow;
+      const int ho = h0 + MT * wave + m, wo = w0 + lrow;
       if (ho >= Ho || wo >= Wo) continue;
       float* row = y + ((long)ho * Wo + wo) * Cs;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int n0 = 16 * t + 4 * lgrp;
-        f32x4 v = {f(acc[m][t][0]), f(acc[m][t][1]), f(acc[m][t][2]), f(acc[m][t][3])};
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = f(fmaf(acc[m][t][e], rs[t][e], bn[t][e]));
         if (16 * t + 16 > K) {  // (uniform) the tile that holds padding channels
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = n0 + e < K ? v[e] : 0.f;
@@ -310,7 +439,7 @@ size_t split_packed_bytes(int K, int C, int KH, int KW) {
   size_t n = 0;
   with_split_cfg(K, C, KH, KW, [&](auto cfg) {
     using Cfg = decltype(cfg);
-    n = (size_t)Cfg::NQ * Cfg::NT * 3 * 1024;
+    n = Cfg::packed_bytes;
   });
   return n;
 }
@@ -318,7 +447,7 @@ size_t split_packed_bytes(int K, int C, int KH, int KW) {
 void split_pack(const float* w, int K, int C, int KH, int KW, int adj, void* packed, hipStream_t st) {
   with_split_cfg(K, C, KH, KW, [&](auto cfg) {
     using Cfg = decltype(cfg);
-    k_pack_split<Cfg><<<ceil_div((long)Cfg::NQ * Cfg::NT * 64, 256), 256, 0, st>>>(w, K, C, adj, (bf16*)packed);
+    k_pack_split<Cfg><<<dim3(Cfg::NT, kPackShares), 256, 0, st>>>(w, K, C, adj, (unsigned char*)packed);
   });
 }
 
@@ -330,7 +459,7 @@ void split_launch(const float* x, int H, int W, int C, const void* packed, const
     const int Ho = H - KH + 1, Wo = W - KW + 1;
     const int tx = (int)ceil_div(Wo, Cfg::TS), tiles = tx * (int)ceil_div(Ho, Cfg::TS);
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::lds_bytes);
-    kern<<<8 * ((tiles + 7) / 8), 256, Cfg::lds_bytes, st>>>(x, H, W, (const bf16*)packed, b, K, act, y, Ho, Wo, tx,
+    kern<<<8 * ((tiles + 7) / 8), Cfg::threads, Cfg::lds_bytes, st>>>(x, H, W, (const unsigned char*)packed, b, K, act, y, Ho, Wo, tx,
                                                              tiles);
   });
 }

@@ -1,4 +1,4 @@
-// float32 convolution layers on the bf16 matrix cores (conv_split.hip).
+// float32 convolution layers on the 16-bit matrix cores (conv_split.hip).
 #pragma once
 
 #include "common.hpp"
@@ -38,6 +38,38 @@ __device__ __forceinline__ void split3(const float (&x)[N], bf16 (&h)[N], bf16 (
     const float r = v - (float)h[e];
     m[e] = (bf16)r;
     l[e] = (bf16)(fin ? r - (float)m[e] : x[e]);
+  }
+}
+
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+
+// x s = h + l in float16 with one rounding, for a power of two s that takes the
+// largest |x| of a block to [2^14, 2^15): h is x s rounded to nearest, l the
+// rest rounded to nearest.  What is left out is at most 2^-24 |x|, and never
+// more than 2^-39 of the block's largest value (float16's subnormals are exact
+// in the matrix core).  An infinity or a NaN goes to l alone, as in split3.
+__device__ __forceinline__ unsigned finite_bits(float x) {  // |x| as ordered bits, 0 where it is not finite
+  const unsigned b = __float_as_uint(x) & 0x7fffffffu;
+  return b < 0x7f800000u ? b : 0u;
+}
+// A block's biased exponent from its largest finite_bits (from 29, so that the
+// factors below are normal numbers: smaller blocks keep a share of the bits).
+__device__ __forceinline__ int split_exp(unsigned mx) { return max((int)(mx >> 23), 29); }
+// s, and 2^-28 / s: what a sum of products of two split blocks takes back, but
+// for the other block's own scale 2^(eb - 127).
+__device__ __forceinline__ float split_scale(int eb) { return __uint_as_float((unsigned)(268 - eb) << 23); }
+__device__ __forceinline__ float split_unscale(int eb) { return __uint_as_float((unsigned)(eb - 28) << 23); }
+
+template <bool FINITE>  // every value is finite
+__device__ __forceinline__ void split2(const float (&x)[8], float s, f16x8& h, f16x8& l) {
+  float v[8], r[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool fin = FINITE || (__float_as_uint(x[e]) & 0x7fffffffu) < 0x7f800000u;
+    v[e] = fin ? x[e] * s : 0.f;
+    h[e] = (_Float16)v[e];
+    r[e] = fin ? v[e] - (float)h[e] : x[e];
+    l[e] = (_Float16)r[e];
   }
 }
 

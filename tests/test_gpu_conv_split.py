@@ -1,10 +1,11 @@
-"""float32 layers on split bf16 products: tile edges, value ranges, non-finite inputs.
+"""float32 layers on split 16-bit products: tile edges, value ranges, non-finite inputs.
 
-The layer's six partial products leave out less than 2^-26 |x w| of each
-product; a 32-deep step has at most six roundings at the size of its partial
-sums and the 30 steps one each, so |error| <= 48 * 2^-24 * (sum |x w| + |b|).
-The relative 2-norm is held to 3e-7: 30 random roundings give about 1.5e-7, one
-missing partial product 1e-6 or more.
+A float16 pair holds a value to 2^-24 of itself and 2^-39 of its block's largest
+value, and the products leave out 2^-24 |x w| more: 4 * 2^-24 |x w| in all; the
+exact three-way split leaves out 2^-26 |x w|.  A 32-deep step has at most six
+roundings at the size of its partial sums and the 30 steps one each, so |error|
+<= 48 * 2^-24 * (sum |x w| + |b|).  The relative 2-norm is held to 3e-7: 30 random
+roundings give about 1.5e-7, one missing partial product 1e-6 or more.
 """
 import numpy as np
 import pytest
@@ -55,6 +56,19 @@ def test_split_layer(handle, C, K, k, H, W, scale):
 
 
 @pytest.mark.parametrize("C,k", [(100, 3), (100, 2), (64, 3)])
+def test_split_layer_of_uneven_pixels(handle, C, k):
+    """Pixels and output channels of sizes 1e-12 to 1e12 side by side: every
+    output keeps the precision of its own terms."""
+    rng = np.random.default_rng(C + 7 * k)
+    x = (rng.uniform(-1, 1, (C, 20, 37)) * 10.0 ** rng.uniform(-12, 12, (1, 20, 37))).astype(np.float32)
+    w = (rng.uniform(-0.1, 0.1, (C, C, k, k)) * 10.0 ** rng.uniform(-12, 12, (C, 1, 1, 1))).astype(np.float32)
+    b = np.zeros(C, np.float32)
+    ref, size = reference(x, w, b)
+    got = layer_out(handle, x, w, b).astype(np.float64)
+    assert np.all(np.abs(got - ref) <= 48 * 2.0**-24 * size)
+
+
+@pytest.mark.parametrize("C,k", [(100, 3), (100, 2), (64, 3)])
 def test_split_layer_keeps_infinities_and_nan(handle, C, k):
     """An infinity keeps its sign through every weight (0.5 and 300 split with
     zero and opposite-sign residuals), a NaN stays NaN, and the largest finite
@@ -72,4 +86,4 @@ def test_split_layer_keeps_infinities_and_nan(handle, C, k):
     fin = np.isfinite(ref)
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
-    assert np.all(np.abs(got - ref)[fin] <= 48 * 2.0**-24 * size[fin])
+    assert np.all(np.abs(got[fin] - ref[fin]) <= 48 * 2.0**-24 * size[fin])
