@@ -14,12 +14,13 @@
 // dword (j = 2), the fifth dword read beside them.  (A copy of the row per tap,
 // stored two bytes at a time, took 64 LDS writes per thread and segment.)
 //
-// Bound by the reads of dz and the input (each tap row reads both; timed without
-// them the 1488 x 992 bf16 layer takes two thirds), then by LDS.  Measured with
-// the reduction and k_dz_pad, against the kernels it replaces: bf16 3x3 at 524 x
-// 268 190 -> 108 us, at 1488 x 992 1490 -> 920 us; float32 3x3 at 524 x 268 473
-// -> 332 us.  Two input halves per chunk on four-wave workgroups, two or three
-// per CU, measured the same (110, 990, 357 us): they read dz twice as often.
+// Bound by the steps' LDS reads and, with float32 maps, by splitting them (1.1 us
+// of 4.4 per segment).  Measured with the reduction and k_dz_pad (the kernels it
+// replaced -> with the zeros past a row's end selected beside the loads, which
+// waited for each segment's reads -> now): bf16 3x3 at 524 x 268 190 -> 112 ->
+// 94 us, at 1488 x 992 1490 -> 949 -> 708 us; float32 3x3 at 524 x 268 473 -> 328
+// -> 301 us.  Two input halves per chunk on four-wave workgroups, two or three
+// per CU, measured the same as one (110, 990, 357 us): they read dz twice as often.
 //
 // Blocks b and b + 8 share an XCD: the tap rows of a chunk, which read the same
 // dz and overlapping inputs, are consecutive there.  The block's sums go to
@@ -86,10 +87,14 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
     u.ok = u.g < (u.z ? Csk : Csx) / VE;
     return u;
   };
-  // The next segment to load, as an output row and its first pixel.
+  // The next segment to load, as an output row and its first pixel, and the first
+  // pixel of the loaded one.  A pixel past its row is loaded from the row's start
+  // and zeroed when it is stored: a select beside the load would wait for it.
+  int wo_loaded = 0;
   int lho = (int)(s0 / segs_per_row), lseg = (int)(s0 % segs_per_row);
   auto load_next = [&]() {
     const int ho = lho, wo0 = lseg * SEG;
+    wo_loaded = wo0;
 #pragma unroll
     for (int n = 0; n < Cfg::NU; ++n) {
       const int b = wave + NT * n;
@@ -101,8 +106,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       for (int i = 0; i < 4; ++i) {
         const int px = 4 * u.q + i;
         const bool ok = u.ok && px < left;
-        const u32x4 r = *reinterpret_cast<const u32x4*>(row + (ok ? px * cs + u.g * VE : 0));
-        reg[n][i] = ok ? r : u32x4{0u, 0u, 0u, 0u};
+        reg[n][i] = *reinterpret_cast<const u32x4*>(row + (ok ? px * cs + u.g * VE : 0));
       }
     }
     if (++lseg == segs_per_row) {
@@ -117,6 +121,12 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       if (b > 8) break;
       const Unit u = unit(b);
       if (!u.ok) continue;
+      const int left = (u.z ? Wo : Win) - wo_loaded;
+      if (left < SEG + 4) {  // (uniform) the row may end in this segment
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (4 * u.q + i >= left) reg[n][i] = u32x4{0u, 0u, 0u, 0u};
+      }
       unsigned char* d =
           lds + buf * Cfg::buffer + (u.z ? 0 : PLANES * Cfg::plane) + (u.g * VE * PITCH + 4 * u.q) * 2;
       if constexpr (Cfg::kF32) {
@@ -222,13 +232,19 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   __syncthreads();
   // Segment s is multiplied from buffer (s - s0) % 2 while the next one's
   // registers go into the other (whose readers finished before the barrier).
+  // Waves w and w + 4 share a SIMD: with bf16 maps one stages while the other
+  // multiplies (float32 maps would spill).
   for (long s = s0; s < s1; ++s) {
     const int buf = (int)((s - s0) & 1);
-    if (s + 1 < s1) {
-      store(buf ^ 1);
-      if (s + 2 < s1) load_next();
-    }
+    auto stage = [&]() {
+      if (s + 1 < s1) {
+        store(buf ^ 1);
+        if (s + 2 < s1) load_next();
+      }
+    };
+    if (Cfg::kF32 || wave < 4) stage();
     multiply(buf);
+    if (!Cfg::kF32 && wave >= 4) stage();
     __syncthreads();
   }
 #pragma unroll
