@@ -22,8 +22,9 @@
 //   16-bit products of split operands.
 // k_conv_f32: 8-channel float32 layers on v_mfma_f32_16x16x4_f32 (2-row tile),
 //   whose reduction is too short to fill a 32-deep step's four groups.
-// k_conv_generic: VALU direct convolution for the 1- and 3-channel input layer
-//   and any shape the MFMA kernels do not cover.
+// k_conv_image_split (conv_image.hip): the image layer of 2 and 3 planes (large
+//   float32 maps: of 1), on bf16 products; k_conv_image: the other image layers.
+// k_conv_generic: VALU direct convolution for any shape the others do not cover.
 #include <cmath>
 
 #include <mutex>
@@ -940,6 +941,11 @@ static int conv_generic(ccs_handle_t h, const void* x, int x_layout, int H, int 
   const int Ho = H - KH + 1, Wo = W - KW + 1;
   const int Cs_out = feature_stride(K);
   if (x_layout == CCS_LAYOUT_NCHW && KH == 3 && KW == 3 && K <= 128 && C <= 5) {
+    if (image_split_supported(H, W, C, K, precision)) {
+      image_split_launch((const float*)x, H, W, C, w, b, K, act, precision, y, h->stream);
+      CCS_LAUNCH_CHECK();
+      return CCS_OK;
+    }
     switch (C) {
       case 1: launch_image<1>((const float*)x, H, W, w, b, K, act, precision, y, h->stream); break;
       case 2: launch_image<2>((const float*)x, H, W, w, b, K, act, precision, y, h->stream); break;

@@ -14,6 +14,11 @@ void split_pack(const float* w, int K, int C, int KH, int KW, int adj, void* pac
 void split_launch(const float* x, int H, int W, int C, const void* packed, const float* b, int K, int KH, int KW,
                   int act, float* y, hipStream_t st);
 
+// The image layer (C planes, 3x3) of K channels (conv_image.hip).
+bool image_split_supported(int H, int W, int C, int K, int precision);
+void image_split_launch(const float* x, int H, int W, int C, const float* w, const float* b, int K, int act,
+                        int precision, void* y, hipStream_t st);
+
 // Input gradient of a layer with filters w (K x C x KH x KW) on the MFMA
 // forward kernels: dx (C channels) = true convolution of the padded dz (H x W,
 // K channels) with Wt[c][k][a][b] = w[k][c][KH-1-a][KW-1-b].  *done is false
