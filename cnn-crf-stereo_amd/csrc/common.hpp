@@ -84,6 +84,9 @@ constexpr int kXentBlocks = 4096;
 constexpr int kSumSlots = 64;
 inline size_t run_chain_doubles(int nmax) { return 2 * (size_t)nmax * kSumSlots; }
 
+// Compute units of the current device (crf_chain.hip).
+int cu_count();
+
 inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
 typedef __bf16 bf16;

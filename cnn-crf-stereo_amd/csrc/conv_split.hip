@@ -17,39 +17,39 @@
 // error of a layer against 64 bits is 1.3e-7 (3x3) and 1.1e-7 (2x2), where
 // v_mfma_f32_16x16x4_f32 left 5.4e-7 and 3.6e-7 (tanh off, 200 x 300 maps).
 //
-// k_conv_split: a workgroup of 4 waves computes a 16 x 16-pixel output tile for
-// all output channels; a wave owns four rows of 16 pixels (MT = 4) times NT
-// 16-channel tiles of accumulators.  The (16+KH-1) x (16+KW-1) input halo tile
-// is staged in LDS one stage of four 8-channel groups at a time, split into its
-// planes on the way (324 pixels x 64 bytes x 2 = 41 KB for 3x3); a step's weights
-// (14 KB for 100 channels) are copied to LDS once per workgroup while the step
-// before runs.  Two workgroups share a CU, and one's staging and epilogue run
-// under the other's MFMAs.  A square tile has the least halo and wastes least at
-// the edges of odd frames.  A step issues 3 * 4 * NT MFMAs (84, 1400 cycles);
-// its additions are spread between the next tile's MFMAs.
+// k_conv_split: a workgroup of 4 waves computes a tile of 8 x 16 pixels for all
+// output channels; a wave owns MT = 2 rows of 16 pixels times NT 16-channel tiles
+// of accumulators.  The (8+KH-1) x (16+KW-1) input halo tile is staged in LDS one
+// stage of four 8-channel groups at a time, split into its planes on the way (180
+// pixels x 64 bytes x 2 = 23 KB for 3x3); a step's weights (14 KB for 100
+// channels) are copied to LDS once per workgroup while the step before runs.
+// Three workgroups share a CU, and one's staging and epilogue run under the
+// others' MFMAs.  A step issues 3 * MT * NT MFMAs (42, 700 cycles); its additions
+// are spread between the next tile's MFMAs.
 //
-// Measured (100 channels; the float32-MFMA kernel -> six bfloat16 products with
-// the weights read from L2 by every wave -> this): 3x3 at 1256 x 389
-// 1456 -> 565 -> 400 us, 3x3 at 524 x 268 - -> 175 -> 128 us, 2x2 at 749 x 501
-// 530 -> 205 -> 159 us, 2x2 at 325 x 245 140 -> 65 -> 50 us.  At 400 us the
-// matrix cores are busy half of the time at 1.9 GHz; a tile spends 66 % of its
-// time in the steps, 18 % staging and 11 % in the epilogue's tanh.  Four waves per
-// SIMD (half the rows per wave) took 449 us, two steps' loads in flight 439 us.
+// Measured (100 channels, us; the float32-MFMA kernel -> six bfloat16 products
+// with the weights read from L2 by every wave -> this): 3x3 at 1256 x 389
+// 1456 -> 565 -> 417, at 524 x 268 - -> 175 -> 110, 2x2 at 749 x 501
+// 530 -> 205 -> 157, at 325 x 245 140 -> 65 -> 42, at 200 x 100 - -> 37 -> 18.  At
+// 1256 x 389 the matrix cores are busy half of the time at 1.9 GHz; the rest is
+// staging, the epilogue's tanh, and waits.  Tiles of 16 x 16 (MT = 4, two
+// workgroups per CU) took 412, 128, 163, 52 and 30 us.
 #include <type_traits>
 
 #include "conv_split.hpp"
 
 namespace ccs {
 
-template <int KH_, int KW_, int CG_, int NT_>
+template <int KH_, int KW_, int CG_, int NT_, int MT_ = 2>
 struct SplitCfg {
   static constexpr int KH = KH_, KW = KW_, CG = CG_, NT = NT_;
-  static constexpr int Cs = CG * 8, MT = 4, TS = 16, threads = 256;
+  static constexpr int Cs = CG * 8, MT = MT_, threads = 256;
+  static constexpr int TH = 4 * MT, TW = 16;  // output tile: MT rows of 16 pixels per wave
   static constexpr int taps = KH * KW;
   static constexpr int FULL = CG / 4, REM = CG % 4;  // stages of four groups, groups of the last stage
   static constexpr int REM_NQ = (taps * REM + 3) / 4;
   static constexpr int NQ = FULL * taps + REM_NQ;  // 32-deep reduction steps
-  static constexpr int AR = TS + KH - 1, AC = TS + KW - 1, NPX = AR * AC;
+  static constexpr int AR = TH + KH - 1, AC = TW + KW - 1, NPX = AR * AC;
   static constexpr int plane = NPX * 64;  // bytes of one plane of a four-group stage
   static constexpr int rplane = NPX * REM * 16;  // and of the last stage
   static constexpr int scale_off = 2 * plane > 3 * rplane ? 2 * plane : 3 * rplane;
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   const int per = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (tile >= tiles) return;  // (uniform) the grid is rounded up to 8 runs
-  const int h0 = (tile / tiles_x) * Cfg::TS, w0 = (tile % tiles_x) * Cfg::TS;
+  const int h0 = (tile / tiles_x) * Cfg::TH, w0 = (tile % tiles_x) * Cfg::TW;
   if (tid == 0) *reinterpret_cast<u32x4*>(lds + Cfg::zero_off) = u32x4{0u, 0u, 0u, 0u};
 
   // Stage of G groups from channel group cg0: unit (pixel, group) of eight
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     }
   };
 
-  // Lane (lrow, lgrp) holds pixel lrow of row 4 wave + m and channels
+  // Lane (lrow, lgrp) holds pixel lrow of row MT wave + m and channels
   // 16 t + 4 lgrp .. +3 (the weights are the A operand), over the rows' scales.
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -453,14 +453,25 @@ void split_pack(const float* w, int K, int C, int KH, int KW, int adj, void* pac
 
 void split_launch(const float* x, int H, int W, int C, const void* packed, const float* b, int K, int KH, int KW,
                   int act, float* y, hipStream_t st) {
-  with_split_cfg(K, C, KH, KW, [&](auto cfg) {
+  const int Ho = H - KH + 1, Wo = W - KW + 1;
+  auto launch = [&](auto cfg) {
     using Cfg = decltype(cfg);
     const auto kern = k_conv_split<Cfg>;
-    const int Ho = H - KH + 1, Wo = W - KW + 1;
-    const int tx = (int)ceil_div(Wo, Cfg::TS), tiles = tx * (int)ceil_div(Ho, Cfg::TS);
+    const int tx = (int)ceil_div(Wo, Cfg::TW), tiles = tx * (int)ceil_div(Ho, Cfg::TH);
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::lds_bytes);
-    kern<<<8 * ((tiles + 7) / 8), Cfg::threads, Cfg::lds_bytes, st>>>(x, H, W, (const unsigned char*)packed, b, K, act, y, Ho, Wo, tx,
-                                                             tiles);
+    kern<<<8 * ((tiles + 7) / 8), Cfg::threads, Cfg::lds_bytes, st>>>(x, H, W, (const unsigned char*)packed, b, K, act,
+                                                                     y, Ho, Wo, tx, tiles);
+  };
+  with_split_cfg(K, C, KH, KW, [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    using Small = SplitCfg<Cfg::KH, Cfg::KW, Cfg::CG, Cfg::NT, 1>;
+    // Tiles of four rows while they do not fill two workgroups per CU: the layer
+    // then takes as long as one tile does (us, four rows / eight: 64 x 64 3x3
+    // 24 / 33, 200 x 100 2x2 (325 tiles) 18 / 22, 325 x 245 2x2 (1281) 48 / 42).
+    if ((long)ceil_div(Wo, Small::TW) * ceil_div(Ho, Small::TH) <= 2 * cu_count())
+      launch(Small{});
+    else
+      launch(cfg);
   });
 }
 

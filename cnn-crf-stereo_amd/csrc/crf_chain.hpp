@@ -54,9 +54,6 @@ constexpr size_t row_seg_lds(int lpl, bool per_edge, int n) {
                           (size_t)kRowRing * seg_length(lpl) * 64 * lpl);
 }
 
-// Compute units of the current device.
-int cu_count();
-
 // One sweep of MODE for LPL (1, 2 or 4) labels per lane; seg: the checkpointed schemes.
 template <int LPL, int MODE>
 int launch_labels(ChainArgs& a, bool seg, hipStream_t st);
