@@ -10,7 +10,7 @@
 //
 // k_conv_bf16_st: the 100-channel layers (3x3 and 2x2) on
 //   v_mfma_f32_16x16x32_bf16: a workgroup of 4 waves computes a 4-row x
-//   64-pixel output tile for all 112 (padded) output channels, the input halo
+//   32- or 64-pixel output tile for all 112 (padded) output channels, the input halo
 //   tile staged in LDS one channel half at a time, the weights streaming
 //   through a ring of chunk slots filled by direct global->LDS loads.
 //   Epilogue: + bias (the accumulators' start value), tanh, bf16, stored from
@@ -306,35 +306,46 @@ __global__ __launch_bounds__(256, MINW) void k_conv_bf16(const bf16* __restrict_
 // BF16 MFMA implicit GEMM for the 100-channel layers (13 channel groups, two
 // channel stages of the packed layout).
 //
-// A workgroup of 4 waves computes a 4-row x 64-pixel output tile for all 112
-// (padded) output channels; wave w owns output row w: four 16-pixel M-tiles x
-// seven 16-channel N-tiles of accumulators.  Per 32-deep reduction chunk a wave
-// reads 4 input + 7 weight fragments of 1 KB from LDS for 28 MFMAs (the
-// 32-pixel tile of k_conv_bf16 reads 2 + 7 for 14).  The (4+KH-1) x (64+KW-1)
-// input halo tile is staged one channel stage at a time (groups 0-6, then 7-12,
-// at a 112-byte pixel pitch, 44 KB), and the weights stream through a ring of
-// four 8 KB chunk slots filled by direct global->LDS loads, so two 76 KB
-// workgroups share a CU and no staging passes through registers.
+// A workgroup of 4 waves computes a 4-row x TW-pixel output tile (TW = 32 or 64)
+// for all 112 (padded) output channels; wave w owns output row w: TW / 16 M-tiles
+// of 16 pixels x seven 16-channel N-tiles of accumulators.  Per 32-deep reduction
+// chunk a wave reads TW / 16 input + 7 weight fragments of 1 KB from LDS for
+// 7 TW / 16 MFMAs.  The (4+KH-1) x (TW+KW-1) input halo tile is staged one channel
+// stage at a time (groups 0-6, then 7-12, at a 112-byte pixel pitch: 23 or 44 KB),
+// and the weights stream through a ring of four chunk slots filled by direct
+// global->LDS loads; no staging passes through registers.
+//
+// A 32-pixel tile takes 53 KB and 160 registers, so three workgroups share a CU
+// (two of 64 pixels, 76 KB); which is faster is a matter of how full the last
+// round of workgroups is (try_bf16_st).  Measured (us, TW = 64 / 32): 3x3 at
+// 1256 x 389 113 / 115 (4 rounds / 6), at 524 x 268 51 / 42 (2 / 2), at 64 x 64
+// 18 / 13 (1 / 1), 2x2 at 749 x 501 56 / 53 (3 / 4), at 325 x 245 21 / 19 (1 / 1),
+// at 627 x 191 23.7 / 25.5 (1 / 2).
 //
 // Ring protocol (chunk c in slot c % 4): the loads of chunk c are issued after
 // the barrier that ends iteration c-4 (all reads of chunk c-4's slot are done by
 // then); every wave waits for its loads of chunk c+2 (vmcnt: only chunk c+3's
 // two loads may be younger) before the barrier that ends iteration c, so chunk
 // c+2 is complete for every wave when iteration c+1 reads its fragments.
-template <int KH, int KW>
+template <int KH, int KW, int TW_>
 struct StCfg {
-  static constexpr int CG = 13, NT = 7, NP = 16 * NT, TW = 64, MT = TW / 16;
+  static constexpr int CG = 13, NT = 7, NP = 16 * NT, TW = TW_, MT = TW / 16;
   static constexpr int taps = KH * KW;
   static constexpr int PG = stage_ng(CG, 0);  // 16-byte groups per LDS pixel (the larger stage)
   static constexpr int NQ0 = stage_nq(CG, taps, 0), NQ = packed_chunks(CG, taps);
   static constexpr int AR = kTH + KH - 1, AC = TW + KW - 1;
   static constexpr int a_vec = AR * AC * PG;
   static constexpr int A_RND = (a_vec + 255) / 256;  // direct loads per wave per stage
-  static constexpr int a_bytes = A_RND * 256 * 16;   // the tile, padded to whole rounds
+  static constexpr bool kTight = TW < 64;  // three workgroups per CU: no byte to spare
+  // the tile, padded to whole rounds (tight: to whole waves)
+  static constexpr int a_bytes = kTight ? (a_vec + 63) / 64 * 1024 : A_RND * 256 * 16;
   static constexpr int chunk_vec = NP * RPB * 2 / 16;  // 448 vectors of 16 bytes
-  static constexpr int slot_bytes = 8192;              // two loads of 64 vectors per wave
+  // Two loads of 64 vectors per wave fill 8 KB; the last is padding, which (tight)
+  // all slots share behind the ring.
+  static constexpr int slot_bytes = kTight ? 7168 : 8192;
   static constexpr int NSLOT = 4;
-  static constexpr int zero_off = a_bytes + NSLOT * slot_bytes;  // 16 zero bytes (padding groups read them)
+  static constexpr int dump_off = NSLOT * slot_bytes;
+  static constexpr int zero_off = a_bytes + dump_off + (kTight ? 1024 : 0);  // 16 zero bytes (padding groups read them)
   static constexpr int lds_bytes = zero_off + 16;
   static constexpr int Cs = CG * 8;
   static_assert(chunk_vec <= slot_bytes / 16, "a chunk fits its slot");
@@ -362,11 +373,11 @@ __device__ __forceinline__ void tile_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int KH, int KW>
+template <int KH, int KW, int TW>
 __global__ __launch_bounds__(256, 2) void k_conv_bf16_st(const bf16* __restrict__ x, int Hin, int Win,
                                                         const bf16* __restrict__ wpk, const float* __restrict__ bias,
                                                         int K, int act, bf16* __restrict__ y, int Ho, int Wo) {
-  using Cfg = StCfg<KH, KW>;
+  using Cfg = StCfg<KH, KW, TW>;
   constexpr int Cs = Cfg::Cs, MT = Cfg::MT, NT = Cfg::NT, PG = Cfg::PG, AC = Cfg::AC;
   extern __shared__ __align__(16) unsigned char lds[];
   unsigned char* As = lds;
@@ -386,8 +397,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_bf16_st(const bf16* __restrict_
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int v = (2 * wave + i) * 64 + lane;
+        const bool dump = Cfg::kTight && 2 * wave + i == 7;
         load_lds16(wsrc + min(c * Cfg::chunk_vec + v, wvec_last),
-                   Bs + (c % Cfg::NSLOT) * Cfg::slot_bytes + (2 * wave + i) * 1024);
+                   Bs + (dump ? Cfg::dump_off : (c % Cfg::NSLOT) * Cfg::slot_bytes + (2 * wave + i) * 1024));
       }
     }
   };
@@ -402,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_bf16_st(const bf16* __restrict_
       const int r = v / (AC * PG), px = (v / PG) % AC, g = v % PG;
       const int hi = min(h0 + r, Hin - 1), wi = min(w0 + px, Win - 1);
       const bf16* src = x + (((long)hi * Win + wi) * Cs + min(cg0 + g, Cfg::CG - 1) * 8);
-      load_lds16(src, As + (i * 4 + wave) * 1024);
+      if (!Cfg::kTight || (i * 4 + wave) * 64 < Cfg::a_vec) load_lds16(src, As + (i * 4 + wave) * 1024);
     }
   };
 
@@ -789,16 +801,24 @@ template <int KH, int KW>
 static bool try_bf16_st(const ConvShape& s, const void* x, const void* wpk, const float* b, int act, void* y,
                         hipStream_t st) {
   if (s.KH != KH || s.KW != KW || feature_stride(s.C) != 104 || (s.K + 15) / 16 != 7) return false;
-  using Cfg = StCfg<KH, KW>;
-  const auto kern = k_conv_bf16_st<KH, KW>;
   const int Ho = s.H - KH + 1, Wo = s.W - KW + 1;
-  static bool configured = false;
-  if (!configured) {
+  auto launch = [&](auto tw) {
+    constexpr int TW = decltype(tw)::value;
+    using Cfg = StCfg<KH, KW, TW>;
+    const auto kern = k_conv_bf16_st<KH, KW, TW>;
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::lds_bytes);
-    configured = true;
-  }
-  kern<<<dim3(ceil_div(Wo, Cfg::TW), ceil_div(Ho, kTH)), 256, Cfg::lds_bytes, st>>>(
-      (const bf16*)x, s.H, s.W, (const bf16*)wpk, b, s.K, act, (bf16*)y, Ho, Wo);
+    kern<<<dim3(ceil_div(Wo, TW), ceil_div(Ho, kTH)), 256, Cfg::lds_bytes, st>>>(
+        (const bf16*)x, s.H, s.W, (const bf16*)wpk, b, s.K, act, (bf16*)y, Ho, Wo);
+  };
+  // The fewer rounds of resident workgroups, a round of 32-pixel tiles (three per
+  // CU) taking 0.7 of a round of 64-pixel tiles (two): 19 / 28 us in 3x3, 13 / 19 in
+  // 2x2.
+  const long rows = ceil_div(Ho, kTH), cus = cu_count();
+  const long narrow = ceil_div(rows * ceil_div(Wo, 32), 3 * cus), wide = ceil_div(rows * ceil_div(Wo, 64), 2 * cus);
+  if (7 * narrow < 10 * wide)
+    launch(std::integral_constant<int, 32>{});
+  else
+    launch(std::integral_constant<int, 64>{});
   return true;
 }
 
