@@ -9,7 +9,7 @@
 // feature rows are staged in LDS (f1 as the window of columns the band needs,
 // zero outside the image), each wave computes the 16 x (16*NTM) block
 // S[w][w'] of its 16 pixels against the window with MFMA (a banded GEMM over
-// the channels), parks it in LDS over the dead feature tiles, and the epilogue
+// the channels; float32 maps a stage of 32 channels at a time, see CorrSplit), parks it in LDS over the dead feature tiles, and the epilogue
 // gathers the band w' = w + o_k, applies -softmax over k and writes the
 // H x W x D volume with 16-byte stores, D contiguous floats per pixel.
 #include <algorithm>
@@ -18,20 +18,10 @@
 #include <vector>
 
 #include "common.hpp"
+#include "conv_split.hpp"
 #include "corr_bwd.hpp"
 
 namespace ccs {
-
-template <typename T>
-struct CorrTraits;
-template <>
-struct CorrTraits<bf16> {
-  static constexpr int kChunk = 32;  // channels per MFMA
-};
-template <>
-struct CorrTraits<float> {
-  static constexpr int kChunk = 4;
-};
 
 struct CorrArgs {
   const void* f0;
@@ -45,6 +35,28 @@ struct CorrArgs {
   int win;        // f1 window columns
   int sp;         // S row pitch (floats)
   int stats_off;  // byte offset of the softmax statistics in LDS
+};
+
+// float32 maps: the same product on the float16 matrix cores.  Features are split
+// into two float16 terms (split2) with one power-of-two scale per pixel and stage
+// of 32 channels; a stage's three products are summed from zero and taken into
+// the accumulators with both pixels' scales.  Only the stage is held in LDS (132
+// bytes per pixel and window column instead of 420 for the whole float32 row of
+// 100 channels), so two or three workgroups share a CU and their phases overlap;
+// the next stage's loads are in flight under the products.  Bound by the volume's
+// store and the softmax.  Measured (us, v_mfma_f32_16x16x4_f32 kernel with whole
+// pixels in LDS -> this): 320 x 240 D = 32 37 -> 27, 744 x 496 D = 64 229 -> 124,
+// 512 x 256 D = 128 97 -> 62, 1242 x 375 D = 128 344 -> 211, 1488 x 992 D = 256
+// 2807 -> 1366 (1.14 TB/s of volume), 96 x 64 D = 16 14 -> 13.
+template <int NTM>
+struct CorrSplit {
+  static constexpr int NW = NTM > 9 ? 4 : 8, TW = 16 * NW, WIN = 16 * (NW - 1) + 16 * NTM, NPX = TW + WIN;
+  static constexpr int SP = 16 * NTM + 3;  // as CorrArgs::sp
+  static constexpr int THREADS = 64 * NW, PER = (NPX * 4 + THREADS - 1) / THREADS;
+  static constexpr int plane = NPX * 64, scale_off = 2 * plane;
+  static constexpr int feat = scale_off + NPX * 4, sbytes = NW * 16 * SP * 4;
+  static constexpr int stats_off = ((feat > sbytes ? feat : sbytes) + 15) / 16 * 16;
+  static constexpr int lds_bytes = stats_off + NW * 16 * 4;
 };
 
 template <typename T, int NTM>
@@ -66,45 +78,37 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
 
   const T* f0 = reinterpret_cast<const T*>(a.f0) + (long)h * a.W * Cs;
   const T* f1 = reinterpret_cast<const T*>(a.f1) + (long)h * a.W * Cs;
-  const int wbase = w0 + a.o_lo;  // first f1 column of the window
-  // Both feature rows go to LDS in batches of 16-byte loads (one memory latency
-  // per batch); columns outside the image read as zero.
-  const int nthr = blockDim.x;
-  const int vpp = Cs * (int)sizeof(T) / 16;  // 16-byte vectors per pixel
-  auto fetch = [&](const T* row, int wi) -> const u32x4* {
-    return reinterpret_cast<const u32x4*>(row + (long)min(max(wi, 0), a.W - 1) * Cs);
-  };
-  auto put = [&](T* dst, int px, int g, const u32x4& val) {
-    if constexpr (sizeof(T) == 2) {
-      *reinterpret_cast<u32x4*>(dst + px * P + 8 * g) = val;
-    } else {  // odd float pitch: scalar stores
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[px * P + 4 * g + e] = __uint_as_float(val[e]);
-    }
-  };
-  batched_copy16<8>(
-      TW * vpp, tid, nthr,
-      [&](int v) {
-        const int px = v / vpp, g = v % vpp, wi = w0 + px;
-        const u32x4 val = fetch(f0, wi)[g];
-        return wi < a.W ? val : u32x4{0u, 0u, 0u, 0u};
-      },
-      [&](int v, const u32x4& val) { put(F0, v / vpp, v % vpp, val); });
-  batched_copy16<8>(
-      a.win * vpp, tid, nthr,
-      [&](int v) {
-        const int px = v / vpp, g = v % vpp, wi = wbase + px;
-        const u32x4 val = fetch(f1, wi)[g];
-        return (wi >= 0 && wi < a.W) ? val : u32x4{0u, 0u, 0u, 0u};
-      },
-      [&](int v, const u32x4& val) { put(F1, v / vpp, v % vpp, val); });
-  __syncthreads();
-
   f32x4 acc[NTM];
 #pragma unroll
   for (int t = 0; t < NTM; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int arow = 16 * wave + lrow;  // pixel of this lane's A row
   if constexpr (sizeof(T) == 2) {
+    const int wbase = w0 + a.o_lo;  // first f1 column of the window
+    // Both feature rows go to LDS in batches of 16-byte loads (one memory latency
+    // per batch); columns outside the image read as zero.
+    const int nthr = blockDim.x;
+    const int vpp = Cs * (int)sizeof(T) / 16;  // 16-byte vectors per pixel
+    auto fetch = [&](const T* row, int wi) -> const u32x4* {
+      return reinterpret_cast<const u32x4*>(row + (long)min(max(wi, 0), a.W - 1) * Cs);
+    };
+    auto put = [&](T* dst, int px, int g, const u32x4& val) { *reinterpret_cast<u32x4*>(dst + px * P + 8 * g) = val; };
+    batched_copy16<8>(
+        TW * vpp, tid, nthr,
+        [&](int v) {
+          const int px = v / vpp, g = v % vpp, wi = w0 + px;
+          const u32x4 val = fetch(f0, wi)[g];
+          return wi < a.W ? val : u32x4{0u, 0u, 0u, 0u};
+        },
+        [&](int v, const u32x4& val) { put(F0, v / vpp, v % vpp, val); });
+    batched_copy16<8>(
+        a.win * vpp, tid, nthr,
+        [&](int v) {
+          const int px = v / vpp, g = v % vpp, wi = wbase + px;
+          const u32x4 val = fetch(f1, wi)[g];
+          return (wi >= 0 && wi < a.W) ? val : u32x4{0u, 0u, 0u, 0u};
+        },
+        [&](int v, const u32x4& val) { put(F1, v / vpp, v % vpp, val); });
+    __syncthreads();
     const int cg = Cs / 8;
     for (int q = 0; q < (cg + 3) / 4; ++q) {
       const int g = 4 * q + lgrp;
@@ -118,13 +122,86 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
       }
     }
   } else {
-    for (int q = 0; q < Cs / 4; ++q) {
-      const int c = 4 * q + lgrp;
-      const float av = F0[arow * P + c];
+    using Cfg = CorrSplit<NTM>;
+    constexpr int NPX = Cfg::NPX, PER = Cfg::PER;
+    const int cg = Cs / 8;
+    auto swz = [](int px, int g) { return (g ^ ((px >> 1) & 3)) * 16; };
+
+    // Unit (pixel, group of eight channels) v of a stage: pixels TW .. are the
+    // window's columns.  What lies outside the image or past the channels is zero,
+    // set when the unit is stored.
+    f32x4 r[PER][2];
+    auto column = [&](int px) { return px < TW ? w0 + px : w0 + a.o_lo + px - TW; };
+    auto load = [&](int st) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int v = min(tid + Cfg::THREADS * i, NPX * 4 - 1), px = v >> 2, g = min(4 * st + (v & 3), cg - 1);
+        const float* row = px < TW ? f0 : f1;
+        const f32x4* src = reinterpret_cast<const f32x4*>(row + (long)min(max(column(px), 0), a.W - 1) * Cs + 8 * g);
+        r[i][0] = src[0];
+        r[i][1] = src[1];
+      }
+    };
+    auto store = [&](int st) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int v = tid + Cfg::THREADS * i, px = v >> 2, g = v & 3, col = column(px);
+        const bool ok = 4 * st + g < cg && col >= 0 && col < a.W;
+        float f[8];
+        unsigned mx = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          f[e] = ok ? r[i][e >> 2][e & 3] : 0.f;
+          mx = max(mx, __float_as_uint(f[e]) & 0x7fffffffu);
+        }
+        const bool finite = !__any(mx >= 0x7f800000u);
+        if (!finite) {
+          mx = 0;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) mx = max(mx, finite_bits(f[e]));
+        }
+        mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0xb1, 0xf, 0xf, true));
+        mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0x4e, 0xf, 0xf, true));
+        const int eb = split_exp(mx);
+        f16x8 p[2];
+        if (finite)
+          split2<true>(f, split_scale(eb), p[0], p[1]);
+        else
+          split2<false>(f, split_scale(eb), p[0], p[1]);
+        if (v < NPX * 4) {
+          const int off = px * 64 + swz(px, g);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) *reinterpret_cast<f16x8*>(lds + k * Cfg::plane + off) = p[k];
+          if (g == 0)  // 2^-28 goes to the first map's pixels
+            *reinterpret_cast<float*>(lds + Cfg::scale_off + px * 4) =
+                px < TW ? split_unscale(eb) : __uint_as_float((unsigned)eb << 23);
+        }
+      }
+    };
+
+    const int stages = (cg + 3) / 4;
+    load(0);
+    for (int st = 0; st < stages; ++st) {
+      if (st > 0) __syncthreads();  // the previous stage is read
+      store(st);
+      __syncthreads();
+      if (st + 1 < stages) load(st + 1);
+      const float* scale = reinterpret_cast<const float*>(lds + Cfg::scale_off);
+      auto frag = [&](int px, int k) {
+        return *reinterpret_cast<const f16x8*>(lds + k * Cfg::plane + px * 64 + swz(px, lgrp));
+      };
+      const f16x8 ah = frag(arow, 0), al = frag(arow, 1);
+      const f32x4 s0 = *reinterpret_cast<const f32x4*>(scale + 16 * wave + 4 * lgrp);
 #pragma unroll
       for (int t = 0; t < NTM; ++t) {
-        const int col = 16 * wave + 16 * t + lrow;
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, F1[col * P + c], acc[t], 0, 0, 0);
+        const int px = TW + 16 * wave + 16 * t + lrow;
+        const f16x8 bh = frag(px, 0), bl = frag(px, 1);
+        const float s1 = scale[px];
+        f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, c, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][e] = fmaf(c[e], s0[e] * s1, acc[t][e]);
       }
     }
   }
@@ -426,23 +503,34 @@ __global__ void k_sum_f64_corr(const double* __restrict__ in, int n, double* __r
 }
 
 // LDS bytes of one workgroup: the feature tiles, later overlaid by S, then the statistics.
-static size_t corr_lds_bytes(CorrArgs& a, int NW, size_t esz) {
-  const size_t feat = (size_t)(16 * NW + a.win) * a.pitch * esz;
+static size_t corr_lds_bytes(CorrArgs& a, int NW) {
+  const size_t feat = (size_t)(16 * NW + a.win) * a.pitch * sizeof(bf16);
   const size_t sbytes = (size_t)NW * 16 * a.sp * 4;
   a.stats_off = (int)((feat > sbytes ? feat : sbytes) + 15) / 16 * 16;
   return (size_t)a.stats_off + (size_t)NW * 16 * 4;
 }
 
-template <typename T, int NTM>
+template <int NTM>
 static int launch_volume(CorrArgs a, int NW, hipStream_t st) {
-  const size_t bytes = corr_lds_bytes(a, NW, sizeof(T));
+  const size_t bytes = corr_lds_bytes(a, NW);
   static bool configured = false;
   if (!configured) {
-    CCS_HIP(hipFuncSetAttribute((const void*)k_corr_volume<T, NTM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    CCS_HIP(hipFuncSetAttribute((const void*)k_corr_volume<bf16, NTM>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 160 * 1024));
     configured = true;
   }
-  k_corr_volume<T, NTM><<<dim3(ceil_div(a.W, 16 * NW), a.H), 64 * NW, bytes, st>>>(a);
+  k_corr_volume<bf16, NTM><<<dim3(ceil_div(a.W, 16 * NW), a.H), 64 * NW, bytes, st>>>(a);
+  CCS_LAUNCH_CHECK();
+  return CCS_OK;
+}
+
+template <int NTM>
+static int launch_split(CorrArgs a, hipStream_t st) {
+  using Cfg = CorrSplit<NTM>;
+  a.stats_off = Cfg::stats_off;
+  CCS_HIP(hipFuncSetAttribute((const void*)k_corr_volume<float, NTM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              Cfg::lds_bytes));
+  k_corr_volume<float, NTM><<<dim3(ceil_div(a.W, Cfg::TW), a.H), Cfg::THREADS, Cfg::lds_bytes, st>>>(a);
   CCS_LAUNCH_CHECK();
   return CCS_OK;
 }
@@ -477,33 +565,36 @@ extern "C" int ccs_correlation_volume(ccs_handle_t h, const void* f0, const void
   // (mod 32) words apart and the softmax pass's four-word groups of eight rows
   // fall on distinct banks (with a multiple of 16 the rows met every 2).
   a.sp = 16 * ntm + 3;
-  const size_t esz = precision == CCS_BF16 ? 2 : 4;
-  a.pitch = precision == CCS_BF16 ? a.Cs : a.Cs + 1;
+  hipStream_t st = h->stream;
+  if (precision == CCS_FP32) {
+    // The limit on channels and span: one wave's tile as whole float32 pixels in LDS.
+    const size_t tile = (size_t)(16 + 16 * ntm) * (a.Cs + 1) * sizeof(float);
+    CCS_CHECK((tile + 15) / 16 * 16 + 64 <= 160 * 1024, CCS_ERR_UNSUPPORTED,
+              "ccs_correlation_volume: tile does not fit in LDS");
+    switch (ntm) {
+      case 3: return launch_split<3>(a, st);
+      case 5: return launch_split<5>(a, st);
+      case 9: return launch_split<9>(a, st);
+      default: return launch_split<17>(a, st);
+    }
+  }
+  a.pitch = a.Cs;
   // Waves per workgroup: the most resident waves per CU (160 KB of LDS), ties
   // to the wider tile (its f1 window is shared by more pixels).
   int NW = 0, best = 0;
   for (int nw = 8; nw >= 1; nw >>= 1) {
     a.win = 16 * (nw - 1) + 16 * ntm;
-    const size_t bytes = corr_lds_bytes(a, nw, esz);
+    const size_t bytes = corr_lds_bytes(a, nw);
     const int resident = nw * (int)((160 * 1024) / bytes);
     if (resident > best) best = resident, NW = nw;
   }
   CCS_CHECK(NW >= 1, CCS_ERR_UNSUPPORTED, "ccs_correlation_volume: tile does not fit in LDS");
   a.win = 16 * (NW - 1) + 16 * ntm;
-  hipStream_t st = h->stream;
-  if (precision == CCS_BF16) {
-    switch (ntm) {
-      case 3: return launch_volume<bf16, 3>(a, NW, st);
-      case 5: return launch_volume<bf16, 5>(a, NW, st);
-      case 9: return launch_volume<bf16, 9>(a, NW, st);
-      default: return launch_volume<bf16, 17>(a, NW, st);
-    }
-  }
   switch (ntm) {
-    case 3: return launch_volume<float, 3>(a, NW, st);
-    case 5: return launch_volume<float, 5>(a, NW, st);
-    case 9: return launch_volume<float, 9>(a, NW, st);
-    default: return launch_volume<float, 17>(a, NW, st);
+    case 3: return launch_volume<3>(a, NW, st);
+    case 5: return launch_volume<5>(a, NW, st);
+    case 9: return launch_volume<9>(a, NW, st);
+    default: return launch_volume<17>(a, NW, st);
   }
 }
 
