@@ -24,7 +24,8 @@
 // passes and the cost volume only in its forward pass (4 volume passes per
 // sweep instead of 3 for rows and 5 for columns).
 //
-// GPU mapping: one wavefront per chain, label s = lane * LPL + j held in VGPRs,
+// GPU mapping: one wavefront per chain (k_chain; with few chains two more waves
+// move its data, k_line), label s = lane * LPL + j held in VGPRs,
 // DPP wave_shr/wave_shl for the label neighbours and a DPP tree for the minimum
 // over labels.  The volume streams through HBM once per pass (node i is D
 // contiguous floats), backward messages go to a scratch volume (column sweeps
@@ -1323,10 +1324,10 @@ __global__ __launch_bounds__(MODE != kColsMinorant && SEG ? 256 : 64) void k_cha
 // workgroup of eight waves, two of them idle: waves go to the four SIMDs in turn,
 // so that each chain wave keeps a SIMD to itself.
 //
-// Measured, one sweep (us, k_chain -> this): rows 320 x 240 x 32 72 -> 54,
-// 744 x 496 x 64 141 -> 120, 1242 x 128 x 128 261 -> 217 (88 of them backward),
-// 1242 x 375 x 128 270 -> 257 (streaming the costs; 954 MB, 3.7 TB/s); columns
-// 320 x 240 x 32 73 -> 43, 744 x 496 x 64 126 -> 100.
+// Measured, one sweep (us, k_chain -> this): rows 320 x 240 x 32 72 -> 50,
+// 744 x 496 x 64 141 -> 115, 1242 x 128 x 128 261 -> 212 (88 of them backward),
+// 1242 x 375 x 128 270 -> 262 (streaming the costs; 954 MB, 3.6 TB/s); columns
+// 320 x 240 x 32 73 -> 40, 744 x 496 x 64 126 -> 95.
 constexpr int kLineK = 8;
 constexpr int kLineRing = 3 * 2 + 2;  // segments of node vectors in the two rings
 enum LineRole { kChain = 0, kMessages = 1, kOut = 2, kIdle = 3 };
