@@ -1,7 +1,8 @@
-// Weight gradient of the 100-channel layers on the bf16 matrix cores:
+// Weight gradient of the 100-channel layers on the 16-bit matrix cores:
 //   dW[tap][k][c] = sum over output pixels p of dz[p][k] x[p + tap][c]
-// for float32 maps (both operands split exactly into three bfloat16 terms, six
-// products, as conv_split.hip) and bfloat16 maps.
+// for bfloat16 maps and float32 maps (two float16 terms per operand with a scale
+// per channel and segment, three products summed from zero per segment, as
+// conv_split.hip).
 //
 // k_dw_split: a workgroup takes one tap row i (its KW taps) and a chunk of
 // SEG-pixel segments of output rows; each of its seven waves owns 16 channels of
@@ -14,13 +15,14 @@
 // dword (j = 2), the fifth dword read beside them.  (A copy of the row per tap,
 // stored two bytes at a time, took 64 LDS writes per thread and segment.)
 //
-// Bound by the steps' LDS reads and, with float32 maps, by splitting them (1.1 us
-// of 4.4 per segment).  Measured with the reduction and k_dz_pad (the kernels it
-// replaced -> with the zeros past a row's end selected beside the loads, which
-// waited for each segment's reads -> now): bf16 3x3 at 524 x 268 190 -> 112 ->
-// 94 us, at 1488 x 992 1490 -> 949 -> 708 us; float32 3x3 at 524 x 268 473 -> 328
-// -> 301 us.  Two input halves per chunk on four-wave workgroups, two or three
-// per CU, measured the same as one (110, 990, 357 us): they read dz twice as often.
+// Bound by the steps' LDS reads and, with float32 maps, by splitting them.
+// Measured with the reduction and k_dz_pad (the kernels it replaced -> with the
+// zeros past a row's end selected beside the loads, which waited for each segment's
+// reads -> now): bf16 3x3 at 524 x 268 190 -> 112 -> 94 us, at 1488 x 992
+// 1490 -> 949 -> 708 us; float32 3x3 at 524 x 268 473 -> 328 -> 263 us (301 with
+// three bfloat16 terms and six products).  Two input halves per chunk on four-wave
+// workgroups, two or three per CU, measured the same as one (110, 990, 357 us): they
+// read dz twice as often.
 //
 // Blocks b and b + 8 share an XCD: the tap rows of a chunk, which read the same
 // dz and overlapping inputs, are consecutive there.  The block's sums go to
@@ -35,18 +37,21 @@ namespace ccs {
 template <typename T>
 struct DwCfg {
   static constexpr bool kF32 = sizeof(T) == 4;
-  static constexpr int PLANES = kF32 ? 3 : 1;
+  static constexpr int PLANES = kF32 ? 2 : 1;
   static constexpr int SEG = kF32 ? 32 : 64;  // output pixels per segment
   static constexpr int NT = 7, CP = 16 * NT, THREADS = 64 * NT;  // channel tiles, one wave each for dz
   static constexpr int VE = 16 / (int)sizeof(T);                 // channels per 16-byte vector
   // Staging blocks of 64 units (four pixels of a 16-byte channel group): QL
-  // pixel quads times GL groups; four blocks of dz, four of the input row and
-  // one of the input row's last quad, two per wave at most.
-  static constexpr int QL = SEG / 4, GL = 64 / QL, NU = 2;
-  static_assert(4 * GL >= CP / VE && 9 <= NU * NT, "the blocks cover the channels");
+  // pixel quads times GL groups; four blocks of dz and four of the input row.  The
+  // pixels past the segment that the shifted taps read: bfloat16 a ninth block
+  // with the input row's last quad, float32 two more pixels in its blocks (their
+  // channel's scale must cover them).  Two blocks per wave at most.
+  static constexpr int QL = SEG / 4, GL = 64 / QL, NU = 2, BLOCKS = kF32 ? 8 : 9;
+  static_assert(4 * GL >= CP / VE && BLOCKS <= NU * NT, "the blocks cover the channels");
   static constexpr int PITCH = SEG + 8;         // pixels; an odd multiple of 16 bytes
   static constexpr int plane = CP * PITCH * 2;  // bytes
-  static constexpr int buffer = 2 * PLANES * plane;
+  static constexpr int scales = 2 * PLANES * plane;  // float32: a scale per channel of dz, then of the input
+  static constexpr int buffer = scales + (kF32 ? 2 * CP * 4 : 0);
   static constexpr int lds_bytes = 2 * buffer;
 };
 
@@ -75,6 +80,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   // consecutive quads of one group, so a pixel is read 64 (128) bytes at a time
   // and the stores of a channel are contiguous.
   u32x4 reg[Cfg::NU][4];
+  u32x4 ext[Cfg::NU][2];  // float32: input pixels SEG, SEG + 1
   struct Unit {
     bool z, ok;
     int q, g;
@@ -98,7 +104,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
 #pragma unroll
     for (int n = 0; n < Cfg::NU; ++n) {
       const int b = wave + NT * n;
-      if (b > 8) break;
+      if (b >= Cfg::BLOCKS) break;
       const Unit u = unit(b);
       const T* row = u.z ? dz + ((long)ho * zpitch + wo0) * Csk : x + ((long)(ho + ti) * Win + wo0) * Csx;
       const int cs = u.z ? Csk : Csx, left = (u.z ? Wo : Win) - wo0;  // pixels of the row from wo0 on
@@ -107,6 +113,13 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
         const int px = 4 * u.q + i;
         const bool ok = u.ok && px < left;
         reg[n][i] = *reinterpret_cast<const u32x4*>(row + (ok ? px * cs + u.g * VE : 0));
+      }
+      if constexpr (Cfg::kF32) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const bool ok = !u.z && u.ok && SEG + i < left;
+          ext[n][i] = *reinterpret_cast<const u32x4*>(row + (ok ? (SEG + i) * cs + u.g * VE : 0));
+        }
       }
     }
     if (++lseg == segs_per_row) {
@@ -118,30 +131,76 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
 #pragma unroll
     for (int n = 0; n < Cfg::NU; ++n) {
       const int b = wave + NT * n;
-      if (b > 8) break;
+      if (b >= Cfg::BLOCKS) break;
       const Unit u = unit(b);
-      if (!u.ok) continue;
+      if (!Cfg::kF32 && !u.ok) continue;
       const int left = (u.z ? Wo : Win) - wo_loaded;
       if (left < SEG + 4) {  // (uniform) the row may end in this segment
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (4 * u.q + i >= left) reg[n][i] = u32x4{0u, 0u, 0u, 0u};
+        if constexpr (Cfg::kF32) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            if (SEG + i >= left) ext[n][i] = u32x4{0u, 0u, 0u, 0u};
+        }
       }
       unsigned char* d =
           lds + buf * Cfg::buffer + (u.z ? 0 : PLANES * Cfg::plane) + (u.g * VE * PITCH + 4 * u.q) * 2;
       if constexpr (Cfg::kF32) {
+        // Four pixels and the two past the segment of four channels; the eight
+        // lanes of a group agree on each channel's scale.
+        unsigned mx[4], all = 0;
+        auto bits = [&](int e, int i) { return i < 4 ? reg[n][i][e] : ext[n][i - 4][e]; };
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float f[4];
-          bf16 p[3][4];
+          mx[e] = 0;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(reg[n][i][e]);
-          split3(f, p[0], p[1], p[2]);
-          typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-            *reinterpret_cast<bf16x4*>(d + k * Cfg::plane + e * PITCH * 2) = bf16x4{p[k][0], p[k][1], p[k][2], p[k][3]};
+          for (int i = 0; i < 6; ++i)
+            if (i < 4 || !u.z) mx[e] = max(mx[e], bits(e, i) & 0x7fffffffu);
+          all = max(all, mx[e]);
         }
+        const bool finite = !__any(all >= 0x7f800000u);
+        f32x4 unscale;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (!finite) {
+            mx[e] = 0;
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+              if (i < 4 || !u.z) mx[e] = max(mx[e], finite_bits(__uint_as_float(bits(e, i))));
+          }
+          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0xb1, 0xf, 0xf, true));
+          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x4e, 0xf, 0xf, true));
+          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x141, 0xf, 0xf, true));  // row_half_mirror
+          const int eb = split_exp(mx[e]);
+          const float sc = split_scale(eb);
+          unscale[e] = u.z ? split_unscale(eb) : __uint_as_float((unsigned)eb << 23);
+          typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+          typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+          f16x4 hi, lo;
+          f16x2 hx, lx;
+#pragma unroll
+          for (int i = 0; i < 6; ++i) {
+            if (i >= 4 && u.z) break;
+            const float f = __uint_as_float(bits(e, i));
+            const bool fin = finite || (__float_as_uint(f) & 0x7fffffffu) < 0x7f800000u;
+            const float v = fin ? f * sc : 0.f;
+            const _Float16 h = (_Float16)v, l = (_Float16)(fin ? v - (float)h : f);
+            if (i < 4) hi[i] = h, lo[i] = l;
+            else hx[i - 4] = h, lx[i - 4] = l;
+          }
+          if (u.ok) {
+            *reinterpret_cast<f16x4*>(d + e * PITCH * 2) = hi;
+            *reinterpret_cast<f16x4*>(d + Cfg::plane + e * PITCH * 2) = lo;
+            if (!u.z && u.q == Cfg::QL - 1) {  // (the next quad's first half)
+              *reinterpret_cast<f16x2*>(d + (e * PITCH + 4) * 2) = hx;
+              *reinterpret_cast<f16x2*>(d + Cfg::plane + (e * PITCH + 4) * 2) = lx;
+            }
+          }
+        }
+        if (u.ok && u.q == 0)
+          *reinterpret_cast<f32x4*>(lds + buf * Cfg::buffer + Cfg::scales + ((u.z ? 0 : CP) + u.g * VE) * 4) = unscale;
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -162,6 +221,9 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   auto multiply = [&](int buf) {
     const unsigned char* zb = lds + buf * Cfg::buffer;
     const unsigned char* xb = zb + PLANES * Cfg::plane;
+    const float* scale = reinterpret_cast<const float*>(zb + Cfg::scales);  // (float32)
+    f32x4 sz;
+    if constexpr (Cfg::kF32) sz = *reinterpret_cast<const f32x4*>(scale + k0 + 4 * lgrp);
 #pragma unroll
     for (int st = 0; st < SEG / 32; ++st) {
       const int off = (32 * st + 8 * lgrp) * 2;
@@ -172,7 +234,9 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       // Fragments of channel tile t: five dwords, read one tile ahead.
       u32x4 d[PLANES];
       unsigned d4[PLANES];
+      float sx = 0.f;
       auto read_x = [&](int t) {
+        if constexpr (Cfg::kF32) sx = scale[CP + 16 * t + lrow];
 #pragma unroll
         for (int k = 0; k < PLANES; ++k) {
           const unsigned char* src = xb + k * Cfg::plane + (16 * t + lrow) * PITCH * 2 + off;
@@ -197,6 +261,8 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
                             __builtin_amdgcn_alignbit(e[3], e[2], 16), __builtin_amdgcn_alignbit(d4[k], e[3], 16)});
           if constexpr (KW == 3) b[k][2] = __builtin_bit_cast(bf16x8, u32x4{e[1], e[2], e[3], d4[k]});
         }
+        f32x4 both;  // the scales of this lane's four sums
+        if constexpr (Cfg::kF32) both = sz * sx;
         if (t + 1 < NT) read_x(t + 1);
         __builtin_amdgcn_sched_barrier(0);
         f32x4 c[KW];
@@ -204,20 +270,27 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
         for (int j = 0; j < KW; ++j) c[j] = Cfg::kF32 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j][t];
         auto mm = [&](int ka, int kb) {
 #pragma unroll
-          for (int j = 0; j < KW; ++j) c[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ka], b[kb][j], c[j], 0, 0, 0);
+          for (int j = 0; j < KW; ++j) {
+            if constexpr (Cfg::kF32)
+              c[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[ka]),
+                                                           __builtin_bit_cast(f16x8, b[kb][j]), c[j], 0, 0, 0);
+            else
+              c[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ka], b[kb][j], c[j], 0, 0, 0);
+          }
         };
         if constexpr (Cfg::kF32) {
-          mm(0, 2);
-          mm(2, 0);
-          mm(1, 1);
-          mm(0, 1);
-          mm(1, 0);
+          mm(PLANES - 1, 0);
+          mm(0, PLANES - 1);
         }
         mm(0, 0);
 #pragma unroll
         for (int j = 0; j < KW; ++j) {
-          if constexpr (Cfg::kF32) acc[j][t] += c[j];
-          else acc[j][t] = c[j];
+          if constexpr (Cfg::kF32) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[j][t][e] = fmaf(c[j][e], both[e], acc[j][t][e]);
+          } else {
+            acc[j][t] = c[j];
+          }
         }
       }
     }
@@ -233,7 +306,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   // Segment s is multiplied from buffer (s - s0) % 2 while the next one's
   // registers go into the other (whose readers finished before the barrier).
   // Waves w and w + 4 share a SIMD: with bf16 maps one stages while the other
-  // multiplies (float32 maps would spill).
+  // multiplies (float32 maps would spill: 477 us).
   for (long s = s0; s < s1; ++s) {
     const int buf = (int)((s - s0) & 1);
     auto stage = [&]() {

@@ -1,4 +1,4 @@
-// Weight gradient on the bf16 matrix cores (conv_grad.hip).
+// Weight gradient on the 16-bit matrix cores (conv_grad.hip).
 #pragma once
 
 #include "common.hpp"

@@ -2,7 +2,8 @@
 tiles and padding, against float64.
 
 dz is formed and rounded in the maps' type, and the reference starts from that
-dz.  Products are exact (float32: but for 2^-26 of each).  A chunk sums n steps
+dz.  Products are exact (float32: but for 2^-22 of each, four times a float16
+pair's 2^-24, inside the 8 units below).  A chunk sums n steps
 of 32 pixels, at most six roundings each at the size of its partial sums and
 one more in the running sum, then at most 128 chunks are added:
 |error| <= (8 + n + 128) 2^-24 sum |dz x| for n = ceil(pixels of a chunk / 32).
