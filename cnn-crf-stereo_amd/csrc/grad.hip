@@ -82,10 +82,10 @@ __global__ __launch_bounds__(256) void k_dz_pad(const T* __restrict__ y, const T
   }
 }
 
-// out[c] = sum of the n partials part[c][0..n) (one block per c, a fixed tree).
-__global__ void k_reduce_cols(const float* __restrict__ part, int n, float* __restrict__ out) {
+// out[c] = sum of the n partials part[c][0..n) (one block of 256 per c, a fixed tree).
+__device__ __forceinline__ void reduce_col(const float* __restrict__ part, int n, int c, float* __restrict__ out) {
   __shared__ float sh[256];
-  const float* row = part + (long)blockIdx.x * n;
+  const float* row = part + (long)c * n;
   float s = 0.f;
   for (int i = threadIdx.x; i < n; i += 256) s += row[i];
   sh[threadIdx.x] = s;
@@ -94,7 +94,10 @@ __global__ void k_reduce_cols(const float* __restrict__ part, int n, float* __re
     if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+  if (threadIdx.x == 0) out[c] = sh[0];
+}
+__global__ __launch_bounds__(256) void k_reduce_cols(const float* __restrict__ part, int n, float* __restrict__ out) {
+  reduce_col(part, n, blockIdx.x, out);
 }
 
 __global__ void k_reduce_rows(const float* __restrict__ part, int nb, int n, float* __restrict__ out) {
@@ -224,8 +227,15 @@ __global__ __launch_bounds__(64 * KT, 4) void k_dw_mfma(const TX* __restrict__ x
 // a block takes 64 outputs (consecutive c), four threads each, which sum a
 // quarter of the chunks and are added in order.  (One thread per output left
 // 80 strided loads in a row: 24 us for 80 chunks of a 3x3 layer, 9.5 us now.)
+// Blocks past the first nw sum the bias gradient's partials, one channel each (a
+// launch of their own took 5 us).
 __global__ __launch_bounds__(256) void k_dw_reduce(const float* __restrict__ part, int nch, int taps, int KP, int CP,
-                                                   int K, int C, int KH, int KW, float* __restrict__ dw) {
+                                                   int K, int C, int KH, int KW, float* __restrict__ dw, int nw,
+                                                   const float* __restrict__ bpart, int nbz, float* __restrict__ db) {
+  if ((int)blockIdx.x >= nw) {
+    reduce_col(bpart, nbz, blockIdx.x - nw, db);
+    return;
+  }
   const long idx = (long)blockIdx.x * 64 + (threadIdx.x & 63);
   const int quarter = threadIdx.x >> 6;
   const bool in = idx < (long)K * C * taps;
@@ -367,31 +377,33 @@ int conv_backward(ccs_handle_t h, const TX* x, const T* y, int H, int W, int C, 
   const long Pp = (long)Hp * Wp;
   const int dz_chunk = 64;  // padded pixels per block of k_dz_pad
   const int nbz = (int)((Pp + dz_chunk - 1) / dz_chunk);
-  const size_t part_n =
-      std::max((size_t)nbz * Csk, mfma ? (size_t)nch * taps * 256 * KT * CT : (size_t)nb * wcount);
+  const size_t part_n = mfma ? (size_t)nch * taps * 256 * KT * CT : (size_t)nb * wcount;
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-  const size_t need = al(sizeof(T) * Pp * Csk) + al(sizeof(float) * part_n) + sizeof(float) * wcount;
+  const size_t bpart_b = al(sizeof(float) * nbz * Csk);
+  const size_t need = al(sizeof(T) * Pp * Csk) + bpart_b + al(sizeof(float) * part_n) + sizeof(float) * wcount;
   int rc = h->misc2.reserve(need, h->stream);
   if (rc) return rc;
   T* zpad = (T*)h->misc2.ptr;
-  float* part = (float*)((char*)zpad + al(sizeof(T) * Pp * Csk));
+  float* bpart = (float*)((char*)zpad + al(sizeof(T) * Pp * Csk));
+  float* part = (float*)((char*)bpart + bpart_b);
   float* wt = (float*)((char*)part + al(sizeof(float) * part_n));
   const T* z = zpad + ((long)py * Wp + px) * Csk;  // output pixel 0, rows Wp pixels apart
 
   constexpr int V = 16 / (int)sizeof(T);
   if (((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0)
-    k_dz_pad<T, V><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, part);
+    k_dz_pad<T, V><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, bpart);
   else
-    k_dz_pad<T, 1><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, part);
-  if (db) k_reduce_cols<<<K, 256, 0, h->stream>>>(part, nbz, db);
+    k_dz_pad<T, 1><<<nbz, 256, 0, h->stream>>>(y, dy, Ho, Wo, Csk, K, act, py, px, dz_chunk, zpad, bpart);
   if (mfma) {
     if (split)
       dw_split({x, z, part, W, Csx, Wp, Ho, Wo, Csk, nch, segs_row, nseg, spc}, precision, KH, KW, h->stream);
     else
       dw_mfma<TX, T>(KT, CT, x, W, Csx, z, Wp, Wo, Csk, KW, taps, segs_row, nseg, spc, nch, part, h->stream);
-    k_dw_reduce<<<ceil_div((long)wcount, 64), 256, 0, h->stream>>>(part, nch, taps, 16 * KT, 16 * CT, K, C, KH, KW,
-                                                                 dw);
+    const int nw = (int)ceil_div((long)wcount, 64);
+    k_dw_reduce<<<nw + (db ? K : 0), 256, 0, h->stream>>>(part, nch, taps, 16 * KT, 16 * CT, K, C, KH, KW, dw, nw, bpart,
+                                                          nbz, db);
   } else {
+    if (db) k_reduce_cols<<<K, 256, 0, h->stream>>>(bpart, nbz, db);
     dim3 grid(ceil_div(K, 16), ceil_div(C, 16) * KH * KW, nb);
     k_dw_partial<TX, T><<<grid, 256, 0, h->stream>>>(x, W, Csx, z, Wp, Ho, Wo, Csk, K, C, KH, KW, chunk, part);
     k_reduce_rows<<<ceil_div((long)wcount, 256), 256, 0, h->stream>>>(part, nb, (int)wcount, dw);
