@@ -86,7 +86,7 @@ __host__ __device__ inline void split_step(int q, int lgrp, int* tap, int* c0) {
 // (lrow, lgrp) holding output channel 16 t + lrow; then the row scales.  All
 // weights of a row are divided by its scale.  Block (t, y) packs a share of tile
 // t's steps; its 16 groups of 16 lanes each look at one row first.
-constexpr int kPackShares = 8;
+constexpr int kPackShares = 16;
 template <class Cfg>
 __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w, int K, int C, int adj,
                                                     unsigned char* __restrict__ out) {
@@ -99,8 +99,10 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
   {
     const int n = 16 * t + (tid >> 4);
     unsigned mx = 0;
-    if (n < K)
+    if (n < K) {  // (eight loads in flight)
+#pragma unroll 8
       for (int i = tid & 15; i < C * Cfg::taps; i += 16) mx = max(mx, finite_bits(at(n, i / Cfg::taps, i % Cfg::taps)));
+    }
     for (int o = 1; o < 16; o <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 16));
     if ((tid & 15) == 0) {
       exps[tid >> 4] = split_exp(mx);
