@@ -205,6 +205,43 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
       }
     }
   }
+  // -softmax over the band, in the accumulators where the disparities are
+  // consecutive columns: lane (lrow, lgrp) holds columns 16 t + lrow of pixels
+  // 4 lgrp + e, and a pixel's band is the D columns from its own on.  (Through LDS
+  // every entry is read twice and written once more.)  It works on whole column
+  // tiles, so it pays for wide bands that nearly fill theirs (us, through LDS / here,
+  // bf16): 1242 x 375 D = 128 129 / 124, 1488 x 992 D = 256 1040 / 883, but D = 64 (80
+  // columns) 69 / 70, D = 70 (144) 117 / 124, D = 24 67 / 71.
+  const int D = a.D;
+  const bool neg_softmax = a.epilogue == CCS_EPILOGUE_NEG_SOFTMAX;
+  const bool in_place = neg_softmax && (a.ostep == 1 || a.ostep == -1) && NTM >= 9 && D + 32 >= 16 * NTM;
+  if (in_place) {
+    auto row16 = [](float x, auto op) {  // over the 16 lanes of a row
+      x = op(x, dpp_rot<0xb1>(x));
+      x = op(x, dpp_rot<0x4e>(x));
+      x = op(x, dpp_rot<0x124>(x));
+      return op(x, dpp_rot<0x128>(x));
+    };
+    const int d0 = lrow - 4 * lgrp;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NTM; ++t)
+        if ((unsigned)(d0 + 16 * t - e) < (unsigned)D) mx = fmaxf(mx, acc[t][e]);
+      mx = row16(mx, [](float x, float y) { return fmaxf(x, y); });
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < NTM; ++t) {
+        acc[t][e] = __expf(acc[t][e] - mx);
+        if ((unsigned)(d0 + 16 * t - e) < (unsigned)D) sum += acc[t][e];
+      }
+      sum = row16(sum, [](float x, float y) { return x + y; });
+      const float sc = -1.f / sum;
+#pragma unroll
+      for (int t = 0; t < NTM; ++t) acc[t][e] *= sc;
+    }
+  }
   __syncthreads();  // the feature tiles are dead: S overwrites them
   // S_w[r][j] = f0[pixel 16*wave + r] . f1[window column 16*wave + j]
 #pragma unroll
@@ -214,10 +251,9 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
   __syncthreads();
 
   // Band entry of pixel r, disparity k: S_w[r * sp + r + o_k - o_lo] = band(r)[k * ostep].
-  const int D = a.D;
-  const bool neg_softmax = a.epilogue == CCS_EPILOGUE_NEG_SOFTMAX;
   auto band = [&](int r) { return S_w + r * a.sp + r + a.o0 - a.o_lo; };
-  if (neg_softmax) {
+  const bool scaled = neg_softmax && !in_place;  // by stats, when stored
+  if (scaled) {
     // 4 lanes per pixel: max, then exp(s - max) written back in place, then 1 / sum.
     const int r = lane >> 2, s4 = lane & 3;
     float* br = band(r);
@@ -247,7 +283,7 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
       const int r = r0 + rr;
       if (r < npx) {
         const float* br = band(r);
-        const float sc = neg_softmax ? stats[wave * 16 + r] : 1.f;
+        const float sc = scaled ? stats[wave * 16 + r] : 1.f;
         float4 v;
         v.x = br[k * a.ostep] * sc;
         v.y = br[(k + 1) * a.ostep] * sc;
@@ -259,7 +295,7 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
   } else {
     for (int f = lane; f < npx * D; f += 64) {
       const int r = f / D, k = f % D;
-      outp[f] = band(r)[k * a.ostep] * (neg_softmax ? stats[wave * 16 + r] : 1.f);
+      outp[f] = band(r)[k * a.ostep] * (scaled ? stats[wave * 16 + r] : 1.f);
     }
   }
 }

@@ -64,3 +64,22 @@ def test_non_finite_features(handle):
     inf = ~fin & ~np.isnan(ref)
     assert np.array_equal(got[inf], ref[inf])
     assert np.all(np.abs(got[fin] - ref[fin]) <= 16 * 2.0**-24 * size[fin])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W,dmin,step,D", [
+    (150, 0, 1, 128), (70, 3, 1, 112), (150, 0, -1, 127),  # in the accumulators, 9 column tiles
+    (150, 0, 1, 111),                                      # the widest band that goes through LDS
+    (300, 0, 1, 256), (66, 0, 1, 240),                     # 17 column tiles
+])
+def test_softmax_epilogue(handle, dtype, W, dmin, step, D):
+    """-softmax of the raw volume, which the raw epilogue gives: exp(s - max) has
+    2^-21 (the hardware's exp2 and the rounding of its argument, |s - max| < 16), the
+    sum D more roundings at most, the quotient three."""
+    g = torch.Generator(device="cuda").manual_seed(W + D)
+    f0, f1 = (torch.randn((3, W, 104), generator=g, device="cuda").mul(0.3).to(dtype) for _ in range(2))
+    raw = ops.correlation_volume(handle, f0, f1, 104, dmin, step, D, epilogue="raw").double()
+    got = ops.correlation_volume(handle, f0, f1, 104, dmin, step, D).double()
+    want = -torch.softmax(raw, dim=-1)
+    tol = (2.0**-20 + (D + 3) * 2.0**-24) * want.abs() + 1e-30
+    assert ((got - want).abs() <= tol).all()
