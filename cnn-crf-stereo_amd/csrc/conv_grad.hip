@@ -161,6 +161,8 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
           all = max(all, mx[e]);
         }
         const bool finite = !__any(all >= 0x7f800000u);
+        const unsigned neg = u.z && buf ? kNegate : 0u;  // every other segment's dz
+        const unsigned scale0 = (268u << 23) + neg, unscale0 = u.z ? neg - (28u << 23) : 0u;
         f32x4 unscale;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -169,13 +171,18 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
 #pragma unroll
             for (int i = 0; i < 6; ++i)
               if (i < 4 || !u.z) mx[e] = max(mx[e], finite_bits(__uint_as_float(bits(e, i))));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // (a value that the scale does not reach)
+              if ((reg[n][i][e] & 0x7fffffffu) >= 0x7f800000u) reg[n][i][e] ^= neg;
           }
           mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0xb1, 0xf, 0xf, true));
           mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x4e, 0xf, 0xf, true));
           mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x141, 0xf, 0xf, true));  // row_half_mirror
           const int eb = split_exp(mx[e]);
-          const float sc = split_scale(eb);
-          unscale[e] = u.z ? split_unscale(eb) : __uint_as_float((unsigned)eb << 23);
+          // split_scale and split_unscale (x's side: 2^(eb - 127)) with the sign,
+          // which is carried through by sums modulo 2^32
+          const float sc = __uint_as_float(scale0 - ((unsigned)eb << 23));
+          unscale[e] = __uint_as_float(((unsigned)eb << 23) + unscale0);
           typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
           typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
           f16x4 hi, lo;

@@ -75,6 +75,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_image_split(const float* __rest
       for (int e = 0; e < 8; ++e) wf[t][k][e] = p[k][e];
   }
 
+  // Odd pixels of a float32 map are multiplied negated (see kNegate).
+  const unsigned neg = sizeof(TO) == 4 ? (unsigned)lrow << 31 : 0u;
+  const float sg = sizeof(TO) == 4 && (lrow & 1) ? -1.f : 1.f;
   auto run = [&](auto f) {
     for (; tile < tiles; tile += nw) {
       const long p = tile * 16 + lrow;
@@ -82,7 +85,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_image_split(const float* __rest
       bf16 s[3][8];
       bf16x8 a[3];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 8 * lgrp + e < T ? in[e] : 0.f;
+      for (int e = 0; e < 8; ++e) v[e] = 8 * lgrp + e < T ? with_sign(in[e], neg) : 0.f;
       split3(v, s[0], s[1], s[2]);
 #pragma unroll
       for (int k = 0; k < 3; ++k)
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_image_split(const float* __rest
         vec4 o;
         const f32x4 bn = *reinterpret_cast<const f32x4*>(bs + n0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (TO)(n0 + e < K ? f(c[t][e] + bn[e]) : 0.f);
+        for (int e = 0; e < 4; ++e) o[e] = (TO)(n0 + e < K ? f(fmaf(c[t][e], sg, bn[e])) : 0.f);
         if (p < P && n0 < Cs) *reinterpret_cast<vec4*>(row + n0) = o;
       }
     }

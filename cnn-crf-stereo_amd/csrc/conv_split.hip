@@ -211,16 +211,20 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
           for (int e = 0; e < 8; ++e) mx = max(mx, finite_bits(f[e]));
         }
         const int eb = split_exp(quad_max(mx));
+        const unsigned neg = (unsigned)(px / AC + px % AC) << 31;  // (a checkerboard of signs: see kNegate)
         f16x8 p[2];
-        if (finite)
-          split2<true>(f, split_scale(eb), p[0], p[1]);
-        else
+        if (finite) {
+          split2<true>(f, with_sign(split_scale(eb), neg), p[0], p[1]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] = with_sign(f[e], neg);
           split2<false>(f, split_scale(eb), p[0], p[1]);
+        }
         if (v < NU) {
           const int off = px * 64 + split_swz(px, g) * 16;
 #pragma unroll
           for (int k = 0; k < 2; ++k) *reinterpret_cast<f16x8*>(lds + k * Cfg::plane + off) = p[k];
-          if (g == 0) *reinterpret_cast<float*>(lds + Cfg::scale_off + px * 4) = split_unscale(eb);
+          if (g == 0) *reinterpret_cast<float*>(lds + Cfg::scale_off + px * 4) = with_sign(split_unscale(eb), neg);
         }
       } else {
         bf16 p[3][8];
@@ -319,13 +323,20 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     const bool ok = kg < Cfg::taps * R;
     const int tap = ok ? kg / R : 0, g = ok ? kg % R : 0;
     const int ti = tap / Cfg::KW, tj = tap % Cfg::KW;
+    // (the output pixel's sign here)
+    const unsigned par = (unsigned)(MT * wave + lrow) & 1u, odd = par * 0x80008000u;
     bf16x8 a[3][MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int px = (MT * wave + m + ti) * AC + tj + lrow;
       const int o = ok ? (px * R + g) * 16 : Cfg::zero_off;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) a[k][m] = *reinterpret_cast<const bf16x8*>(lds + o + (ok ? k * Cfg::rplane : 0));
+      for (int k = 0; k < 3; ++k) {
+        u32x4 v = *reinterpret_cast<const u32x4*>(lds + o + (ok ? k * Cfg::rplane : 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] ^= (m & 1) ? odd ^ 0x80008000u : odd;
+        a[k][m] = __builtin_bit_cast(bf16x8, v);
+      }
     }
     const bf16x8* p = reinterpret_cast<const bf16x8*>(lds + Cfg::w3_off + (ql & 1) * Cfg::w3) + lane;
 #pragma unroll
@@ -349,7 +360,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
       mm(0, 0);
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        acc[m][t] += cur[m];
+        const float sg = ((m & 1) ^ (int)par) ? -1.f : 1.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[m][t][e] = fmaf(cur[m][e], sg, acc[m][t][e]);
         asm volatile("" : "+v"(acc[m][t]));  // added here, not behind the step (the sums of all tiles would spill)
       }
     }

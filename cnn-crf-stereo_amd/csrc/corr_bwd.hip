@@ -112,6 +112,12 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
   const T* frow = (const T*)(gather ? a.f0 : a.f1) + rowpix * Cs;
   const float* grow = a.G + rowpix * D;
 
+  // Odd rows of a float32 map are multiplied negated (see kNegate).  A bfloat16
+  // result is rounded at 2^-9 of itself, to nearest, which hides an offset of
+  // 1e-7 also in a sum over a frame (and the sign cost 1361 -> 1610 us there).
+  const unsigned neg = kF32 && (h & 1) ? kNegate : 0u;
+  const float sg = kF32 && (h & 1) ? -1.f : 1.f;
+
   // Rows Cs .. 112 of the planes stay zero.
   for (int v = tid; v < Cfg::PLANES * (16 * NT - Cs) * (PITCH / 8); v += Cfg::THREADS) {
     const int pl = v / ((16 * NT - Cs) * (PITCH / 8)), w = v % ((16 * NT - Cs) * (PITCH / 8));
@@ -136,7 +142,7 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
         const int R = 4 * q + i, col = col0 + s * R;
         const bool ok = R < last && col >= 0 && col < W;
         const u32x4 val = *reinterpret_cast<const u32x4*>(frow + (long)(ok ? col : 0) * Cs + g * VE);
-        r[i] = ok ? val : u32x4{0u, 0u, 0u, 0u};
+        r[i] = ok ? (kF32 ? val ^ neg : val) : u32x4{0u, 0u, 0u, 0u};
       }
       unsigned char* d = lds + (g * VE * PITCH + 4 * q) * 2;
       if constexpr (kF32) {
@@ -284,7 +290,8 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
     for (int t = 0; t < NT; ++t) {
       const int c = 16 * t + 4 * lgrp;
       typedef __attribute__((ext_vector_type(4))) T vec4;
-      if (c < Cs) *reinterpret_cast<vec4*>(out + (long)pix[mt] * Cs + c) = __builtin_convertvector(acc[mt][t], vec4);
+      const f32x4 v = kF32 ? acc[mt][t] * sg : acc[mt][t];
+      if (c < Cs) *reinterpret_cast<vec4*>(out + (long)pix[mt] * Cs + c) = __builtin_convertvector(v, vec4);
     }
   }
 }
