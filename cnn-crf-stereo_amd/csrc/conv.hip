@@ -1025,7 +1025,7 @@ extern "C" int ccs_conv_forward_packed(ccs_handle_t h, const void* x, int x_layo
 // GPU (held until the process ends) instead of the handle's scratch.  The
 // array's name is a host-side stand-in, not a device address: host code uses
 // only the address hipGetSymbolAddress returns on each device.
-constexpr size_t kNoAllocScratchBytes = 512u << 10;  // the largest MFMA pack is 452,032 bytes
+constexpr size_t kNoAllocScratchBytes = 512u << 10;  // the largest MFMA pack is 452,064 bytes
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -3,12 +3,17 @@
 //
 // gfx950 runs v_mfma_f32_16x16x32_f16 (and _bf16) at 16 times the rate of
 // v_mfma_f32_16x16x4_f32.  Both operands are split into two float16 terms,
-// x s = xh + xl and w t = wh + wl (split2: one rounding of at most 2^-24), with a
-// power of two s for each pixel's 32 channels of a stage and t for each output
-// channel, and a product is formed from
-//   wl xh + wh xl + wh xh,
+// x s = xh + xl / 4096 and w t = wh + wl / 4096 (split_pair), with a power of two s
+// for each pixel's 32 channels of a stage and t for each output channel, and a
+// product is formed from
+//   (wl xh + wh xl) / 4096 + wh xh,
 // each exact in the matrix core and accumulated in float32; wl xl, the one left
-// out, is below 2^-24 |x w|.  Channels past the last multiple of 32 take an exact
+// out, is at most 2^-22 |x w| (2^-25 root mean square).  A tile whose inputs a pair does
+// not hold (BlockRange: non-zero channels of a pixel more than 2^29 apart, huge or
+// infinite values) is computed on v_mfma_f32_16x16x4_f32 from memory instead, and so
+// are all tiles where the weights of a row are so far apart (their pack then
+// holds them in float32): every output keeps float32's precision for any inputs.
+// Channels past the last multiple of 32 take an exact
 // three-way bfloat16 split (split3) and six of its nine products instead: their
 // reduction steps hold several taps, hence several pixels, in one instruction, so
 // no scale fits.  A 32-deep step is summed from zero and added to the accumulator
@@ -28,12 +33,14 @@
 // are spread between the next tile's MFMAs.
 //
 // Measured (100 channels, us; the float32-MFMA kernel -> six bfloat16 products
-// with the weights read from L2 by every wave -> this): 3x3 at 1256 x 389
-// 1456 -> 565 -> 417, at 524 x 268 - -> 175 -> 110, 2x2 at 749 x 501
-// 530 -> 205 -> 157, at 325 x 245 140 -> 65 -> 42, at 200 x 100 - -> 37 -> 18.  At
-// 1256 x 389 the matrix cores are busy half of the time at 1.9 GHz; the rest is
-// staging, the epilogue's tanh, and waits.  Tiles of 16 x 16 (MT = 4, two
-// workgroups per CU) took 412, 128, 163, 52 and 30 us.
+// with the weights read from L2 by every wave -> both terms in one unit, which lost
+// the small channels of uneven pixels -> this): 3x3 at 1256 x 389 1456 -> 565 -> 426
+// -> 453, at 524 x 268 - -> 175 -> 120 -> 129, 2x2 at 749 x 501 530 -> 205 -> 165 ->
+// 172, at 325 x 245 140 -> 65 -> 41 -> 43, at 200 x 100 - -> 37 -> 18 -> 19.  (The
+// second unit takes one more addition per value and step, 4 %, looking for blocks
+// that pairs do not hold 2 %.)  At 1256 x 389 the matrix cores are busy half of the
+// time; the rest is staging, the epilogue's tanh, and waits.  Tiles of 16 x 16 (MT =
+// 4, two workgroups per CU; with one unit) took 412, 128, 163, 52 and 30 us.
 #include <type_traits>
 
 #include "conv_split.hpp"
@@ -58,10 +65,13 @@ struct SplitCfg {
   static constexpr int w2_off = (scale_off + NPX * 4 + 1023) & ~1023;
   static constexpr int w3_off = (3 * rplane + 1023) & ~1023;
   static constexpr int zero_off = w2_off + 2 * w2 > w3_off + 2 * w3 ? w2_off + 2 * w2 : w3_off + 2 * w3;
-  static constexpr int lds_bytes = zero_off + 16;
-  // packed weights: two-plane fragments, three-plane fragments, row scales
+  static constexpr int fail_off = zero_off + 16;  // per wave: its share of the inputs fails
+  static constexpr int lds_bytes = fail_off + 16;
+  // packed weights: two-plane fragments, three-plane fragments, row scales, per tile
+  // of 16 rows whether its two-plane fragments are float32 values instead
   static constexpr size_t frag_bytes = (size_t)NT * 1024 * (2 * FULL * taps + 3 * REM_NQ);
-  static constexpr size_t packed_bytes = frag_bytes + NT * 16 * sizeof(float);
+  static constexpr size_t wide_off = frag_bytes + NT * 16 * sizeof(float);
+  static constexpr size_t packed_bytes = wide_off + (NT + 3) / 4 * 16;
 };
 
 // Reduction step q of the packed weights, lane group lgrp: the tap and the
@@ -84,8 +94,10 @@ __host__ __device__ inline void split_step(int q, int lgrp, int* tap, int* c0) {
 // Packed layout: step q < FULL * taps as [q][t][2][lane][8] float16, the others
 // as [q][t][3][lane][8] bfloat16, the fragment of channel tile t with lane
 // (lrow, lgrp) holding output channel 16 t + lrow; then the row scales.  All
-// weights of a row are divided by its scale.  Block (t, y) packs a share of tile
-// t's steps; its 16 groups of 16 lanes each look at one row first.
+// weights of a row are divided by its scale.  A tile with a row that pairs do not
+// hold has scales of 1 and its first fragments as [q][t][2][lane][4] float32.
+// Block (t, y) packs a share of tile t's steps; its 16 groups of 16 lanes each look
+// at one row first.
 constexpr int kPackShares = 16;
 template <class Cfg>
 __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w, int K, int C, int adj,
@@ -96,20 +108,24 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
   auto at = [&](int n, int c, int tap) {
     return w[adj ? ((long)c * K + n) * Cfg::taps + tap : ((long)n * C + c) * Cfg::taps + (Cfg::taps - 1 - tap)];
   };
-  {
-    const int n = 16 * t + (tid >> 4);
-    unsigned mx = 0;
-    if (n < K) {  // (eight loads in flight)
+  const int row = 16 * t + (tid >> 4);
+  BlockRange r;
+  if (row < K) {  // (eight loads in flight)
 #pragma unroll 8
-      for (int i = tid & 15; i < C * Cfg::taps; i += 16) mx = max(mx, finite_bits(at(n, i / Cfg::taps, i % Cfg::taps)));
-    }
-    for (int o = 1; o < 16; o <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 16));
-    if ((tid & 15) == 0) {
-      exps[tid >> 4] = split_exp(mx);
-      if (blockIdx.y == 0)
-        reinterpret_cast<float*>(out + Cfg::frag_bytes)[n] = __uint_as_float((unsigned)split_exp(mx) << 23);
+    for (int i = tid & 15; i < C * Cfg::taps; i += 16) {
+      const float v = at(row, i / Cfg::taps, i % Cfg::taps);
+      r.add(v, v);
     }
   }
+  unsigned mx = r.largest();
+  for (int o = 1; o < 16; o <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 16));
+  const bool wide = __syncthreads_or(r.fails(split_exp(mx)));
+  if ((tid & 15) == 0) {
+    exps[tid >> 4] = wide ? 127 : split_exp(mx);
+    if (blockIdx.y == 0)
+      reinterpret_cast<float*>(out + Cfg::frag_bytes)[row] = wide ? 1.f : __uint_as_float((unsigned)split_exp(mx) << 23);
+  }
+  if (blockIdx.y == 0 && tid == 0) reinterpret_cast<int*>(out + Cfg::wide_off)[t] = wide;
   __syncthreads();
   for (int u = blockIdx.y * 256 + tid; u < Cfg::NQ * 64; u += kPackShares * 256) {
     const int q = u >> 6, lane = u & 63, n = 16 * t + (lane & 15);
@@ -122,7 +138,13 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
     constexpr int NQ2 = Cfg::FULL * Cfg::taps;
     if (q < NQ2) {
       f16x8 p[2];
-      split2<false>(v, split_scale(eb), p[0], p[1]);
+      if (wide) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          p[k] = __builtin_bit_cast(f16x8, f32x4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]});
+      } else {
+        split_pair(v, split_scale(eb), p[0], p[1]);
+      }
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         *reinterpret_cast<f16x8*>(out + ((long)((q * Cfg::NT + t) * 2 + k) * 64 + lane) * 16) = p[k];
@@ -170,6 +192,11 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   if (tile >= tiles) return;  // (uniform) the grid is rounded up to 8 runs
   const int h0 = (tile / tiles_x) * Cfg::TH, w0 = (tile % tiles_x) * Cfg::TW;
   if (tid == 0) *reinterpret_cast<u32x4*>(lds + Cfg::zero_off) = u32x4{0u, 0u, 0u, 0u};
+  bool fails = false;  // an input of this lane is not held by its pair
+  int wide_rows = 0;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wide_rows |= reinterpret_cast<const int*>(wpk + Cfg::wide_off)[t];
+  bool again = wide_rows != 0;  // (uniform) the tile takes float32 products
 
   // Stage of G groups from channel group cg0: unit (pixel, group) of eight
   // channels, all loads issued before the first is split and stored.
@@ -178,15 +205,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   auto stage = [&](auto gc, int cg0) {
     constexpr int G = decltype(gc)::value;
     constexpr int NU = NPX * G, PER = (NU + Cfg::threads - 1) / Cfg::threads;
-    f32x4 r[PER][2];
+    f32x4 in[PER][2];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int v = min(tid + Cfg::threads * i, NU - 1);
       const int px = v / G, g = v % G;
       const int hi = min(h0 + px / AC, Hin - 1), wi = min(w0 + px % AC, Win - 1);
       const f32x4* src = reinterpret_cast<const f32x4*>(x + ((long)hi * Win + wi) * Cs + (cg0 + g) * 8);
-      r[i][0] = src[0];
-      r[i][1] = src[1];
+      in[i][0] = src[0];
+      in[i][1] = src[1];
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -194,32 +221,21 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
       const int px = v / G, g = v % G;
       float f[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = r[i][e >> 2][e & 3];
+      for (int e = 0; e < 8; ++e) f[e] = in[i][e >> 2][e & 3];
       if constexpr (G == 4) {
         // A pixel's four units lie in a quad of lanes: one scale for its 32 channels.
         auto quad_max = [](unsigned m) {
           m = max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0xb1, 0xf, 0xf, true));
           return max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x4e, 0xf, 0xf, true));
         };
-        unsigned mx = 0;
+        BlockRange r;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) mx = max(mx, __float_as_uint(f[e]) & 0x7fffffffu);
-        const bool finite = !__any(mx >= 0x7f800000u);
-        if (!finite) {
-          mx = 0;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) mx = max(mx, finite_bits(f[e]));
-        }
-        const int eb = split_exp(quad_max(mx));
+        for (int e = 0; e < 8; e += 2) r.add(f[e], f[e + 1]);
+        const int eb = split_exp(quad_max(r.largest()));
+        fails |= r.fails(eb);
         const unsigned neg = (unsigned)(px / AC + px % AC) << 31;  // (a checkerboard of signs: see kNegate)
         f16x8 p[2];
-        if (finite) {
-          split2<true>(f, with_sign(split_scale(eb), neg), p[0], p[1]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) f[e] = with_sign(f[e], neg);
-          split2<false>(f, split_scale(eb), p[0], p[1]);
-        }
+        split_pair(f, with_sign(split_scale(eb), neg), p[0], p[1]);
         if (v < NU) {
           const int off = px * 64 + split_swz(px, g) * 16;
 #pragma unroll
@@ -228,6 +244,10 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         }
       } else {
         bf16 p[3][8];
+        BlockRange r;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) r.add(f[e], f[e + 1]);
+        fails |= r.fails(29);  // (only the largest values: no scale is shared)
         split3(f, p[0], p[1], p[2]);
         if (v < NU) {
 #pragma unroll
@@ -240,6 +260,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         }
       }
     }
+    const bool any = __any(fails);  // (read behind the barrier that follows)
+    if (lane == 0) *reinterpret_cast<int*>(lds + Cfg::fail_off + 4 * wave) = any;
   };
 
   // Lane (lrow, lgrp) holds pixel lrow of row MT wave + m and channels
@@ -283,14 +305,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     }
     const f16x8* wb = reinterpret_cast<const f16x8*>(lds + Cfg::w2_off + (q & 1) * Cfg::w2) + lane;
     f16x8 b0[2] = {wb[0], wb[64]}, b1[2];
-    f32x4 cur[2][MT];
+    f32x4 low[2][MT], high[2][MT];  // the products with a low term, and the others
     auto add = [&](int t, int m) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[m][t][e] = fmaf(cur[t & 1][m][e], sc[m], acc[m][t][e]);
+      for (int e = 0; e < 4; ++e)
+        acc[m][t][e] = fmaf(fmaf(low[t & 1][m][e], 1.f / kLowUnit, high[t & 1][m][e]), sc[m], acc[m][t][e]);
     };
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      f32x4(&c)[MT] = cur[t & 1];
+      f32x4(&c)[MT] = low[t & 1];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         c[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[1], a[0][m], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -307,7 +330,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         if (t > 0 && m > 0) add(t - 1, m);
       }
 #pragma unroll
-      for (int m = 0; m < MT; ++m) c[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[0], a[0][m], c[m], 0, 0, 0);
+      for (int m = 0; m < MT; ++m)
+        high[t & 1][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[0], a[0][m], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       b0[0] = b1[0];
       b0[1] = b1[1];
@@ -368,13 +392,21 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     }
   };
 
+  // Whether the staged inputs fail in one of the waves (behind the barrier).
+  auto failed = [&]() {
+    const u32x4 f = *reinterpret_cast<const u32x4*>(lds + Cfg::fail_off);
+    return __builtin_amdgcn_readfirstlane(f[0] | f[1] | f[2] | f[3]) != 0;
+  };
+  // (from the first failure on, without steps: leaving the loops instead takes 50 registers more)
   copy2(0);
 #pragma unroll 1
   for (int s = 0; s < Cfg::FULL; ++s) {
     stage(std::integral_constant<int, 4>{}, 4 * s);
     step_barrier();
+    again |= failed();
+    const int taps = again ? 0 : Cfg::taps;
 #pragma unroll 1
-    for (int tap = 0; tap < Cfg::taps; ++tap) {
+    for (int tap = 0; tap < taps; ++tap) {
       const int q = s * Cfg::taps + tap;
       if (q + 1 < Cfg::FULL * Cfg::taps) copy2(q + 1);
       step2(q, tap / Cfg::KW, tap % Cfg::KW);
@@ -385,19 +417,85 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     copy3(0);
     stage(std::integral_constant<int, Cfg::REM>{}, 4 * Cfg::FULL);
     step_barrier();
+    again |= failed();
+    const int steps = again ? 0 : Cfg::REM_NQ;
 #pragma unroll 1
-    for (int ql = 0; ql < Cfg::REM_NQ; ++ql) {
+    for (int ql = 0; ql < steps; ++ql) {
       if (ql + 1 < Cfg::REM_NQ) copy3(ql + 1);
       step3(ql);
       if (ql + 1 < Cfg::REM_NQ) step_barrier();
     }
   }
 
+  // The tile on v_mfma_f32_16x16x4_f32, for what the pairs do not hold.  Inputs and
+  // weights come from memory: as slow as a layer in float32 products (3x3 at 1256 x
+  // 389 with every tile out of range 1.5 to 1.6 ms, 1.46 ms by the kernel that this one
+  // replaced), and rare.
+  const f32x4* rows = reinterpret_cast<const f32x4*>(wpk + Cfg::frag_bytes);
+  auto float_tile = [&]() {
+    const int* wide = reinterpret_cast<const int*>(wpk + Cfg::wide_off);
+    const float* scale = reinterpret_cast<const float*>(rows) + lrow;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int q = 0; q < Cfg::NQ; ++q) {
+      int tap, c0;
+      split_step<Cfg>(q, lgrp, &tap, &c0);
+      const bool ok = c0 >= 0;
+      f32x4 xv[MT][2];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int hi = min(h0 + MT * wave + m + (ok ? tap / Cfg::KW : 0), Hin - 1);
+        const int wi = min(w0 + lrow + (ok ? tap % Cfg::KW : 0), Win - 1);
+        const f32x4* src = reinterpret_cast<const f32x4*>(x + ((long)hi * Win + wi) * Cs + (ok ? c0 : 0));
+        xv[m][0] = src[0];
+        xv[m][1] = src[1];
+        if (!ok) xv[m][0] = xv[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      const int ql = q - Cfg::FULL * Cfg::taps;
+#pragma unroll 1
+      for (int t = 0; t < NT; ++t) {
+        float v[8];
+        if (ql < 0) {
+          const u32x4* p = reinterpret_cast<const u32x4*>(wpk + (long)(q * NT + t) * 2048) + lane;
+          const u32x4 p0 = p[0], p1 = p[64];
+          if (wide[t]) {  // (uniform)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(e < 4 ? p0[e & 3] : p1[e & 3]);
+          } else {
+            const f16x8 h = __builtin_bit_cast(f16x8, p0), l = __builtin_bit_cast(f16x8, p1);
+            const float s = scale[16 * t] * 0x1p-14f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = fmaf((float)l[e], 1.f / kLowUnit, (float)h[e]) * s;
+          }
+        } else {
+          const bf16x8* p =
+              reinterpret_cast<const bf16x8*>(wpk + (long)Cfg::FULL * Cfg::taps * Cfg::w2 + (long)(ql * NT + t) * 3072) + lane;
+          const bf16x8 h = p[0], mid = p[64], l = p[128];
+          const float s = scale[16 * t];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = ((float)h[e] + (float)mid[e] + (float)l[e]) * s;
+        }
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)  // (the accumulators' index is a constant)
+          if (tt == t) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                acc[m][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], xv[m][e >> 2][e & 3], acc[m][tt], 0, 0, 0);
+          }
+      }
+    }
+  };
+  if (again) float_tile();
+
   // Epilogue: row scale, bias, tanh, four channels of one pixel per lane and
   // store (16 bytes).  Padding channels are stored as zeros (an infinite input
   // times their zero weights is NaN).
   __builtin_amdgcn_sched_barrier(0);  // (its loads stay behind the last step: registers)
-  const f32x4* rows = reinterpret_cast<const f32x4*>(wpk + Cfg::frag_bytes);
   f32x4 rs[NT], bn[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -407,6 +505,10 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
       const int n = 16 * t + 4 * lgrp + e;
       bn[t][e] = (n < K && bias) ? bias[n] : 0.f;
     }
+  }
+  if (again) {  // (in float32 products the scales are taken with the weights)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) rs[t] = f32x4{1.f, 1.f, 1.f, 1.f};
   }
   auto epilogue = [&](auto f) {
 #pragma unroll

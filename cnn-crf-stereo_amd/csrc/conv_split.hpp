@@ -57,7 +57,7 @@ __device__ __forceinline__ unsigned finite_bits(float x) {  // |x| as ordered bi
   const unsigned b = __float_as_uint(x) & 0x7fffffffu;
   return b < 0x7f800000u ? b : 0u;
 }
-// A block's biased exponent from its largest finite_bits (from 29, so that the
+// A block's biased exponent from its largest |x| bits (from 29, so that the
 // factors below are normal numbers: smaller blocks keep a share of the bits).
 __device__ __forceinline__ int split_exp(unsigned mx) { return max((int)(mx >> 23), 29); }
 // s, and 2^-28 / s: what a sum of products of two split blocks takes back, but
@@ -77,6 +77,42 @@ constexpr unsigned kNegate = 0x80000000u;
 __device__ __forceinline__ float with_sign(float x, unsigned sign) {  // x, negated by sign = kNegate
   return __uint_as_float(__float_as_uint(x) ^ sign);
 }
+
+// x s = h + l / kLowUnit in float16, as split2, but the rest is scaled up to h's
+// size before it is rounded, so that it stays a normal number for values down to
+// 2^-29 of the block's largest: what is left out is at most 2^-22 |x| for those and
+// 2^-24 |x| down to 2^-16.  (In one unit, the rest of a value below 2^-15 of the largest
+// is a subnormal number or lost: uneven channels of one pixel came out wrong.)  The
+// products with a low term are summed apart from those without.  No value of the
+// block may be infinite.
+constexpr float kLowUnit = 4096.f;
+__device__ __forceinline__ void split_pair(const float (&x)[8], float s, f16x8& h, f16x8& l) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = x[e] * s;
+    h[e] = (_Float16)v;
+    l[e] = (_Float16)fmaf((float)h[e], -kLowUnit, v * kLowUnit);
+  }
+}
+
+// The largest |x| of a block and the smallest that is not 0, as ordered bits, one
+// instruction per value for the smallest and half of one for the largest: above,
+// |x| (a NaN is passed over), below, 2 |x| - 2, which makes 0 the largest.
+struct BlockRange {
+  float above = 0.f;
+  unsigned below = ~0u;
+  __device__ __forceinline__ void add(float x, float y) {
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(above) : "v"(x), "v"(y));
+    below = min(below, min((__float_as_uint(x) << 1) - 2u, (__float_as_uint(y) << 1) - 2u));
+  }
+  __device__ __forceinline__ unsigned largest() const { return __float_as_uint(above); }
+  // Whether split_pair does not hold a value of the block, or its sums of products may
+  // leave float32's range before their scales are taken back (from 2^115).  eb: the
+  // block's split_exp.  A NaN is held: both terms are NaN.
+  __device__ __forceinline__ bool fails(int eb, unsigned huge = 242u << 23) const {
+    return largest() >= huge || below < (unsigned)(eb - 29) << 24;
+  }
+};
 
 template <bool FINITE>  // every value is finite
 __device__ __forceinline__ void split2(const float (&x)[8], float s, f16x8& h, f16x8& l) {

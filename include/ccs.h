@@ -104,7 +104,7 @@ int ccs_conv2d_forward(ccs_handle_t h, const void* x, int x_layout, int H, int W
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The weights
  * are packed into one fixed 512 KiB array per GPU, held until the process
  * ends, instead of the handle's scratch; every MFMA shape fits (100 -> 100 3x3
- * in FP32 packs to 452,032 bytes) and a larger pack returns
+ * in FP32 packs to 452,064 bytes) and a larger pack returns
  * CCS_ERR_UNSUPPORTED.  All calls on one GPU share that array, which keeps the
  * last call's packed weights: calls that overlap on one GPU (other streams,
  * other host threads) race.  Same arguments, outputs and kernels as

@@ -1,0 +1,76 @@
+"""float32 kernels on split products keep float32's precision for every input: values
+of any sizes inside one block of a common scale, and sums near the largest float.
+
+Every case has outputs whose terms are small beside other values of their block,
+which meet a zero.  A pair must hold each value to 2^-22 of itself or leave the block
+to float32 products, whose chain of N additions is off by 2^-24 sqrt(N / 6) of the
+sum's 2-norm (partial sums grow with sqrt(i / N), roundings are uniform): 3.7e-7 for
+the 234 steps of a 3x3 layer, 4.5e-7 with 2^-22 / sqrt(12) per factor beside it.  The
+2-norm of each output channel's error is held to 8e-7 of the channel's.
+"""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from cnn_crf_stereo_amd import capi, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def uniform(rng, *shape):
+    """Magnitudes of one size: in (-1, 1) without what lies near zero."""
+    return rng.uniform(0.25, 1, shape) * rng.choice([-1.0, 1.0], shape)
+
+
+def check(got, ref):
+    """got, ref: channels x outputs, float64."""
+    err = np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= 8e-7, err.max()
+
+
+LAYER_CASES = ["one channel 1e8", "one channel 1e12", "one channel 1e30", "one weight 1e9", "one weight 1e25", "both",
+               "units", "huge", "tiny"]
+
+
+def layer_case(rng, case, C, k):
+    x, w = uniform(rng, C, 20, 37), 0.1 * uniform(rng, C, C, k, k)
+    if case.startswith("one channel") or case == "both":  # channel 5, as far as the weights are concerned not there
+        x[5] *= float(case.split()[-1]) if case != "both" else 1e12
+        w[:, 5] = 0
+    if case.startswith("one weight") or case == "both":  # a weight that only meets zeros
+        w[:, 9] *= float(case.split()[-1]) if case != "both" else 1e12
+        x[9] = 0
+    if case == "units":  # every channel in a unit of its own, which its weights take back
+        unit = 10.0 ** rng.uniform(-12, 12, C)
+        x, w = x * unit[:, None, None], w / unit[None, :, None, None]
+    if case == "huge":
+        x, w = x * 2e37, w * 1e-3
+    if case == "tiny":
+        x = x * 1e-30
+    return x.astype(np.float32), w.astype(np.float32)
+
+
+@pytest.mark.parametrize("case", LAYER_CASES)
+@pytest.mark.parametrize("C,k", [(100, 3), (100, 2), (64, 3)])
+def test_layer(handle, C, k, case):
+    x, w = layer_case(np.random.default_rng(C + k), case, C, k)
+    hwc = torch.zeros((*x.shape[1:], capi.feature_stride(C)), device="cuda")
+    hwc[:, :, :C] = torch.as_tensor(x, device="cuda").permute(1, 2, 0)
+    y = ops.ConvLayer(handle, w, None, "fp32", act=False)(handle, hwc)
+    ref = F.conv2d(torch.as_tensor(x).double()[None], torch.as_tensor(w).double().flip(2, 3))[0].numpy()
+    check(y[:, :, :C].permute(2, 0, 1).double().cpu().numpy().reshape(C, -1), ref.reshape(C, -1))
+
+
+def test_layer_pixels_apart(handle):
+    """A pixel out of range leaves the outputs that it does not reach to the bit as
+    they are in another tile, and takes the others' tile to float32 products."""
+    rng = np.random.default_rng(0)
+    x, w = layer_case(rng, "", 100, 3)
+    layer = ops.ConvLayer(handle, w, None, "fp32")
+    hwc = torch.zeros((20, 37, 104), device="cuda")
+    hwc[:, :, :100] = torch.as_tensor(x, device="cuda").permute(1, 2, 0)
+    want = layer(handle, hwc)
+    hwc[2, 3, 7] = 1e-30
+    got = layer(handle, hwc)
+    assert torch.equal(got[8:], want[8:]) and torch.equal(got[:, 16:], want[:, 16:])
