@@ -8,11 +8,11 @@
 // product is formed from
 //   (wl xh + wh xl) / 4096 + wh xh,
 // each exact in the matrix core and accumulated in float32; wl xl, the one left
-// out, is at most 2^-22 |x w| (2^-25 root mean square).  A tile whose inputs a pair does
-// not hold (BlockRange: non-zero channels of a pixel more than 2^29 apart, huge or
-// infinite values) is computed on v_mfma_f32_16x16x4_f32 from memory instead, and so
-// are all tiles where the weights of a row are so far apart (their pack then
-// holds them in float32): every output keeps float32's precision for any inputs.
+// out, is at most 2^-22 |x w| (2^-25 root mean square).  Where that does not do
+// (BlockRange) a tile is computed on v_mfma_f32_16x16x4_f32 from memory instead: with
+// huge or infinite inputs, or channels of a pixel more than 2^29 apart that meet
+// uneven weights; and all tiles where the weights of a row are so far apart (their pack
+// then holds them in float32).  Every output keeps float32's precision for any inputs.
 // Channels past the last multiple of 32 take an exact
 // three-way bfloat16 split (split3) and six of its nine products instead: their
 // reduction steps hold several taps, hence several pixels, in one instruction, so
@@ -34,13 +34,13 @@
 //
 // Measured (100 channels, us; the float32-MFMA kernel -> six bfloat16 products
 // with the weights read from L2 by every wave -> both terms in one unit, which lost
-// the small channels of uneven pixels -> this): 3x3 at 1256 x 389 1456 -> 565 -> 426
-// -> 453, at 524 x 268 - -> 175 -> 120 -> 129, 2x2 at 749 x 501 530 -> 205 -> 165 ->
-// 172, at 325 x 245 140 -> 65 -> 41 -> 43, at 200 x 100 - -> 37 -> 18 -> 19.  (The
-// second unit takes one more addition per value and step, 4 %, looking for blocks
-// that pairs do not hold 2 %.)  At 1256 x 389 the matrix cores are busy half of the
-// time; the rest is staging, the epilogue's tanh, and waits.  Tiles of 16 x 16 (MT =
-// 4, two workgroups per CU; with one unit) took 412, 128, 163, 52 and 30 us.
+// the small channels of uneven pixels -> this): 3x3 at 1256 x 389 1456 -> 565 -> 411
+// -> 431, at 524 x 268 - -> 175 -> 109 -> 115, 2x2 at 749 x 501 530 -> 205 -> 151 ->
+// 157, at 325 x 245 140 -> 65 -> 41 -> 43, at 200 x 100 - -> 37 -> 18 -> 19.  (The
+// second unit takes one more addition per value and step.)  At 1256 x 389 the matrix
+// cores are busy half of the time; the rest is staging, the epilogue's tanh, and waits.
+// Tiles of 16 x 16 (MT = 4, two workgroups per CU; with one unit) took 412, 128, 163,
+// 52 and 30 us.
 #include <type_traits>
 
 #include "conv_split.hpp"
@@ -67,12 +67,13 @@ struct SplitCfg {
   static constexpr int zero_off = w2_off + 2 * w2 > w3_off + 2 * w3 ? w2_off + 2 * w2 : w3_off + 2 * w3;
   static constexpr int fail_off = zero_off + 16;  // per wave: its share of the inputs fails
   static constexpr int lds_bytes = fail_off + 16;
-  // packed weights: two-plane fragments, three-plane fragments, row scales, per tile
-  // of 16 rows whether its two-plane fragments are float32 values instead
+  // packed weights: two-plane fragments, three-plane fragments, row scales, and per
+  // tile of 16 rows kWide (its two-plane fragments are float32 values instead) and kUneven
   static constexpr size_t frag_bytes = (size_t)NT * 1024 * (2 * FULL * taps + 3 * REM_NQ);
-  static constexpr size_t wide_off = frag_bytes + NT * 16 * sizeof(float);
-  static constexpr size_t packed_bytes = wide_off + (NT + 3) / 4 * 16;
+  static constexpr size_t flag_off = frag_bytes + NT * 16 * sizeof(float);
+  static constexpr size_t packed_bytes = flag_off + (NT + 3) / 4 * 16;
 };
+enum RowFlag { kWide = 1, kUneven = 2 };
 
 // Reduction step q of the packed weights, lane group lgrp: the tap and the
 // first channel of its eight (c0 < 0: padding).  The first FULL * taps steps
@@ -114,18 +115,21 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
 #pragma unroll 8
     for (int i = tid & 15; i < C * Cfg::taps; i += 16) {
       const float v = at(row, i / Cfg::taps, i % Cfg::taps);
-      r.add(v, v);
+      r.add_largest(v, v);
+      r.add_least(v, v);
+      r.add_nonzero(v, v);
     }
   }
   unsigned mx = r.largest();
   for (int o = 1; o < 16; o <<= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 16));
-  const bool wide = __syncthreads_or(r.fails(split_exp(mx)));
+  const bool wide = __syncthreads_or(mx >= 242u << 23 || r.apart(split_exp(mx)));
+  const bool uneven = __syncthreads_or(r.uneven(mx));
   if ((tid & 15) == 0) {
     exps[tid >> 4] = wide ? 127 : split_exp(mx);
     if (blockIdx.y == 0)
       reinterpret_cast<float*>(out + Cfg::frag_bytes)[row] = wide ? 1.f : __uint_as_float((unsigned)split_exp(mx) << 23);
   }
-  if (blockIdx.y == 0 && tid == 0) reinterpret_cast<int*>(out + Cfg::wide_off)[t] = wide;
+  if (blockIdx.y == 0 && tid == 0) reinterpret_cast<int*>(out + Cfg::flag_off)[t] = wide ? kWide : uneven ? kUneven : 0;
   __syncthreads();
   for (int u = blockIdx.y * 256 + tid; u < Cfg::NQ * 64; u += kPackShares * 256) {
     const int q = u >> 6, lane = u & 63, n = 16 * t + (lane & 15);
@@ -192,11 +196,11 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   if (tile >= tiles) return;  // (uniform) the grid is rounded up to 8 runs
   const int h0 = (tile / tiles_x) * Cfg::TH, w0 = (tile % tiles_x) * Cfg::TW;
   if (tid == 0) *reinterpret_cast<u32x4*>(lds + Cfg::zero_off) = u32x4{0u, 0u, 0u, 0u};
-  bool fails = false;  // an input of this lane is not held by its pair
-  int wide_rows = 0;
+  bool fails = false;  // an input of this lane needs float32 products
+  int flags = 0;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) wide_rows |= reinterpret_cast<const int*>(wpk + Cfg::wide_off)[t];
-  bool again = wide_rows != 0;  // (uniform) the tile takes float32 products
+  for (int t = 0; t < NT; ++t) flags |= reinterpret_cast<const int*>(wpk + Cfg::flag_off)[t];
+  bool again = flags & kWide;  // (uniform) the tile takes float32 products
 
   // Stage of G groups from channel group cg0: unit (pixel, group) of eight
   // channels, all loads issued before the first is split and stored.
@@ -230,9 +234,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         };
         BlockRange r;
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) r.add(f[e], f[e + 1]);
+        for (int e = 0; e < 8; e += 2) r.add_largest(f[e], f[e + 1]);
         const int eb = split_exp(quad_max(r.largest()));
-        fails |= r.fails(eb);
+        fails |= r.huge();
+        if (flags & kUneven) {  // (uniform)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) r.add_nonzero(f[e], f[e + 1]);
+          fails |= r.apart(eb);
+        }
         const unsigned neg = (unsigned)(px / AC + px % AC) << 31;  // (a checkerboard of signs: see kNegate)
         f16x8 p[2];
         split_pair(f, with_sign(split_scale(eb), neg), p[0], p[1]);
@@ -246,8 +255,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         bf16 p[3][8];
         BlockRange r;
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) r.add(f[e], f[e + 1]);
-        fails |= r.fails(29);  // (only the largest values: no scale is shared)
+        for (int e = 0; e < 8; e += 2) r.add_largest(f[e], f[e + 1]);
+        fails |= r.huge();
         split3(f, p[0], p[1], p[2]);
         if (v < NU) {
 #pragma unroll
@@ -433,7 +442,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   // replaced), and rare.
   const f32x4* rows = reinterpret_cast<const f32x4*>(wpk + Cfg::frag_bytes);
   auto float_tile = [&]() {
-    const int* wide = reinterpret_cast<const int*>(wpk + Cfg::wide_off);
+    const int* flag = reinterpret_cast<const int*>(wpk + Cfg::flag_off);
     const float* scale = reinterpret_cast<const float*>(rows) + lrow;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -461,7 +470,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         if (ql < 0) {
           const u32x4* p = reinterpret_cast<const u32x4*>(wpk + (long)(q * NT + t) * 2048) + lane;
           const u32x4 p0 = p[0], p1 = p[64];
-          if (wide[t]) {  // (uniform)
+          if (flag[t] & kWide) {  // (uniform)
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(e < 4 ? p0[e & 3] : p1[e & 3]);
           } else {

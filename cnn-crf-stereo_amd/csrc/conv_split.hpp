@@ -86,31 +86,53 @@ __device__ __forceinline__ float with_sign(float x, unsigned sign) {  // x, nega
 // products with a low term are summed apart from those without.  No value of the
 // block may be infinite.
 constexpr float kLowUnit = 4096.f;
+__device__ __forceinline__ void split_value(float x, float s, _Float16& h, _Float16& l) {
+  const float v = x * s;
+  h = (_Float16)v;
+  l = (_Float16)fmaf((float)h, -kLowUnit, v * kLowUnit);
+}
 __device__ __forceinline__ void split_pair(const float (&x)[8], float s, f16x8& h, f16x8& l) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float v = x[e] * s;
-    h[e] = (_Float16)v;
-    l[e] = (_Float16)fmaf((float)h[e], -kLowUnit, v * kLowUnit);
+    _Float16 a, b;
+    split_value(x[e], s, a, b);
+    h[e] = a;
+    l[e] = b;
   }
 }
 
-// The largest |x| of a block and the smallest that is not 0, as ordered bits, one
-// instruction per value for the smallest and half of one for the largest: above,
-// |x| (a NaN is passed over), below, 2 |x| - 2, which makes 0 the largest.
+// What a pair leaves out of a value below 2^-29 of its block's largest is 2^-52 of
+// that largest, and the low products that are dropped are 2^-50 of the largest product.
+// That is nothing beside the largest value's own product, unless this meets a zero or
+// a very small factor: where all factors of a sum are within 2^-22 of their largest
+// (even), 32 such values leave out 2^-23 of the sum's terms at most.  So a sum needs other
+// products than the pairs' only where one side has values that far apart and the other
+// is uneven.
+//
+// BlockRange collects what tells: the largest |x| of a block, the smallest (as ordered
+// bits, one instruction per two values each; a NaN is passed over: both its terms
+// are NaN), and the smallest that is not 0 (as 2 |x| - 2, which makes 0 the largest).
 struct BlockRange {
-  float above = 0.f;
+  float above = 0.f, least = __builtin_huge_valf();
   unsigned below = ~0u;
-  __device__ __forceinline__ void add(float x, float y) {
+  __device__ __forceinline__ void add_largest(float x, float y) {
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(above) : "v"(x), "v"(y));
+  }
+  __device__ __forceinline__ void add_least(float x, float y) {
+    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least) : "v"(x), "v"(y));
+  }
+  __device__ __forceinline__ void add_nonzero(float x, float y) {
     below = min(below, min((__float_as_uint(x) << 1) - 2u, (__float_as_uint(y) << 1) - 2u));
   }
   __device__ __forceinline__ unsigned largest() const { return __float_as_uint(above); }
-  // Whether split_pair does not hold a value of the block, or its sums of products may
-  // leave float32's range before their scales are taken back (from 2^115).  eb: the
-  // block's split_exp.  A NaN is held: both terms are NaN.
-  __device__ __forceinline__ bool fails(int eb, unsigned huge = 242u << 23) const {
-    return largest() >= huge || below < (unsigned)(eb - 29) << 24;
+  // Sums of products may leave float32's range before their scales are taken back
+  // (from 2^115), or a value is infinite.
+  __device__ __forceinline__ bool huge(unsigned from = 242u << 23) const { return largest() >= from; }
+  // A value that is not 0 is below 2^-29 of the block's largest; eb: its split_exp.
+  __device__ __forceinline__ bool apart(int eb) const { return below < (unsigned)(eb - 29) << 24; }
+  // A value, 0 or not, is below 2^-22 of the block's largest (its ordered bits).
+  __device__ __forceinline__ bool uneven(unsigned block) const {
+    return __float_as_int(least) < (int)block - (22 << 23);
   }
 };
 

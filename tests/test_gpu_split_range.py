@@ -62,11 +62,26 @@ def test_layer(handle, C, k, case):
     check(y[:, :, :C].permute(2, 0, 1).double().cpu().numpy().reshape(C, -1), ref.reshape(C, -1))
 
 
+@pytest.mark.parametrize("C,k", [(100, 3), (100, 2), (64, 3)])
+def test_layer_of_values_apart(handle, C, k):
+    """Values of any sizes side by side, weights of one size: every output pixel is
+    off by a share of its own size."""
+    rng = np.random.default_rng(2 * C + k)
+    x = (uniform(rng, C, 20, 37) * 10.0 ** rng.uniform(-20, 10, (C, 20, 37))).astype(np.float32)
+    w = uniform(rng, C, C, k, k).astype(np.float32)
+    hwc = torch.zeros((20, 37, capi.feature_stride(C)), device="cuda")
+    hwc[:, :, :C] = torch.as_tensor(x, device="cuda").permute(1, 2, 0)
+    y = ops.ConvLayer(handle, w, None, "fp32", act=False)(handle, hwc)[:, :, :C].double().cpu().numpy().reshape(-1, C)
+    ref = F.conv2d(torch.as_tensor(x).double()[None], torch.as_tensor(w).double().flip(2, 3))[0].numpy()
+    check(y, ref.reshape(C, -1).T)
+
+
 def test_layer_pixels_apart(handle):
-    """A pixel out of range leaves the outputs that it does not reach to the bit as
-    they are in another tile, and takes the others' tile to float32 products."""
+    """A pixel out of range takes its tile to float32 products and leaves the other
+    tiles' outputs as they are, to the bit."""
     rng = np.random.default_rng(0)
     x, w = layer_case(rng, "", 100, 3)
+    w[3, 4] = 0
     layer = ops.ConvLayer(handle, w, None, "fp32")
     hwc = torch.zeros((20, 37, 104), device="cuda")
     hwc[:, :, :100] = torch.as_tensor(x, device="cuda").permute(1, 2, 0)
