@@ -1,8 +1,9 @@
 // Weight gradient of the 100-channel layers on the 16-bit matrix cores:
 //   dW[tap][k][c] = sum over output pixels p of dz[p][k] x[p + tap][c]
 // for bfloat16 maps and float32 maps (two float16 terms per operand with a scale
-// per channel and segment, three products summed from zero per segment, as
-// conv_split.hip).
+// per channel and segment, three products in two sums from zero per segment, as
+// conv_split.hip; a segment in which that does not do, see BlockRange, takes
+// v_mfma_f32_16x16x4_f32 from memory after the others).
 //
 // k_dw_split: a workgroup takes one tap row i (its KW taps) and a chunk of
 // SEG-pixel segments of output rows; each of its seven waves owns 16 channels of
@@ -20,7 +21,8 @@
 // zeros past a row's end selected beside the loads, which waited for each segment's
 // reads -> now): bf16 3x3 at 524 x 268 190 -> 112 -> 94 us, at 1488 x 992
 // 1490 -> 949 -> 708 us; float32 3x3 at 524 x 268 473 -> 328 -> 263 us (301 with
-// three bfloat16 terms and six products).  Two input halves per chunk on four-wave
+// three bfloat16 terms and six products), and 271 with both units and the range tests
+// (850 where every segment goes to float32 products).  Two input halves per chunk on four-wave
 // workgroups, two or three per CU, measured the same as one (110, 990, 357 us): they
 // read dz twice as often.
 //
@@ -52,8 +54,14 @@ struct DwCfg {
   static constexpr int plane = CP * PITCH * 2;  // bytes
   static constexpr int scales = 2 * PLANES * plane;  // float32: a scale per channel of dz, then of the input
   static constexpr int buffer = scales + (kF32 ? 2 * CP * 4 : 0);
-  static constexpr int lds_bytes = 2 * buffer;
+  // float32: per buffer and wave the DwFlags of its units, then a bit per segment of the chunk
+  static constexpr int flag_off = 2 * buffer, float_off = flag_off + 2 * 8 * 4;
+  static constexpr int lds_bytes(long spc) { return kF32 ? float_off + (int)((spc + 127) / 128) * 16 : 2 * buffer; }
 };
+
+// What the channels of a segment's input (X) and dz (Z) have: values of 2^64 and more, with
+// which the product of two channels' scales may be infinite; uneven() ones; apart() ones.
+enum DwFlag { kUnevenX = 1, kUnevenZ = 2, kApartX = 4, kApartZ = 8, kHuge = 16 };
 
 template <typename T, int KW>
 __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __restrict__ x, int Win, int Csx,
@@ -72,7 +80,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   const int k0 = 16 * wave;
   const long s0 = (long)chunk * spc;
   const long s1 = s0 + spc < nseg ? s0 + spc : nseg;
-  for (int i = tid; i < Cfg::lds_bytes / 16; i += Cfg::THREADS)  // the pad channels stay zero
+  for (int i = tid; i < Cfg::lds_bytes(spc) / 16; i += Cfg::THREADS)  // the pad channels stay zero
     reinterpret_cast<u32x4*>(lds)[i] = u32x4{0u, 0u, 0u, 0u};
 
   // This lane's units: block 0-3 dz, 4-7 the input row, 8 the input row's last
@@ -128,6 +136,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
     }
   };
   auto store = [&](int buf) {
+    int flags = 0;  // float32: the units' DwFlags (uniform over the wave)
 #pragma unroll
     for (int n = 0; n < Cfg::NU; ++n) {
       const int b = wave + NT * n;
@@ -135,54 +144,71 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       const Unit u = unit(b);
       if (!Cfg::kF32 && !u.ok) continue;
       const int left = (u.z ? Wo : Win) - wo_loaded;
-      if (left < SEG + 4) {  // (uniform) the row may end in this segment
+      // Fills the pixels past the row's end, if it is in this segment (uniform).
+      auto fill_end = [&](unsigned v) {
+        if (left >= SEG + 4) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (4 * u.q + i >= left) reg[n][i] = u32x4{0u, 0u, 0u, 0u};
+          if (4 * u.q + i >= left) reg[n][i] = u32x4{v, v, v, v};
         if constexpr (Cfg::kF32) {
 #pragma unroll
           for (int i = 0; i < 2; ++i)
-            if (SEG + i >= left) ext[n][i] = u32x4{0u, 0u, 0u, 0u};
+            if (SEG + i >= left) ext[n][i] = u32x4{v, v, v, v};
         }
-      }
-      unsigned char* d =
-          lds + buf * Cfg::buffer + (u.z ? 0 : PLANES * Cfg::plane) + (u.g * VE * PITCH + 4 * u.q) * 2;
+      };
+      [[maybe_unused]] auto at = [&](int e, int i) {
+        return __uint_as_float(i < 4 ? reg[n][i][e] : ext[n][i - 4][e]);
+      };
+      [[maybe_unused]] int eb[4];
       if constexpr (Cfg::kF32) {
         // Four pixels and the two past the segment of four channels; the eight
         // lanes of a group agree on each channel's scale.
-        unsigned mx[4], all = 0;
-        auto bits = [&](int e, int i) { return i < 4 ? reg[n][i][e] : ext[n][i - 4][e]; };
+        fill_end(0x7fc00000u);  // (a NaN, which the ranges pass over)
+        unsigned long huge = 0, uneven = 0, apart = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          mx[e] = 0;
+          BlockRange r;
 #pragma unroll
-          for (int i = 0; i < 6; ++i)
-            if (i < 4 || !u.z) mx[e] = max(mx[e], bits(e, i) & 0x7fffffffu);
-          all = max(all, mx[e]);
+          for (int i = 0; i < 6; i += 2) {
+            if (i >= 4 && u.z) break;
+            r.add_largest(at(e, i), at(e, i + 1));
+            r.add_least(at(e, i), at(e, i + 1));
+          }
+          unsigned mx = r.largest();
+          mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0xb1, 0xf, 0xf, true));
+          mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0x4e, 0xf, 0xf, true));
+          mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0x141, 0xf, 0xf, true));  // row_half_mirror
+          eb[e] = split_exp(mx);
+          huge |= __ballot(u.ok && r.huge(191u << 23));
+          uneven |= __ballot(u.ok && r.uneven(mx));
         }
-        const bool finite = !__any(all >= 0x7f800000u);
+        if (uneven) {  // (uniform; a value that is apart is uneven too)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            BlockRange r;
+#pragma unroll
+            for (int i = 0; i < 6; i += 2) {
+              if (i >= 4 && u.z) break;
+              r.add_nonzero(at(e, i), at(e, i + 1));
+            }
+            apart |= __ballot(u.ok && r.apart(eb[e]));
+          }
+        }
+        flags |= (huge ? kHuge : 0) | (uneven ? u.z ? kUnevenZ : kUnevenX : 0) | (apart ? u.z ? kApartZ : kApartX : 0);
+      }
+      fill_end(0u);
+      unsigned char* d =
+          lds + buf * Cfg::buffer + (u.z ? 0 : PLANES * Cfg::plane) + (u.g * VE * PITCH + 4 * u.q) * 2;
+      if constexpr (Cfg::kF32) {
         const unsigned neg = u.z && buf ? kNegate : 0u;  // every other segment's dz
         const unsigned scale0 = (268u << 23) + neg, unscale0 = u.z ? neg - (28u << 23) : 0u;
         f32x4 unscale;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (!finite) {
-            mx[e] = 0;
-#pragma unroll
-            for (int i = 0; i < 6; ++i)
-              if (i < 4 || !u.z) mx[e] = max(mx[e], finite_bits(__uint_as_float(bits(e, i))));
-#pragma unroll
-            for (int i = 0; i < 4; ++i)  // (a value that the scale does not reach)
-              if ((reg[n][i][e] & 0x7fffffffu) >= 0x7f800000u) reg[n][i][e] ^= neg;
-          }
-          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0xb1, 0xf, 0xf, true));
-          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x4e, 0xf, 0xf, true));
-          mx[e] = max(mx[e], (unsigned)__builtin_amdgcn_mov_dpp((int)mx[e], 0x141, 0xf, 0xf, true));  // row_half_mirror
-          const int eb = split_exp(mx[e]);
           // split_scale and split_unscale (x's side: 2^(eb - 127)) with the sign,
           // which is carried through by sums modulo 2^32
-          const float sc = __uint_as_float(scale0 - ((unsigned)eb << 23));
-          unscale[e] = __uint_as_float(((unsigned)eb << 23) + unscale0);
+          const float sc = __uint_as_float(scale0 - ((unsigned)eb[e] << 23));
+          unscale[e] = __uint_as_float(((unsigned)eb[e] << 23) + unscale0);
           typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
           typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
           f16x4 hi, lo;
@@ -190,10 +216,8 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
 #pragma unroll
           for (int i = 0; i < 6; ++i) {
             if (i >= 4 && u.z) break;
-            const float f = __uint_as_float(bits(e, i));
-            const bool fin = finite || (__float_as_uint(f) & 0x7fffffffu) < 0x7f800000u;
-            const float v = fin ? f * sc : 0.f;
-            const _Float16 h = (_Float16)v, l = (_Float16)(fin ? v - (float)h : f);
+            _Float16 h, l;
+            split_value(at(e, i), sc, h, l);
             if (i < 4) hi[i] = h, lo[i] = l;
             else hx[i - 4] = h, lx[i - 4] = l;
           }
@@ -217,6 +241,9 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
                     __builtin_amdgcn_perm(reg[n][3][e >> 1], reg[n][2][e >> 1], sel)};
         }
       }
+    }
+    if constexpr (Cfg::kF32) {
+      if (lane == 0) *reinterpret_cast<int*>(lds + Cfg::flag_off + (8 * buf + wave) * 4) = flags;
     }
   };
 
@@ -272,7 +299,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
         if constexpr (Cfg::kF32) both = sz * sx;
         if (t + 1 < NT) read_x(t + 1);
         __builtin_amdgcn_sched_barrier(0);
-        f32x4 c[KW];
+        f32x4 c[KW], low[KW];  // low (float32): the products with a low term
 #pragma unroll
         for (int j = 0; j < KW; ++j) c[j] = Cfg::kF32 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j][t];
         auto mm = [&](int ka, int kb) {
@@ -288,19 +315,29 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
         if constexpr (Cfg::kF32) {
           mm(PLANES - 1, 0);
           mm(0, PLANES - 1);
+#pragma unroll
+          for (int j = 0; j < KW; ++j) low[j] = c[j], c[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         mm(0, 0);
 #pragma unroll
         for (int j = 0; j < KW; ++j) {
           if constexpr (Cfg::kF32) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[j][t][e] = fmaf(c[j][e], both[e], acc[j][t][e]);
+            for (int e = 0; e < 4; ++e)
+              acc[j][t][e] = fmaf(fmaf(low[j][e], 1.f / kLowUnit, c[j][e]), both[e], acc[j][t][e]);
           } else {
             acc[j][t] = c[j];
           }
         }
       }
     }
+  };
+
+  auto failed = [&](int buf) {  // (behind the barrier)
+    const u32x4* f = reinterpret_cast<const u32x4*>(lds + Cfg::flag_off + 8 * buf * 4);
+    const u32x4 a = f[0], b = f[1];
+    const int any = __builtin_amdgcn_readfirstlane(a[0] | a[1] | a[2] | a[3] | b[0] | b[1] | b[2]);
+    return (any & kHuge) || ((any & kApartX) && (any & kUnevenZ)) || ((any & kApartZ) && (any & kUnevenX));
   };
 
   __syncthreads();  // the zero fill is done
@@ -323,9 +360,49 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       }
     };
     if (Cfg::kF32 || wave < 4) stage();
+    if constexpr (Cfg::kF32) {
+      if (failed(buf)) {  // its products become zeros (a branch around multiply() spills)
+        if (tid == 0) reinterpret_cast<unsigned*>(lds + Cfg::float_off)[(s - s0) >> 5] |= 1u << ((s - s0) & 31);
+        for (int i = tid; i < Cfg::buffer / 16; i += Cfg::THREADS)
+          reinterpret_cast<u32x4*>(lds + buf * Cfg::buffer)[i] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+      }
+    }
     multiply(buf);
     if (!Cfg::kF32 && wave >= 4) stage();
     __syncthreads();
+  }
+  if constexpr (Cfg::kF32) {
+    // The segments left out, on v_mfma_f32_16x16x4_f32 with operands from memory (here,
+    // where the staged values are dead: beside multiply() this spills).
+    for (long w0 = s0; w0 < s1; w0 += 32) {
+      unsigned bits = __builtin_amdgcn_readfirstlane(reinterpret_cast<unsigned*>(lds + Cfg::float_off)[(w0 - s0) >> 5]);
+      for (; bits; bits &= bits - 1) {
+        const long s = w0 + __builtin_ctz(bits);
+        const int ho = (int)(s / segs_per_row), wo0 = (int)(s % segs_per_row) * SEG;
+        const T* zrow = dz + ((long)ho * zpitch + wo0) * Csk;
+        const T* xrow = x + ((long)(ho + ti) * Win + wo0) * Csx;
+        const int left = min(SEG, Wo - wo0);
+#pragma unroll 1
+        for (int p0 = 0; p0 < left; p0 += 4) {
+          // Past the row and the channels another value is loaded (no branches); those
+          // channels' sums are not used.
+          const int p = min(p0 + lgrp, left - 1);
+          const bool in = p0 + lgrp < left;
+          const float zv = in ? (float)zrow[p * Csk + min(k0 + lrow, Csk - 1)] : 0.f;
+          float xv[KW][NT];
+#pragma unroll
+          for (int j = 0; j < KW; ++j)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) xv[j][t] = (float)xrow[(p + j) * Csx + min(16 * t + lrow, Csx - 1)];
+#pragma unroll
+          for (int j = 0; j < KW; ++j)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(zv, in ? xv[j][t] : 0.f, acc[j][t], 0, 0, 0);
+        }
+      }
+    }
   }
 #pragma unroll
   for (int j = 0; j < KW; ++j) {
@@ -349,8 +426,9 @@ static void launch(const DwArgs& a, int KH, int KW, hipStream_t st) {
   const unsigned blocks = (unsigned)(8 * KH * ((a.nch + 7) / 8));
   auto go = [&](auto kwc) {
     const auto kern = k_dw_split<T, decltype(kwc)::value>;
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::lds_bytes);
-    kern<<<blocks, Cfg::THREADS, Cfg::lds_bytes, st>>>((const T*)a.x, a.Win, a.Csx, (const T*)a.dz, a.zpitch, a.Ho,
+    const int lds = Cfg::lds_bytes(a.spc);
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    kern<<<blocks, Cfg::THREADS, lds, st>>>((const T*)a.x, a.Win, a.Csx, (const T*)a.dz, a.zpitch, a.Ho,
                                                       a.Wo, a.Csk, KH, a.nch, a.segs_per_row, a.nseg, a.spc, a.part);
   };
   if (KW == 3) go(std::integral_constant<int, 3>{});

@@ -89,3 +89,43 @@ def test_layer_pixels_apart(handle):
     hwc[2, 3, 7] = 1e-30
     got = layer(handle, hwc)
     assert torch.equal(got[8:], want[8:]) and torch.equal(got[:, 16:], want[:, 16:])
+
+
+DW_CASES = ["one pixel 1e8", "one pixel 1e12", "one dz 1e9", "both", "columns", "huge", "tiny"]
+
+
+@pytest.mark.parametrize("case", DW_CASES)
+@pytest.mark.parametrize("k", [3, 2])
+def test_weight_gradient(handle, case, k):
+    """Pixels of one segment: a large one of the input meets a zero of dz and the reverse."""
+    rng = np.random.default_rng(k)
+    C, H, W = 100, 12, 70
+    Ho, Wo = H - k + 1, W - k + 1
+    x, dz = uniform(rng, H, W, C), 1e-3 * uniform(rng, Ho, Wo, C)
+    if case.startswith("one pixel") or case == "both":
+        f = float(case.split()[-1]) if case != "both" else 1e12
+        dz[4:4 + k, 8:8 + k] = 0
+        x[4 + k - 1, 8 + k - 1] *= f
+    if case.startswith("one dz") or case == "both":
+        f = float(case.split()[-1]) if case != "both" else 1e12
+        x[7:7 + k, 20:20 + k] = 0
+        dz[7, 20] *= f
+    if case == "columns":  # columns of the map in units of their own, alike products at the first column of taps
+        unit = 10.0 ** rng.uniform(-12, 12, (1, W, 1))
+        x, dz = x * unit, dz / unit[:, :Wo]
+    if case == "huge":
+        x, dz = x * 1e30, dz * 1e5
+    if case == "tiny":
+        x, dz = x * 1e-12, dz * 1e-12
+    maps = []
+    for m in (x, dz):
+        t = torch.zeros((*m.shape[:2], 104), device="cuda")
+        t[:, :, :C] = torch.as_tensor(m, device="cuda")
+        maps.append(t)
+    w = torch.zeros((C, C, k, k), device="cuda")
+    _, dw, _ = ops.conv2d_backward_stored(handle, maps[0], torch.zeros_like(maps[1]), w, maps[1], act=False)
+    xd, zd = (m[:, :, :C].double().cpu() for m in maps)
+    ref = torch.stack([zd.reshape(-1, C).t() @ xd[k - 1 - a:k - 1 - a + Ho, k - 1 - b:k - 1 - b + Wo].reshape(-1, C)
+                       for a in range(k) for b in range(k)], dim=2).numpy()
+    per_tap = lambda v: v.transpose(0, 2, 3, 1).reshape(-1, C)  # noqa: E731
+    check(per_tap(dw.double().cpu().numpy()), per_tap(ref.reshape(C, C, k, k)))
