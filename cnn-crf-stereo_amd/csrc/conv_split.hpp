@@ -48,15 +48,6 @@ __device__ __forceinline__ void split3(const float (&x)[N], bf16 (&h)[N], bf16 (
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 
-// x s = h + l in float16 with one rounding, for a power of two s that takes the
-// largest |x| of a block to [2^14, 2^15): h is x s rounded to nearest, l the
-// rest rounded to nearest.  What is left out is at most 2^-24 |x|, and never
-// more than 2^-39 of the block's largest value (float16's subnormals are exact
-// in the matrix core).  An infinity or a NaN goes to l alone, as in split3.
-__device__ __forceinline__ unsigned finite_bits(float x) {  // |x| as ordered bits, 0 where it is not finite
-  const unsigned b = __float_as_uint(x) & 0x7fffffffu;
-  return b < 0x7f800000u ? b : 0u;
-}
 // A block's biased exponent from its largest |x| bits (from 29, so that the
 // factors below are normal numbers: smaller blocks keep a share of the bits).
 __device__ __forceinline__ int split_exp(unsigned mx) { return max((int)(mx >> 23), 29); }
@@ -78,13 +69,13 @@ __device__ __forceinline__ float with_sign(float x, unsigned sign) {  // x, nega
   return __uint_as_float(__float_as_uint(x) ^ sign);
 }
 
-// x s = h + l / kLowUnit in float16, as split2, but the rest is scaled up to h's
-// size before it is rounded, so that it stays a normal number for values down to
-// 2^-29 of the block's largest: what is left out is at most 2^-22 |x| for those and
-// 2^-24 |x| down to 2^-16.  (In one unit, the rest of a value below 2^-15 of the largest
-// is a subnormal number or lost: uneven channels of one pixel came out wrong.)  The
-// products with a low term are summed apart from those without.  No value of the
-// block may be infinite.
+// x s = h + l / kLowUnit in float16, for a power of two s that takes the largest |x| of
+// a block to [2^14, 2^15): h is x s rounded to nearest, l the rest, scaled up to h's size
+// and rounded to nearest.  (float16's subnormals are exact in the matrix core.)  What is
+// left out is at most 2^-24 |x| down to 2^-16 of the block's largest and 2^-22 |x| down
+// to 2^-29; with the rest in h's own unit it is a subnormal number below 2^-15 of the
+// largest, and lost below 2^-39.  The products with a low term are summed apart from
+// those without.  No value of the block may be infinite.
 constexpr float kLowUnit = 4096.f;
 __device__ __forceinline__ void split_value(float x, float s, _Float16& h, _Float16& l) {
   const float v = x * s;
@@ -135,18 +126,5 @@ struct BlockRange {
     return __float_as_int(least) < (int)block - (22 << 23);
   }
 };
-
-template <bool FINITE>  // every value is finite
-__device__ __forceinline__ void split2(const float (&x)[8], float s, f16x8& h, f16x8& l) {
-  float v[8], r[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const bool fin = FINITE || (__float_as_uint(x[e]) & 0x7fffffffu) < 0x7f800000u;
-    v[e] = fin ? x[e] * s : 0.f;
-    h[e] = (_Float16)v[e];
-    r[e] = fin ? v[e] - (float)h[e] : x[e];
-    l[e] = (_Float16)r[e];
-  }
-}
 
 }  // namespace ccs

@@ -38,29 +38,38 @@ struct CorrArgs {
 };
 
 // float32 maps: the same product on the float16 matrix cores.  Features are split
-// into two float16 terms (split2) with one power-of-two scale per pixel and stage
-// of 32 channels; a stage's three products are summed from zero and taken into
-// the accumulators with both pixels' scales.  Only the stage is held in LDS (132
+// into two float16 terms (split_pair) with one power-of-two scale per pixel and stage
+// of 32 channels; a stage's three products are summed from zero, those with a low
+// term apart, and taken into the accumulators with both pixels' scales.  A stage in
+// which that does not do (BlockRange) takes v_mfma_f32_16x16x4_f32 from memory.
+// Only the stage is held in LDS (132
 // bytes per pixel and window column instead of 420 for the whole float32 row of
 // 100 channels), so two or three workgroups share a CU and their phases overlap;
 // the next stage's loads are in flight under the products.  Bound by the volume's
 // store and the softmax.  Measured (us, v_mfma_f32_16x16x4_f32 kernel with whole
-// pixels in LDS -> this): 320 x 240 D = 32 37 -> 27, 744 x 496 D = 64 229 -> 124,
-// 512 x 256 D = 128 97 -> 62, 1242 x 375 D = 128 344 -> 211, 1488 x 992 D = 256
-// 2807 -> 1366 (1.14 TB/s of volume), 96 x 64 D = 16 14 -> 13.
+// pixels in LDS -> both terms in one unit -> this; in float32 products throughout): 320
+// x 240 D = 32 37 -> 27 -> 28 (50), 744 x 496 D = 64 222 -> 122 -> 131 (278), 512 x 256
+// D = 128 95 -> 62 -> 65 (131), 1242 x 375 D = 128 332 -> 211 -> 222 (493), 1488 x 992
+// D = 256 2800 -> 1245 -> 1325 (3400).
 template <int NTM>
 struct CorrSplit {
   static constexpr int NW = NTM > 9 ? 4 : 8, TW = 16 * NW, WIN = 16 * (NW - 1) + 16 * NTM, NPX = TW + WIN;
   static constexpr int SP = 16 * NTM + 3;  // as CorrArgs::sp
   static constexpr int THREADS = 64 * NW, PER = (NPX * 4 + THREADS - 1) / THREADS;
   static constexpr int plane = NPX * 64, scale_off = 2 * plane;
-  static constexpr int feat = scale_off + NPX * 4, sbytes = NW * 16 * SP * 4;
+  static constexpr int flag_off = scale_off + NPX * 4;  // per wave: CorrFlags of the units it staged
+  static constexpr int feat = flag_off + 8 * 4, sbytes = NW * 16 * SP * 4;
   static constexpr int stats_off = ((feat > sbytes ? feat : sbytes) + 15) / 16 * 16;
   static constexpr int lds_bytes = stats_off + NW * 16 * 4;
 };
 
+// What the blocks of a map's pixels in a stage have: values of 2^64 and more, with which
+// the product of two pixels' scales may be infinite; uneven() ones, apart() ones.
+enum CorrFlag { kUneven0 = 1, kUneven1 = 2, kApart0 = 4, kApart1 = 8, kHuge = 16 };
+
+// (float32, NTM 9: the registers of two workgroups of 8 waves per CU)
 template <typename T, int NTM>
-__global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
+__global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_corr_volume(CorrArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int NW = blockDim.x >> 6;
   const int TW = 16 * NW;
@@ -143,31 +152,37 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
       }
     };
     auto store = [&](int st) {
+      unsigned long huge = 0, uneven0 = 0, uneven1 = 0, apart0 = 0, apart1 = 0;
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         const int v = tid + Cfg::THREADS * i, px = v >> 2, g = v & 3, col = column(px);
         const bool ok = 4 * st + g < cg && col >= 0 && col < a.W;
         float f[8];
-        unsigned mx = 0;
+        BlockRange range;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          f[e] = ok ? r[i][e >> 2][e & 3] : 0.f;
-          mx = max(mx, __float_as_uint(f[e]) & 0x7fffffffu);
-        }
-        const bool finite = !__any(mx >= 0x7f800000u);
-        if (!finite) {
-          mx = 0;
+        for (int e = 0; e < 8; ++e) f[e] = ok ? r[i][e >> 2][e & 3] : 0.f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) mx = max(mx, finite_bits(f[e]));
+        for (int e = 0; e < 8; e += 2) {
+          range.add_largest(f[e], f[e + 1]);
+          range.add_least(f[e], f[e + 1]);
         }
+        unsigned mx = range.largest();
         mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0xb1, 0xf, 0xf, true));
         mx = max(mx, (unsigned)__builtin_amdgcn_mov_dpp((int)mx, 0x4e, 0xf, 0xf, true));
         const int eb = split_exp(mx);
+        huge |= __ballot(range.huge(191u << 23));
+        const unsigned long uneven = __ballot(ok && range.uneven(mx));
+        if (uneven) {  // (uniform; a value that is apart is uneven too)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) range.add_nonzero(f[e], f[e + 1]);
+          const unsigned long first = __ballot(px < TW), apart = __ballot(range.apart(eb));
+          uneven0 |= uneven & first;
+          uneven1 |= uneven & ~first;
+          apart0 |= apart & first;
+          apart1 |= apart & ~first;
+        }
         f16x8 p[2];
-        if (finite)
-          split2<true>(f, split_scale(eb), p[0], p[1]);
-        else
-          split2<false>(f, split_scale(eb), p[0], p[1]);
+        split_pair(f, split_scale(eb), p[0], p[1]);
         if (v < NPX * 4) {
           const int off = px * 64 + swz(px, g);
 #pragma unroll
@@ -177,15 +192,60 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
                 px < TW ? split_unscale(eb) : __uint_as_float((unsigned)eb << 23);
         }
       }
+      if (lane == 0)
+        *reinterpret_cast<int*>(lds + Cfg::flag_off + 4 * wave) = (huge ? kHuge : 0) | (uneven0 ? kUneven0 : 0) |
+                                                                  (uneven1 ? kUneven1 : 0) | (apart0 ? kApart0 : 0) |
+                                                                  (apart1 ? kApart1 : 0);
+    };
+    auto failed = [&]() {  // (behind the barrier)
+      const int* f = reinterpret_cast<const int*>(lds + Cfg::flag_off);
+      int any = 0;
+#pragma unroll
+      for (int w = 0; w < Cfg::NW; ++w) any |= f[w];
+      any = __builtin_amdgcn_readfirstlane(any);
+      return (any & kHuge) || ((any & kApart0) && (any & kUneven1)) || ((any & kApart1) && (any & kUneven0));
+    };
+    // Stage st on v_mfma_f32_16x16x4_f32, operands from memory.
+    auto float_stage = [&](int st) {
+      const int g = 4 * st + lgrp;
+      const bool in = g < cg;
+      auto unit = [&](const T* row, int col, f32x4 (&o)[2]) {
+        const bool ok = in && col >= 0 && col < a.W;
+        const f32x4* src = reinterpret_cast<const f32x4*>(row + (long)(ok ? col : 0) * Cs + (ok ? 8 * g : 0));
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          o[k] = src[k];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[k][e] = ok ? o[k][e] : 0.f;
+        }
+      };
+      f32x4 av[2], bv[2];
+      unit(f0, w0 + arow, av);
+#pragma unroll
+      for (int t = 0; t < NTM; ++t) {
+        unit(f1, w0 + a.o_lo + 16 * wave + 16 * t + lrow, bv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e >> 2][e & 3], bv[e >> 2][e & 3], acc[t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     };
 
-    const int stages = (cg + 3) / 4;
+    const int stages = (cg + 3) / 4;  // 20 at most: wider pixels are refused
+    unsigned floats = 0;              // the stages left for float32 products
     load(0);
     for (int st = 0; st < stages; ++st) {
       if (st > 0) __syncthreads();  // the previous stage is read
       store(st);
       __syncthreads();
       if (st + 1 < stages) load(st + 1);
+      if (failed()) {  // its products become zeros (a branch around them takes 50 registers more)
+        floats |= 1u << st;
+        __syncthreads();  // the flags are read
+        for (int i = tid; i < (Cfg::scale_off + NPX * 4) / 16; i += Cfg::THREADS)
+          reinterpret_cast<u32x4*>(lds)[i] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+      }
       const float* scale = reinterpret_cast<const float*>(lds + Cfg::scale_off);
       auto frag = [&](int px, int k) {
         return *reinterpret_cast<const f16x8*>(lds + k * Cfg::plane + px * 64 + swz(px, lgrp));
@@ -197,13 +257,14 @@ __global__ __launch_bounds__(512) void k_corr_volume(CorrArgs a) {
         const int px = TW + 16 * wave + 16 * t + lrow;
         const f16x8 bh = frag(px, 0), bl = frag(px, 1);
         const float s1 = scale[px];
-        f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, c, 0, 0, 0);
+        f32x4 low = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        low = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, low, 0, 0, 0);
+        const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[t][e] = fmaf(c[e], s0[e] * s1, acc[t][e]);
+        for (int e = 0; e < 4; ++e) acc[t][e] = fmaf(fmaf(low[e], 1.f / kLowUnit, c[e]), s0[e] * s1, acc[t][e]);
       }
     }
+    for (; floats; floats &= floats - 1) float_stage(__builtin_ctz(floats));
   }
   // -softmax over the band, in the accumulators where the disparities are
   // consecutive columns: lane (lrow, lgrp) holds columns 16 t + lrow of pixels

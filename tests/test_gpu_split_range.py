@@ -129,3 +129,50 @@ def test_weight_gradient(handle, case, k):
                        for a in range(k) for b in range(k)], dim=2).numpy()
     per_tap = lambda v: v.transpose(0, 2, 3, 1).reshape(-1, C)  # noqa: E731
     check(per_tap(dw.double().cpu().numpy()), per_tap(ref.reshape(C, C, k, k)))
+
+
+CORR_CASES = ["one channel 1e8", "one channel 1e12", "one channel 1e30", "other map 1e9", "both", "units", "huge",
+              "tiny"]
+
+
+@pytest.mark.parametrize("case", CORR_CASES)
+@pytest.mark.parametrize("C,D", [(100, 32), (100, 128), (64, 64), (36, 200)])
+def test_correlation(handle, case, C, D):
+    rng = np.random.default_rng(C + D)
+    H, W = 2, 300
+    f0, f1 = uniform(rng, H, W, C), uniform(rng, H, W, C)
+    if case.startswith("one channel") or case == "both":
+        f0[:, :, 5] *= float(case.split()[-1]) if case != "both" else 1e12
+        f1[:, :, 5] = 0
+    if case.startswith("other map") or case == "both":
+        f1[:, :, 9] *= float(case.split()[-1]) if case != "both" else 1e12
+        f0[:, :, 9] = 0
+    if case == "units":
+        unit = 10.0 ** rng.uniform(-12, 12, C)
+        f0, f1 = f0 * unit, f1 / unit
+    if case == "huge":
+        f0, f1 = f0 * 1e26, f1 * 1e10
+    if case == "tiny":
+        f0, f1 = f0 * 1e-14, f1 * 1e-14
+    maps = []
+    for f in (f0, f1):
+        t = torch.zeros((H, W, capi.feature_stride(C)), device="cuda")
+        t[:, :, :C] = torch.as_tensor(f, device="cuda")
+        maps.append(t)
+    got = ops.correlation_volume(handle, maps[0], maps[1], C, 0, 1, D, epilogue="raw").double().cpu().numpy()
+    a, b = (m[:, :, :C].double().cpu().numpy() for m in maps)
+    ref = np.zeros((H, W, D))
+    for d in range(D):
+        ref[:, d:, d] = (a[:, d:] * b[:, :W - d]).sum(-1)
+    check(got.reshape(-1, D).T, ref.reshape(-1, D).T)
+
+
+def test_correlation_of_values_apart(handle):
+    """Values of any sizes in one map, of one size in the other."""
+    rng = np.random.default_rng(8)
+    f0 = torch.as_tensor(uniform(rng, 2, 300, 104) * 10.0 ** rng.uniform(-20, 10, (2, 300, 104)), dtype=torch.float32)
+    f1 = torch.as_tensor(uniform(rng, 2, 300, 104), dtype=torch.float32)
+    got = ops.correlation_volume(handle, f0.cuda(), f1.cuda(), 104, 0, 1, 64, epilogue="raw").double().cpu().numpy()
+    a, b = f0.double().numpy(), f1.double().numpy()
+    ref = np.stack([(a[:, 63:] * b[:, 63 - d:300 - d]).sum(-1) for d in range(64)], axis=-1)
+    check(got[:, 63:].reshape(-1, 64), ref.reshape(-1, 64))  # every pixel off by a share of its own size
