@@ -68,6 +68,9 @@ constexpr unsigned kNegate = 0x80000000u;
 __device__ __forceinline__ float with_sign(float x, unsigned sign) {  // x, negated by sign = kNegate
   return __uint_as_float(__float_as_uint(x) ^ sign);
 }
+// A sign from a value's bits: as good as a random one over a map, and the same wherever
+// the value lies in it.
+__device__ __forceinline__ unsigned parity_sign(unsigned bits) { return (unsigned)__popc(bits) << 31; }
 
 // x s = h + l / kLowUnit in float16, for a power of two s that takes the largest |x| of
 // a block to [2^14, 2^15): h is x s rounded to nearest, l the rest, scaled up to h's size

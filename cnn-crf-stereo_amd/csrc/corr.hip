@@ -181,15 +181,16 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
           apart0 |= apart & first;
           apart1 |= apart & ~first;
         }
+        const unsigned neg = px < TW ? parity_sign(mx) : 0u;  // (the first map's pixels: see kNegate)
         f16x8 p[2];
-        split_pair(f, split_scale(eb), p[0], p[1]);
+        split_pair(f, with_sign(split_scale(eb), neg), p[0], p[1]);
         if (v < NPX * 4) {
           const int off = px * 64 + swz(px, g);
 #pragma unroll
           for (int k = 0; k < 2; ++k) *reinterpret_cast<f16x8*>(lds + k * Cfg::plane + off) = p[k];
           if (g == 0)  // 2^-28 goes to the first map's pixels
             *reinterpret_cast<float*>(lds + Cfg::scale_off + px * 4) =
-                px < TW ? split_unscale(eb) : __uint_as_float((unsigned)eb << 23);
+                px < TW ? with_sign(split_unscale(eb), neg) : __uint_as_float((unsigned)eb << 23);
         }
       }
       if (lane == 0)
