@@ -135,7 +135,8 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       ++lho;
     }
   };
-  auto store = [&](int buf) {
+  // Stores the loaded segment s into a buffer.
+  auto store = [&](int buf, long s) {
     int flags = 0;  // float32: the units' DwFlags (uniform over the wave)
 #pragma unroll
     for (int n = 0; n < Cfg::NU; ++n) {
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
       unsigned char* d =
           lds + buf * Cfg::buffer + (u.z ? 0 : PLANES * Cfg::plane) + (u.g * VE * PITCH + 4 * u.q) * 2;
       if constexpr (Cfg::kF32) {
-        const unsigned neg = u.z && buf ? kNegate : 0u;  // every other segment's dz
+        const unsigned neg = u.z && (s & 1) ? kNegate : 0u;  // every other segment's dz
         const unsigned scale0 = (268u << 23) + neg, unscale0 = u.z ? neg - (28u << 23) : 0u;
         f32x4 unscale;
 #pragma unroll
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
   __syncthreads();  // the zero fill is done
   if (s0 < s1) {
     load_next();
-    store(0);
+    store(0, s0);
     if (s0 + 1 < s1) load_next();
   }
   __syncthreads();
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(DwCfg<T>::THREADS, 2) void k_dw_split(const T* __re
     const int buf = (int)((s - s0) & 1);
     auto stage = [&]() {
       if (s + 1 < s1) {
-        store(buf ^ 1);
+        store(buf ^ 1, s + 1);
         if (s + 2 < s1) load_next();
       }
     };

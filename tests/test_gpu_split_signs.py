@@ -38,3 +38,20 @@ def test_correlation(handle, W, D, step):
     lo, hi = (D - 1, W) if step > 0 else (0, W - D + 1)  # pixels whose whole band is inside the image
     ref = torch.stack([(a[:, lo:hi] * b[:, lo - step * d:hi - step * d]).sum(-1).flatten() for d in range(D)])
     assert bias(got[:, lo:hi].permute(2, 0, 1), ref) <= 5
+
+
+@pytest.mark.parametrize("k,H", [(3, 74), (3, 40), (2, 110)])
+def test_weight_gradient_of_one_segment_per_workgroup(handle, k, H):
+    """A map of 32 output pixels per row and no more rows than workgroups: the signs
+    alternate over the map's segments, not over a workgroup's."""
+    g = torch.Generator().manual_seed(k)
+    C, W = 100, 31 + k
+    Ho, Wo = H - k + 1, W - k + 1
+    x, dz = maps(g, H, W), maps(g, Ho, Wo)
+    w = torch.zeros((C, C, k, k), device="cuda")
+    _, dw, _ = ops.conv2d_backward_stored(handle, x.cuda(), torch.zeros((Ho, Wo, 104), device="cuda"), w, dz.cuda(),
+                                          act=False)
+    z = dz[:, :, :C].double().reshape(-1, C)
+    ref = torch.stack([z.t() @ x[k - 1 - a:k - 1 - a + Ho, k - 1 - b:k - 1 - b + Wo, :C].double().reshape(-1, C)
+                       for a in range(k) for b in range(k)], dim=2)
+    assert bias(dw.reshape(1, -1), ref.reshape(1, -1)) <= 15
