@@ -47,13 +47,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_image_split(const float* __rest
     const int t = 8 * lgrp + e;
     off[e] = t < T ? (t / 9 * Hin + t % 9 / 3) * Win + t % 3 : 0;
   }
-  float in[8];
+  float in[8], first;  // the taps, and the first plane's middle one
   auto load = [&](long tl) {
     const long p = min(tl * 16 + lrow, P - 1);
     const int ho = (int)(p / Wo), wo = (int)(p % Wo);
     const float* base = x + (long)ho * Win + wo;
 #pragma unroll
     for (int e = 0; e < 8; ++e) in[e] = base[off[e]];
+    if (sizeof(TO) == 4) first = base[Win + 1];
   };
   load(tile);
 
@@ -75,15 +76,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_image_split(const float* __rest
       for (int e = 0; e < 8; ++e) wf[t][k][e] = p[k][e];
   }
 
-  // Odd pixels of a float32 map are multiplied negated (see kNegate).
-  const unsigned neg = sizeof(TO) == 4 ? (unsigned)lrow << 31 : 0u;
-  const float sg = sizeof(TO) == 4 && (lrow & 1) ? -1.f : 1.f;
   auto run = [&](auto f) {
     for (; tile < tiles; tile += nw) {
       const long p = tile * 16 + lrow;
       float v[8];
       bf16 s[3][8];
       bf16x8 a[3];
+      // Half of a float32 map's pixels are multiplied negated (see kNegate).
+      const unsigned neg = sizeof(TO) == 4 ? parity_sign(__float_as_uint(first)) : 0u;
+      const float sg = with_sign(1.f, neg);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = 8 * lgrp + e < T ? with_sign(in[e], neg) : 0.f;
       split3(v, s[0], s[1], s[2]);

@@ -235,14 +235,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
         BlockRange r;
 #pragma unroll
         for (int e = 0; e < 8; e += 2) r.add_largest(f[e], f[e + 1]);
-        const int eb = split_exp(quad_max(r.largest()));
+        const unsigned mx = quad_max(r.largest());
+        const int eb = split_exp(mx);
         fails |= r.huge();
         if (flags & kUneven) {  // (uniform)
 #pragma unroll
           for (int e = 0; e < 8; e += 2) r.add_nonzero(f[e], f[e + 1]);
           fails |= r.apart(eb);
         }
-        const unsigned neg = (unsigned)(px / AC + px % AC) << 31;  // (a checkerboard of signs: see kNegate)
+        const unsigned neg = parity_sign(mx);  // (see kNegate)
         f16x8 p[2];
         split_pair(f, with_sign(split_scale(eb), neg), p[0], p[1]);
         if (v < NU) {
@@ -292,6 +293,9 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
   auto copy3 = [&](int ql) {
     copy_w(wpk + (long)Cfg::FULL * Cfg::taps * Cfg::w2 + (long)ql * Cfg::w3, Cfg::w3_off + (ql & 1) * Cfg::w3, 3 * NT);
   };
+  // The scales of the output pixels' first inputs, whose signs the last stage's products
+  // take (its reduction steps hold several inputs).
+  float corner[MT];
   // The copies of this wave have arrived, and so have everyone's.
   auto step_barrier = [&]() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -356,8 +360,6 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     const bool ok = kg < Cfg::taps * R;
     const int tap = ok ? kg / R : 0, g = ok ? kg % R : 0;
     const int ti = tap / Cfg::KW, tj = tap % Cfg::KW;
-    // (the output pixel's sign here)
-    const unsigned par = (unsigned)(MT * wave + lrow) & 1u, odd = par * 0x80008000u;
     bf16x8 a[3][MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
       for (int k = 0; k < 3; ++k) {
         u32x4 v = *reinterpret_cast<const u32x4*>(lds + o + (ok ? k * Cfg::rplane : 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] ^= (m & 1) ? odd ^ 0x80008000u : odd;
+        for (int e = 0; e < 4; ++e) v[e] ^= corner[m] < 0.f ? 0x80008000u : 0u;
         a[k][m] = __builtin_bit_cast(bf16x8, v);
       }
     }
@@ -393,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
       mm(0, 0);
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        const float sg = ((m & 1) ^ (int)par) ? -1.f : 1.f;
+        const float sg = corner[m] < 0.f ? -1.f : 1.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[m][t][e] = fmaf(cur[m][e], sg, acc[m][t][e]);
         asm volatile("" : "+v"(acc[m][t]));  // added here, not behind the step (the sums of all tiles would spill)
@@ -413,6 +415,11 @@ __global__ __launch_bounds__(256, 2) void k_conv_split(const float* __restrict__
     stage(std::integral_constant<int, 4>{}, 4 * s);
     step_barrier();
     again |= failed();
+    if constexpr (Cfg::REM > 0) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        corner[m] = *reinterpret_cast<const float*>(lds + Cfg::scale_off + ((MT * wave + m) * AC + lrow) * 4);
+    }
     const int taps = again ? 0 : Cfg::taps;
 #pragma unroll 1
     for (int tap = 0; tap < taps; ++tap) {

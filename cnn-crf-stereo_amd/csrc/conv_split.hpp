@@ -59,9 +59,10 @@ __device__ __forceinline__ float split_unscale(int eb) { return __uint_as_float(
 // The matrix unit rounds its 16-bit products' sums down, whatever their sign: an
 // output's error is small but always of one sign, and sums over a map's pixels (the
 // gradients of earlier layers and of biases) gather it.  So one operand is negated
-// for every other pixel, row or segment, and the sum is negated back where it is
+// for half of the pixels, rows or segments, and the sum is negated back where it is
 // added up in the vector unit, which rounds to nearest: over a map the errors
-// cancel.  Six 3x3 layers' bias gradients from exact inputs (512 x 256) were off by
+// cancel.  Which half, the bits of an input value decide (parity_sign), so that equal
+// inputs give equal outputs wherever they lie.  Six 3x3 layers' bias gradients from exact inputs (512 x 256) were off by
 // 1.0e-6 to 2.0e-6 without it and are by 0.7e-7 to 0.9e-7 with it, at the same
 // speed (v_mfma_f32_16x16x4_f32: 0.8e-7 to 1.1e-7).  kNegate is a float's sign bit.
 constexpr unsigned kNegate = 0x80000000u;

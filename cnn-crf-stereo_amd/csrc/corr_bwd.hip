@@ -112,11 +112,16 @@ __global__ __launch_bounds__(CorrBwdTile<T>::THREADS, 2) void k_corr_bwd_split(C
   const T* frow = (const T*)(gather ? a.f0 : a.f1) + rowpix * Cs;
   const float* grow = a.G + rowpix * D;
 
-  // Odd rows of a float32 map are multiplied negated (see kNegate).  A bfloat16
-  // result is rounded at 2^-9 of itself, to nearest, which hides an offset of
-  // 1e-7 also in a sum over a frame (and the sign cost 1361 -> 1610 us there).
-  const unsigned neg = kF32 && (h & 1) ? kNegate : 0u;
-  const float sg = kF32 && (h & 1) ? -1.f : 1.f;
+  // Half of a float32 map's rows are multiplied negated (see kNegate): a sign from
+  // the first pixel's features.  A bfloat16 result is rounded at 2^-9 of itself, to
+  // nearest, which hides an offset of 1e-7 also in a sum over a frame (and the sign cost
+  // 1361 -> 1610 us there).
+  unsigned neg = 0;
+  if constexpr (kF32) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>((const T*)a.f0 + rowpix * Cs);
+    neg = parity_sign(__builtin_amdgcn_readfirstlane(v[0] ^ v[1] ^ v[2] ^ v[3]));
+  }
+  const float sg = with_sign(1.f, neg);
 
   // Rows Cs .. 112 of the planes stay zero.
   for (int v = tid; v < Cfg::PLANES * (16 * NT - Cs) * (PITCH / 8); v += Cfg::THREADS) {
