@@ -311,19 +311,28 @@ static int run(ccs_handle_t h, const float* cost, const float* wx, const float* 
   if (rc) return rc;
   CCS_CHECK(iters >= 0 && iters <= 10000, CCS_ERR_ARG, "ccs_slackprop: bad iteration count %d", iters);
   const size_t vol = (size_t)H * W * D, bytes = vol * sizeof(float);
-  // The state lives in unaries_out where the caller wants the final unaries
-  // (no copy at the end), unless that overlaps the costs every sweep reads.  The
-  // handle's own volume is reserved either way, so that after one run any call
-  // of these sizes can be captured.
-  const uintptr_t u0 = (uintptr_t)unaries_out, c0 = (uintptr_t)cost;
-  const bool own = !unaries_out || (u0 < c0 + bytes && c0 < u0 + bytes);
+  // The state lives in unaries_out where the caller wants the final unaries (no
+  // copy at the end), and the sums in theirs, unless those lie over an input: every
+  // sweep reads the costs and the weights.  The handle's own volume is reserved
+  // either way, so that after one run any call of these sizes can be captured.
+  const size_t plane = (size_t)H * W * sizeof(float);
+  auto over_input = [&](const void* out, size_t n) {
+    auto over = [&](const float* in, size_t m) {
+      const uintptr_t o = (uintptr_t)out, i = (uintptr_t)in;
+      return in && o < i + m && i < o + n;
+    };
+    return over(cost, bytes) || (pen ? over(pen, 2 * levels * plane) : over(wx, plane) || over(wy, plane));
+  };
+  const size_t nsums = 4 * (size_t)iters + 1;
+  const bool own = !unaries_out || over_input(unaries_out, bytes);
+  const bool own_sums = !sums || over_input(sums, sizeof(double) * nsums);
   if ((rc = h->crf_a.reserve(bytes, h->stream))) return rc;
   if ((rc = h->crf_sums.reserve(sizeof(double) * (4 * (size_t)iters + 2), h->stream))) return rc;
   const int nmax = H > W ? H : W;
   if ((rc = h->crf_small.reserve(sizeof(double) * run_chain_doubles(nmax), h->stream))) return rc;
   float* A = own ? (float*)h->crf_a.ptr : unaries_out;
-  double* S = sums ? sums : (double*)h->crf_sums.ptr;  // S_0 .. S_{2 iters}
-  double* K = S + 2 * iters + 1;                       // K_0 .. K_{2 iters - 1}
+  double* S = own_sums ? (double*)h->crf_sums.ptr : sums;  // S_0 .. S_{2 iters}
+  double* K = S + 2 * iters + 1;                           // K_0 .. K_{2 iters - 1}
   double* chains = (double*)h->crf_small.ptr;
   if (iters == 0) {
     CCS_HIP(hipMemcpyAsync(A, cost, bytes, hipMemcpyDeviceToDevice, h->stream));
@@ -348,6 +357,7 @@ static int run(ccs_handle_t h, const float* cost, const float* wx, const float* 
       j0 = j + 1;
     }
   }
+  if (own_sums && sums) CCS_HIP(hipMemcpyAsync(sums, S, sizeof(double) * nsums, hipMemcpyDeviceToDevice, h->stream));
   if (own && unaries_out) CCS_HIP(hipMemcpyAsync(unaries_out, A, bytes, hipMemcpyDeviceToDevice, h->stream));
   CCS_LAUNCH_CHECK();
   return CCS_OK;
