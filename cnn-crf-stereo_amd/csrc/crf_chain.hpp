@@ -47,6 +47,11 @@ constexpr int kRowRing = 3;
 
 constexpr size_t kLdsPerCu = 160 * 1024;
 
+// LDS of one chain of k_chain: b (doubles), w, u, [w2].
+constexpr size_t chain_lds(bool per_edge, int n) {
+  return (sizeof(double) + (per_edge ? 3 : 2) * sizeof(float)) * (size_t)n;
+}
+
 // LDS of one row chain with the message wave: b, w, u, [w2], v floats rounded
 // to 16 bytes, then the message ring.
 constexpr size_t row_seg_lds(int lpl, bool per_edge, int n) {

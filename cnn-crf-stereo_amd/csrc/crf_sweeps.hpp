@@ -2017,13 +2017,30 @@ static void launch_line(ChainArgs& a, hipStream_t st) {
 //   rows, D = 128: 320 x 240 63 / 72, 744 x 496 166 / 169, 1000 x 1000 458 / 414
 //   columns, D = 64:  320 x 240 43 / 63, 1000 x 1000 238 / 281, 1242 x 375 141 / 129
 //   columns, D = 128: 320 x 240 50 / 66, 512 x 256 62 / 74, 640 x 480 206 / 154
+// Long chains take more LDS here than in k_chain, so that fewer share a CU and they may
+// take more rounds of workgroups, of two thirds of the time each:
+//   rows, two rounds / one: 400 of 3000 nodes, D = 128 1140 / 633; 500 of 3300, D = 64 1004 / 570
+//   columns, two / one: 1000 of 2000 nodes, D = 64 712 / 558; 400 of 3000, D = 128 1160 / 796
+//   columns, three / two: 700 of 4096 nodes, D = 32 1811 / 1993
 template <int LPL, int MODE>
-static bool use_line(const ChainArgs& a) {
-  constexpr int kRounds = MODE == kColsMinorant && LPL == 1 ? 4 : 2;
+static bool use_line(const ChainArgs& a, bool seg) {
+  constexpr bool kCols = MODE == kColsMinorant;
+  constexpr int kPerCu = kCols && LPL == 1 ? 4 : 2;
+  const bool pe = a.w2 != nullptr;
+  const int cus = cu_count();
   const long extent = ((long)(a.n - 1) * a.pns * a.D + a.D) * (long)sizeof(float);  // 32-bit byte offsets
   const long msg = (long)a.n * a.D * (long)sizeof(float);
-  return a.n_chains <= kRounds * cu_count() && line_lds(LPL, a.w2 != nullptr, a.n) <= kLdsPerCu &&
-         extent <= 0x7fffffffL && msg <= 0x7fffffffL;
+  const size_t lds = line_lds(LPL, pe, a.n);
+  if (a.n_chains > kPerCu * cus || lds > kLdsPerCu || extent > 0x7fffffffL || msg > 0x7fffffffL) return false;
+  // Rounds of chains, `per` to a workgroup of per * l bytes (0: not launchable).
+  auto rounds = [&](size_t l, int per) {
+    const long resident = (long)(kLdsPerCu / (per * l)) * per * cus;
+    return resident ? (a.n_chains + resident - 1) / resident : 0x7fffffffL;
+  };
+  const bool many = a.n_chains > cus;
+  const size_t chain = !kCols && seg ? row_seg_lds(LPL, pe, a.n) : chain_lds(pe, a.n);
+  const bool pairs = !kCols && seg && many && a.n_chains <= 2 * cus && 2 * chain <= kLdsPerCu;
+  return 2 * rounds(lds, many && 2 * lds <= kLdsPerCu ? 2 : 1) <= 3 * rounds(chain, pairs ? 2 : 1);
 }
 
 // Register-ring depth of the row sweeps with a message wave: three segments.
@@ -2055,7 +2072,7 @@ static void launch_one(ChainArgs& a, size_t lds, bool seg, hipStream_t st) {
     constexpr bool kCols = MODE == kColsMinorant;
     constexpr int PS = kCols ? P : row_seg_p<LPL>();  // ring depth of the checkpointed sweep
     if constexpr (DC == 2 && LPL <= 2) {
-      if (use_line<LPL, MODE>(a)) {
+      if (use_line<LPL, MODE>(a, seg)) {
         auto line = [&](auto fit) {
           constexpr int F = decltype(fit)::value;
           if constexpr (!kCols)
@@ -2118,7 +2135,7 @@ static void launch_lpl(ChainArgs& a, size_t lds, bool seg, hipStream_t st) {
 // translation unit of their own (crf_sweeps_*.hip).
 template <int LPL, int MODE>
 int launch_labels(ChainArgs& a, bool seg, hipStream_t st) {
-  const size_t lds = (sizeof(double) + (a.w2 ? 3 : 2) * sizeof(float)) * (size_t)a.n;
+  const size_t lds = chain_lds(a.w2 != nullptr, a.n);
   constexpr int P = MODE == kColsMinorant ? CCS_CRF_P_COLS : CCS_CRF_P_ROWS;
   launch_lpl<MODE, LPL, LPL < 4 ? P : P / 2>(a, lds, seg, st);
   CCS_LAUNCH_CHECK();
