@@ -67,8 +67,11 @@ struct CorrSplit {
 // the product of two pixels' scales may be infinite; uneven() ones, apart() ones.
 enum CorrFlag { kUneven0 = 1, kUneven1 = 2, kApart0 = 4, kApart1 = 8, kHuge = 16 };
 
+// IN_PLACE: -softmax in the accumulators, see in_place().  (A branch on an argument
+// instead cost the volumes that do not take it up to 1 %, 700 x 300 D = 200 in bf16 179.2
+// us for 177.8, and those that do 2 %, 700 x 300 D = 256 140.4 for 137.3.)
 // (float32, NTM 9: the registers of two workgroups of 8 waves per CU)
-template <typename T, int NTM>
+template <typename T, int NTM, bool IN_PLACE>
 __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_corr_volume(CorrArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int NW = blockDim.x >> 6;
@@ -88,8 +91,6 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
   const T* f0 = reinterpret_cast<const T*>(a.f0) + (long)h * a.W * Cs;
   const T* f1 = reinterpret_cast<const T*>(a.f1) + (long)h * a.W * Cs;
   f32x4 acc[NTM];
-#pragma unroll
-  for (int t = 0; t < NTM; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int arow = 16 * wave + lrow;  // pixel of this lane's A row
   if constexpr (sizeof(T) == 2) {
     const int wbase = w0 + a.o_lo;  // first f1 column of the window
@@ -118,6 +119,8 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
         },
         [&](int v, const u32x4& val) { put(F1, v / vpp, v % vpp, val); });
     __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NTM; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int cg = Cs / 8;
     for (int q = 0; q < (cg + 3) / 4; ++q) {
       const int g = 4 * q + lgrp;
@@ -232,6 +235,8 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
       }
     };
 
+#pragma unroll
+    for (int t = 0; t < NTM; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int stages = (cg + 3) / 4;  // 20 at most: wider pixels are refused
     unsigned floats = 0;              // the stages left for float32 products
     load(0);
@@ -267,17 +272,11 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
     }
     for (; floats; floats &= floats - 1) float_stage(__builtin_ctz(floats));
   }
-  // -softmax over the band, in the accumulators where the disparities are
-  // consecutive columns: lane (lrow, lgrp) holds columns 16 t + lrow of pixels
-  // 4 lgrp + e, and a pixel's band is the D columns from its own on.  (Through LDS
-  // every entry is read twice and written once more.)  It works on whole column
-  // tiles, so it pays for wide bands that nearly fill theirs (us, through LDS / here,
-  // bf16): 1242 x 375 D = 128 129 / 124, 1488 x 992 D = 256 1040 / 883, but D = 64 (80
-  // columns) 69 / 70, D = 70 (144) 117 / 124, D = 24 67 / 71.
+  // -softmax over the band, in the accumulators: lane (lrow, lgrp) holds columns 16 t +
+  // lrow of pixels 4 lgrp + e, and a pixel's band is the D columns from its own on.
   const int D = a.D;
   const bool neg_softmax = a.epilogue == CCS_EPILOGUE_NEG_SOFTMAX;
-  const bool in_place = neg_softmax && (a.ostep == 1 || a.ostep == -1) && NTM >= 9 && D + 32 >= 16 * NTM;
-  if (in_place) {
+  if constexpr (IN_PLACE) {
     auto row16 = [](float x, auto op) {  // over the 16 lanes of a row
       x = op(x, dpp_rot<0xb1>(x));
       x = op(x, dpp_rot<0x4e>(x));
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 && NTM == 9 ? 4 : 1) void k_cor
 
   // Band entry of pixel r, disparity k: S_w[r * sp + r + o_k - o_lo] = band(r)[k * ostep].
   auto band = [&](int r) { return S_w + r * a.sp + r + a.o0 - a.o_lo; };
-  const bool scaled = neg_softmax && !in_place;  // by stats, when stored
+  const bool scaled = !IN_PLACE && neg_softmax;  // by stats, when stored
   if (scaled) {
     // 4 lanes per pixel: max, then exp(s - max) written back in place, then 1 / sum.
     const int r = lane >> 2, s4 = lane & 3;
@@ -608,29 +607,50 @@ static size_t corr_lds_bytes(CorrArgs& a, int NW) {
   return (size_t)a.stats_off + (size_t)NW * 16 * 4;
 }
 
+// Whether the softmax runs in the accumulators: where the disparities are consecutive
+// columns.  (Through LDS every entry is read twice and written once more.)  It works on
+// whole column tiles, so it pays for wide bands that nearly fill theirs (us, through LDS /
+// in the accumulators, at 1242 x 375): bf16 D = 128 124 / 115, D = 112 135 / 126, 1488 x
+// 992 D = 256 989 / 818; float32 209 / 208, 219 / 218, 1402 / 1300; but D = 70 (of 144
+// columns) 111 / 111 and 195 / 201, D = 24 62 / 63 and 126 / 127.  Between D = 70 and the
+// line it still gains in bf16 (D = 100 128 / 122) and is equal in float32 (214 / 215).
+template <int NTM>
+static bool in_place(const CorrArgs& a) {
+  return NTM >= 9 && a.D + 32 >= 16 * NTM && (a.ostep == 1 || a.ostep == -1) &&
+         a.epilogue == CCS_EPILOGUE_NEG_SOFTMAX;
+}
+
+// Calls f with in_place() as a constant (false for the tile counts that never have it).
+template <int NTM, typename F>
+static int with_in_place(const CorrArgs& a, F&& f) {
+  if constexpr (NTM >= 9)
+    if (in_place<NTM>(a)) return f(std::true_type{});
+  return f(std::false_type{});
+}
+
 template <int NTM>
 static int launch_volume(CorrArgs a, int NW, hipStream_t st) {
   const size_t bytes = corr_lds_bytes(a, NW);
-  static bool configured = false;
-  if (!configured) {
-    CCS_HIP(hipFuncSetAttribute((const void*)k_corr_volume<bf16, NTM>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024));
-    configured = true;
-  }
-  k_corr_volume<bf16, NTM><<<dim3(ceil_div(a.W, 16 * NW), a.H), 64 * NW, bytes, st>>>(a);
-  CCS_LAUNCH_CHECK();
-  return CCS_OK;
+  return with_in_place<NTM>(a, [&](auto soft) -> int {
+    const auto kern = k_corr_volume<bf16, NTM, decltype(soft)::value>;
+    CCS_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    kern<<<dim3(ceil_div(a.W, 16 * NW), a.H), 64 * NW, bytes, st>>>(a);
+    CCS_LAUNCH_CHECK();
+    return CCS_OK;
+  });
 }
 
 template <int NTM>
 static int launch_split(CorrArgs a, hipStream_t st) {
   using Cfg = CorrSplit<NTM>;
   a.stats_off = Cfg::stats_off;
-  CCS_HIP(hipFuncSetAttribute((const void*)k_corr_volume<float, NTM>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              Cfg::lds_bytes));
-  k_corr_volume<float, NTM><<<dim3(ceil_div(a.W, Cfg::TW), a.H), Cfg::THREADS, Cfg::lds_bytes, st>>>(a);
-  CCS_LAUNCH_CHECK();
-  return CCS_OK;
+  return with_in_place<NTM>(a, [&](auto soft) -> int {
+    const auto kern = k_corr_volume<float, NTM, decltype(soft)::value>;
+    CCS_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::lds_bytes));
+    kern<<<dim3(ceil_div(a.W, Cfg::TW), a.H), Cfg::THREADS, Cfg::lds_bytes, st>>>(a);
+    CCS_LAUNCH_CHECK();
+    return CCS_OK;
+  });
 }
 
 }  // namespace ccs
