@@ -97,8 +97,57 @@ __host__ __device__ inline void split_step(int q, int lgrp, int* tap, int* c0) {
 // (lrow, lgrp) holding output channel 16 t + lrow; then the row scales.  All
 // weights of a row are divided by its scale.  A tile with a row that pairs do not
 // hold has scales of 1 and its first fragments as [q][t][2][lane][4] float32.
-// Block (t, y) packs a share of tile t's steps; its 16 groups of 16 lanes each look
-// at one row first.
+// Block (t, y) packs row y of tile t and a share of its last steps; its 16 groups of
+// 16 lanes each look at one row first.
+//
+// A pair holds 23 of a float's 24 bits, so that every fourth weight would be off by
+// 2^-24 or 2^-23 of itself, the same for all pixels: maps whose channels have a mean were
+// off by that mean times the sum of a channel's roundings, everywhere alike (the mean of
+// an output channel by 4e-9 in a tower of values around 0.3, where float32 products leave
+// 0.7e-9, and by up to 1e-7 of its size with positive inputs).  So what the low term of a
+// tap leaves out is added to the next one's, what the last leaves to the tap whose low
+// term is finest, and what that leaves to the next of 16 channels.  Only weights of at least half
+// of the channel's largest take part, and from another channel only what is 2^-23 of this
+// channel's largest at most: every weight stays within 2^-22 of itself, and a zero stays 0.
+template <int N>
+__device__ __forceinline__ void split_taps(const float (&v)[N], float s, _Float16 (&h)[N], _Float16 (&l)[N]) {
+  float m = 0.f, carry = 0.f, finest = __builtin_huge_valf();
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(v[i]));
+  int best = -1;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float x = v[i] * s;
+    h[i] = (_Float16)x;
+    const float r = fmaf((float)h[i], -kLowUnit, x * kLowUnit);
+    const bool large = m > 0.f && 2.f * fabsf(v[i]) >= m;
+    const float want = large ? r + carry : r;
+    l[i] = (_Float16)want;
+    carry = large ? want - (float)l[i] : carry + (want - (float)l[i]);
+    if (large && fabsf(r) < finest) {
+      finest = fabsf(r);
+      best = i;
+    }
+  }
+  float fine = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) fine = i == best ? (float)l[i] : fine;
+  const float limit = m * s * kLowUnit * 0x1p-23f;
+  float rest = 0.f;  // what the channels of this row of 16 lanes up to here leave out
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float before = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(rest), 0x111, 0xf, 0xf, true));  // row_shr:1
+    const float want = fine + (carry + before), got = (float)(_Float16)want;
+    const bool take = best >= 0 && fabsf(before) <= limit;
+    if ((int)(threadIdx.x & 15) == i) {
+      rest = take ? want - got : before;
+      fine = take ? got : fine;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) l[i] = i == best ? (_Float16)fine : l[i];
+}
+
 constexpr int kPackShares = 16;
 template <class Cfg>
 __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w, int K, int C, int adj,
@@ -115,8 +164,8 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
 #pragma unroll 8
     for (int i = tid & 15; i < C * Cfg::taps; i += 16) {
       const float v = at(row, i / Cfg::taps, i % Cfg::taps);
-      r.add_largest(v, v);
-      r.add_least(v, v);
+      r.above = fmaxf(r.above, fabsf(v));  // (the class's asm keeps the loop from being unrolled)
+      r.least = fminf(r.least, fabsf(v));
       r.add_nonzero(v, v);
     }
   }
@@ -131,32 +180,38 @@ __global__ __launch_bounds__(256) void k_pack_split(const float* __restrict__ w,
   }
   if (blockIdx.y == 0 && tid == 0) reinterpret_cast<int*>(out + Cfg::flag_off)[t] = wide ? kWide : uneven ? kUneven : 0;
   __syncthreads();
-  for (int u = blockIdx.y * 256 + tid; u < Cfg::NQ * 64; u += kPackShares * 256) {
-    const int q = u >> 6, lane = u & 63, n = 16 * t + (lane & 15);
-    const int eb = exps[lane & 15];
-    int tap, c0;
-    split_step<Cfg>(q, lane >> 4, &tap, &c0);
-    float v[8];
+  constexpr int NQ2 = Cfg::FULL * Cfg::taps, kLast = Cfg::REM_NQ * 64 / kPackShares;
+  static_assert(Cfg::FULL * 32 <= 128 && kLast <= 128, "a thread per channel, then one per lane's share of a last step");
+  if (tid < 128) {  // (whole waves)
+    const int n = 16 * t + blockIdx.y, c = tid, e = c & 7, lane = ((c >> 3) & 3) * 16 + blockIdx.y, stage = c >> 5;
+    float v[Cfg::taps];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = n < K && c0 >= 0 && c0 + e < C ? at(n, c0 + e, tap) : 0.f;
-    constexpr int NQ2 = Cfg::FULL * Cfg::taps;
-    if (q < NQ2) {
-      f16x8 p[2];
-      if (wide) {
+    for (int j = 0; j < Cfg::taps; ++j) v[j] = stage < Cfg::FULL && n < K && c < C ? at(n, c, j) : 0.f;
+    _Float16 h[Cfg::taps], l[Cfg::taps];
+    split_taps(v, split_scale(exps[blockIdx.y]), h, l);
+    if (stage < Cfg::FULL) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-          p[k] = __builtin_bit_cast(f16x8, f32x4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]});
-      } else {
-        split_pair(v, split_scale(eb), p[0], p[1]);
+      for (int j = 0; j < Cfg::taps; ++j) {
+        unsigned char* frag = out + ((long)((stage * Cfg::taps + j) * Cfg::NT + t) * 128 + lane) * 16;
+        if (wide) {
+          reinterpret_cast<float*>(frag + (e >> 2) * 1024)[e & 3] = v[j];
+        } else {
+          reinterpret_cast<_Float16*>(frag)[e] = h[j];
+          reinterpret_cast<_Float16*>(frag + 1024)[e] = l[j];
+        }
       }
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        *reinterpret_cast<f16x8*>(out + ((long)((q * Cfg::NT + t) * 2 + k) * 64 + lane) * 16) = p[k];
-    } else {
+    }
+  } else {
+    const int u = blockIdx.y * kLast + tid - 128;
+    if (tid - 128 < kLast) {
+      const int lane = u & 63, n = 16 * t + (lane & 15), eb = exps[lane & 15], q = NQ2 + (u >> 6);
+      int tap, c0;
+      split_step<Cfg>(q, lane >> 4, &tap, &c0);
       const float unit = __uint_as_float(eb < 254 ? (unsigned)(254 - eb) << 23 : 0x400000u);  // 1 / the row's scale
+      float v[8];
       bf16 p[3][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= unit;
+      for (int e = 0; e < 8; ++e) v[e] = (n < K && c0 >= 0 && c0 + e < C ? at(n, c0 + e, tap) : 0.f) * unit;
       split3(v, p[0], p[1], p[2]);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {

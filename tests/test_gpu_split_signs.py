@@ -55,3 +55,28 @@ def test_weight_gradient_of_one_segment_per_workgroup(handle, k, H):
     ref = torch.stack([z.t() @ x[k - 1 - a:k - 1 - a + Ho, k - 1 - b:k - 1 - b + Wo, :C].double().reshape(-1, C)
                        for a in range(k) for b in range(k)], dim=2)
     assert bias(dw.reshape(1, -1), ref.reshape(1, -1)) <= 15
+
+
+def offset(got, ref):
+    """The largest mean error of a group (groups x outputs), in units of its root mean square."""
+    err = got.double().cpu().reshape(ref.shape) - ref
+    return (err.mean(dim=1).abs() / ref.square().mean(dim=1).sqrt()).max().item()
+
+
+@pytest.mark.parametrize("C,k", [(100, 3), (100, 2), (64, 3)])
+@pytest.mark.parametrize("H,W", [(131, 166), (250, 203)])
+def test_layer_of_positive_maps(handle, C, k, H, W):
+    """Inputs with a mean: what rounding leaves out of a weight is the same for every
+    pixel, but the weights of a row together leave out nothing.  A float32 output is
+    itself off by up to 2^-24; the mean over a map stays within half of that."""
+    g = torch.Generator().manual_seed(C + k + H)
+    x = maps(g, H, W, C).abs()
+    w = (torch.rand((C, C, k, k), generator=g) * 2 - 1) * 0.1
+    got = ops.ConvLayer(handle, w.numpy(), np.zeros(C, np.float32), "fp32", act=False)(handle, x.cuda())[:, :, :C]
+    ref = torch.nn.functional.conv2d(x[:, :, :C].double().permute(2, 0, 1)[None], w.double().flip(2, 3))[0].reshape(C, -1)
+    assert offset(got.permute(2, 0, 1), ref) <= 2.0**-25
+    # the input gradient, whose filters are the adjoint ones
+    dy = maps(g, H - k + 1, W - k + 1, C).abs()
+    dx, _, _ = ops.conv2d_backward_stored(handle, x.cuda(), torch.zeros_like(dy).cuda(), w.cuda(), dy.cuda(), act=False)
+    ref = torch.nn.functional.conv_transpose2d(dy[:, :, :C].double().permute(2, 0, 1)[None], w.double().flip(2, 3))
+    assert offset(dx[:, :, :C].permute(2, 0, 1), ref[0].reshape(C, -1)) <= 2.0**-25
