@@ -655,7 +655,8 @@ void split_launch(const float* x, int H, int W, int C, const void* packed, const
     using Small = SplitCfg<Cfg::KH, Cfg::KW, Cfg::CG, Cfg::NT, 1>;
     // Tiles of four rows while they do not fill two workgroups per CU: the layer
     // then takes as long as one tile does (us, four rows / eight: 64 x 64 3x3
-    // 24 / 33, 200 x 100 2x2 (325 tiles) 18 / 22, 325 x 245 2x2 (1281) 48 / 42).
+    // 24 / 33, 200 x 100 2x2 (325 tiles of four rows) 18 / 22; past that 325 x 245 2x2,
+    // 1281 tiles of four rows or 651 of eight, 48 / 42).
     if ((long)ceil_div(Wo, Small::TW) * ceil_div(Ho, Small::TH) <= 2 * cu_count())
       launch(Small{});
     else

@@ -1358,7 +1358,7 @@ __global__ __launch_bounds__(512) void k_line(ChainArgs a) {
   float* v_lds = u_lds + n;
   float* w2_lds = v_lds + n;  // PE only
   float* msg_ring = reinterpret_cast<float*>(b_lds) + head;  // [3][K] nodes of 64 x (Bh, theta)
-  float* out_ring = msg_ring + 3 * K * 2 * NS;               // [3][K] nodes
+  float* out_ring = msg_ring + 3 * K * 2 * NS;               // [2][K] nodes, by segment
   ShiftCarry cc;
   const float L1v = in_vgpr(a.L1), L2v = in_vgpr(a.L2);
   const long pbase = (long)c * a.pcs;

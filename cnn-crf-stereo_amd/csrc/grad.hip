@@ -6,10 +6,10 @@
 //   dW[k][c][KH-1-i][KW-1-j] = sum_p dz[p][k] x[p + (i,j)][c]
 //   dx = true convolution of dz zero-padded by (KH-1, KW-1) with
 //        Wt[c][k][a][b] = W[k][c][KH-1-a][KW-1-b]
-// dW runs on the bf16 matrix cores (conv_grad.hip) for equal types and 65 to 112
-// channels on both sides, on v_mfma_f32_16x16x4_f32 (k_dw_mfma: per tap, a K x C
-// GEMM reduced over pixels) elsewhere, dx on the forward MFMA kernels.  Maps are float32 or bfloat16
-// (the BF16 form keeps activations and activation gradients in bf16 and
+// dW runs on the 16-bit matrix cores (conv_grad.hip; float32 maps as pairs of
+// float16) for equal types and 65 to 112 channels on both sides, on
+// v_mfma_f32_16x16x4_f32 (k_dw_mfma: per tap, a K x C GEMM reduced over pixels)
+// elsewhere, dx on the forward MFMA kernels.  Maps are float32 or bfloat16 (the BF16 form keeps activations and activation gradients in bf16 and
 // accumulates in float32).  Reductions over pixels are split into blocks and
 // summed in a fixed order: results do not depend on scheduling.
 #include <algorithm>

@@ -93,6 +93,14 @@ int ccs_rgb_to_gray(ccs_handle_t h, const float* rgb, int H, int W, float* gray)
  *    C <= 8, a C x H x W float32 image); y: (H-KH+1) x (W-KW+1) x ccs_feature_stride(K).
  * w: K x C x KH x KW float32 (the reference's npz layout), b: K float32 (or NULL).
  * precision CCS_BF16: x, y are bfloat16 and the MFMA accumulates in float32.
+ * CCS_FP32: float32 in, out and in all sums.  The shapes that the towers use, their
+ * weight gradients and the correlation form their products on the 16-bit matrix
+ * cores from pairs of float16 (which hold a value to 2^-22 of itself) or exactly
+ * from three bfloat16 terms, and on the float32 matrix instruction for a tile,
+ * segment or stage whose values a pair with one power-of-two scale doesn't hold
+ * (huge, infinite, or too far apart): the error against float64 is no larger than
+ * that of float32 products.  Pixels with equal surroundings get equal results
+ * wherever they lie, but for those in a tile that takes the float32 instruction.
  * act: 1 = tanh, 0 = identity.  Weights are repacked into handle scratch on
  * every call; ccs_conv_pack_weights + ccs_conv_forward_packed avoid that. */
 int ccs_conv2d_forward(ccs_handle_t h, const void* x, int x_layout, int H, int W, int C,
@@ -135,9 +143,10 @@ int ccs_conv2d_backward(ccs_handle_t h, const float* x, int H, int W, int C, con
  * shape, may be NULL) have y's element type; dw (K x C x KH x KW) and db (K,
  * may be NULL) are float32.  x_precision may be CCS_FP32 under a CCS_BF16
  * layer (the first layer reads the float32 image).  The weight gradient runs on
- * v_mfma_f32_16x16x4_f32, dx on the forward MFMA kernels, with fixed-order pixel
- * reductions.  No reference counterpart (the reference has no convolution
- * backward). */
+ * the 16-bit matrix cores where x and y have one type and 65 to 112 channels
+ * (float32 maps as pairs, see ccs_conv2d_forward) and on v_mfma_f32_16x16x4_f32
+ * elsewhere, dx on the forward MFMA kernels, with fixed-order pixel reductions.
+ * No reference counterpart (the reference has no convolution backward). */
 int ccs_conv2d_backward_stored(ccs_handle_t h, const void* x, int x_precision, const void* y,
                                int precision, int H, int W, int C, const float* w, int K, int KH,
                                int KW, int act, const void* dy, void* dx, float* dw, float* db);
