@@ -1,7 +1,7 @@
 /*
  * FP64 CPU oracle of the CNN-CRF stereo hot path -- TEST INFRASTRUCTURE ONLY.
  *
- * This file is the checker: tests, the smoke check and the benchmark's CPU
+ * This file is the oracle: tests, the smoke check and the benchmark's CPU
  * baseline load it; the HIP product never does.  Each function restates one
  * reference operator in double precision (citations next to each function,
  * relative to the reference repository root).

@@ -1,7 +1,7 @@
 /*
  * FP64 CPU oracle of the CNN-CRF stereo hot path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker that the HIP
+ * TEST INFRASTRUCTURE ONLY.  This library is what the HIP
  * product path is compared against.  Only tests, the smoke check and the
  * CPU-baseline leg of the benchmark may load it; nothing in the product
  * links, calls or falls back to it.

@@ -1,7 +1,7 @@
 """ctypes wrapper of the FP64 oracle (liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, the smoke check and the CPU
-baseline leg of bench.py as the checker.  The product path never imports it.
+baseline leg of bench.py as the oracle.  The product path never imports it.
 All functions take and return float64 numpy arrays in the layouts documented
 in oracle.h (images C x H x W, cost volumes H x W x D).
 """
